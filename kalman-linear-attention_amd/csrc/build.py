@@ -22,7 +22,7 @@ INCLUDE = os.path.join(REPO, "include")
 DEFAULT_OUT = os.path.join(PKG_ROOT, "kla", "lib", "libkla_hip.so")
 SOURCES = ["kla_hip.hip"]
 HEADERS = ["causal_conv.hpp", "fused_kla.hpp", "gate_skip.hpp", "lookback_scan.hpp", "model_ops.hpp", "rows_linear.hpp",
-           "scan_ops.hpp"]
+           "scan_ops.hpp", "split_gemm.hpp"]
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_{add,mul,fma}_f32.
 HIPCC_FLAGS = [

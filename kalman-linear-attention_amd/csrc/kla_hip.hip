@@ -22,13 +22,14 @@
 #include "model_ops.hpp"
 #include "rows_linear.hpp"
 #include "fused_kla.hpp"
+#include "split_gemm.hpp"
 #include "lookback_scan.hpp"
 
 namespace {
 
 using namespace kla;
 
-constexpr int kAbiVersion = 17;
+constexpr int kAbiVersion = 18;
 
 // Tile shapes: W waves x S steps per wave (chunk = W*S steps), V lanes per
 // thread (tile = 64 V lanes), each chosen by timing the kernel inside the
@@ -1520,6 +1521,69 @@ int rows_linear_launch(const char *fn, int epi, RowsLinearParams &p, hipStream_t
   return hip_status(fn, hipGetLastError());
 }
 
+// The split fp32 product (split_gemm.hpp). Workspace: the planes of x and of W,
+// then their row exponents.
+int64_t linear_f32_bytes(int64_t rows, int64_t n, int64_t k) {
+  const int64_t blocks = sadd(sadd(rows, kSplitRows - 1) / kSplitRows, sadd(n, kSplitRows - 1) / kSplitRows);
+  const int64_t planes = smul(smul(blocks, sadd(k, kSplitK - 1) / kSplitK), kSplitChunk * 2);
+  return sadd(planes, smul(blocks, kSplitRows * 4));
+}
+
+int linear_f32_launch(const char *fn, const float *x, int64_t ldx, const float *w, int64_t ldw, const float *bias,
+                      float *y, int64_t ldy, int64_t rows, int64_t n, int64_t k, void *workspace,
+                      hipStream_t stream) {
+  SplitGemmParams g{};
+  g.x = x, g.w = w, g.bias = bias, g.y = y;
+  g.ldx = ldx, g.ldw = ldw, g.ldy = ldy;
+  g.rows = rows, g.n = n, g.k = k;
+  g.chunks = (k + kSplitK - 1) / kSplitK;
+  g.xblocks = (rows + kSplitRows - 1) / kSplitRows;
+  g.wblocks = (n + kSplitRows - 1) / kSplitRows;
+  if (g.chunks >= (1ll << 30) || g.xblocks + g.wblocks >= (1ll << 31) || smul(2 * g.xblocks, 2 * g.wblocks) >= (1ll << 31))
+    return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
+  _Float16 *xs = static_cast<_Float16 *>(workspace);
+  _Float16 *ws = xs + g.xblocks * g.chunks * kSplitChunk;
+  int *xe = reinterpret_cast<int *>(ws + g.wblocks * g.chunks * kSplitChunk);
+  int *we = xe + g.xblocks * kSplitRows;
+  g.xs = xs, g.ws = ws, g.xe = xe, g.we = we;
+
+  SplitParams sp{};
+  sp.op[0] = SplitOperand{x, ldx, rows, xs, xe, g.xblocks};
+  sp.op[1] = SplitOperand{w, ldw, n, ws, we, g.wblocks};
+  sp.k = k;
+  sp.chunks = g.chunks;
+  const dim3 sgrid(static_cast<uint32_t>(g.xblocks + g.wblocks)), sblock(kSplitThreads);
+  const int64_t per_wave = (g.chunks + kSplitThreads / kWave - 1) / (kSplitThreads / kWave);
+  if (per_wave <= 2)
+    hipLaunchKernelGGL(split_rows_kernel<2>, sgrid, sblock, 0, stream, sp);
+  else if (per_wave <= 4)
+    hipLaunchKernelGGL(split_rows_kernel<4>, sgrid, sblock, 0, stream, sp);
+  else if (per_wave <= 8)
+    hipLaunchKernelGGL(split_rows_kernel<8>, sgrid, sblock, 0, stream, sp);
+  else
+    hipLaunchKernelGGL(split_rows_kernel<0>, sgrid, sblock, 0, stream, sp);
+
+  // The widest tile that still gives every CU two workgroups (512 on 256 CUs):
+  // a workgroup alone on a CU waits out its barriers, and 128 x 128 moves half
+  // the operand bytes per product of 64 x 64. Measured (us, k = 1024): 4096 x
+  // 2048 outputs 53 (128 x 128) / 58 (128 x 64) / 62 (64 x 64), 2048 x 2048
+  // 33.2 / 31.5 / 33.5, 2048 x 512 25.0 / 17.4 / 12.1.
+  constexpr int64_t kFill = 2 * 256;
+  auto tiles = [&](int tn, int tt) { return ((n + tn - 1) / tn) * ((rows + tt - 1) / tt); };
+  auto go = [&](auto kernel, int tn, int tt) {
+    g.tiles_n = (n + tn - 1) / tn;
+    g.tiles_t = (rows + tt - 1) / tt;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(g.tiles_n * g.tiles_t)), dim3(4 * kWave), 0, stream, g);
+  };
+  if (tiles(128, 128) >= kFill)
+    go(split_gemm_kernel<2, 2, 2, 2, 2, 2>, 128, 128);
+  else if (tiles(128, 64) >= kFill)
+    go(split_gemm_kernel<2, 2, 2, 1, 2, 3>, 128, 64);
+  else
+    go(split_gemm_kernel<2, 2, 1, 1, 3, 3>, 64, 64);
+  return hip_status(fn, hipGetLastError());
+}
+
 // Parts per row of the split argmax: about 256 workgroups in all, chunks of at
 // least 2048 columns, at most 64 parts; 1 means the one-kernel path.
 int64_t argmax_parts(int64_t rows, int64_t n) {
@@ -1611,6 +1675,29 @@ int kla_rows_linear_conv_fwd(const float *x, int64_t ldx, const float *w, int64_
   p.conv_k = conv_k;
   p.conv_act = activation;
   return rows_linear_launch(fn, kEpiConv, p, stream);
+}
+
+size_t kla_linear_f32_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
+  if (rows <= 0 || n <= 0 || k <= 0) return 0;
+  const int64_t bytes = linear_f32_bytes(rows, n, k);
+  return bytes >= kHuge ? 0 : static_cast<size_t>(bytes);
+}
+
+int kla_linear_f32_fwd(const float *x, int64_t ldx, const float *w, int64_t ldw, const float *bias, float *y,
+                       int64_t ldy, int64_t rows, int64_t n, int64_t k, void *workspace, size_t workspace_bytes,
+                       hipStream_t stream) {
+  const char *fn = "kla_linear_f32_fwd";
+  if (rows < 0 || n < 0 || k <= 0) return fail(KLA_ERR_INVALID_ARG, "%s: negative size or no columns", fn);
+  if (rows == 0 || n == 0) return KLA_OK;
+  if (!x || !w || !y) return fail(KLA_ERR_INVALID_ARG, "%s: x, w and y must not be NULL", fn);
+  if (ldx < k || ldw < k || ldy < n) return fail(KLA_ERR_INVALID_ARG, "%s: a row stride is below its row length", fn);
+  if (misaligned(x) || misaligned(w) || misaligned(bias) || misaligned(y))
+    return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
+  const int64_t need = linear_f32_bytes(rows, n, k);
+  if (!workspace || need >= kHuge || static_cast<int64_t>(workspace_bytes) < need)
+    return fail(KLA_ERR_WORKSPACE, "%s: a workspace of %lld bytes is needed", fn, (long long)need);
+  if (misaligned_bytes(workspace, 256)) return fail(KLA_ERR_WORKSPACE, "%s: workspace not 256-byte aligned", fn);
+  return linear_f32_launch(fn, x, ldx, w, ldw, bias, y, ldy, rows, n, k, workspace, stream);
 }
 
 int kla_gather_rows(int dtype, const void *table, int64_t ld_table, int64_t vocab, const int64_t *ids, void *out,

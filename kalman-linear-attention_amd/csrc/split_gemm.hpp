@@ -1,0 +1,415 @@
+// split_gemm.hpp -- y = x W^T in fp32 on the fp16 matrix cores, on gfx950.
+//
+// The fp32 MFMA of gfx950 runs at a sixteenth of the fp16 rate. An fp32 value
+// scaled to |s| < 2^15 is the sum of two fp16 values hi = fp16(s) and
+// lo = fp16(s - hi) up to one unit of its own last place (hi carries 11 bits,
+// lo 11 more and the sign a bit), so
+//   x w = hi_x hi_w + hi_x lo_w + lo_x hi_w   (+ lo_x lo_w, below 2^-22 of it)
+// with every product exact and every sum fp32: three MFMA products, a third of
+// the fp16 rate, and sums that round three times a 16-wide step of k instead of
+// up to 16 times, so the result is closer to the exact one than the fp32
+// product's. Relative error (2-norm) against float64, normal entries, this
+// product / the library's fp32 product: k = 512 2.6e-7 / 4.1e-7, k = 1024 3.6e-7
+// / 5.7e-7, k = 1365 4.1e-7 / 6.6e-7, k = 2048 5.0e-7 / 8.1e-7.
+//
+// Each row of x and of W is scaled by the power of two that brings its largest
+// magnitude into [2^14, 2^15); the scales go back in with one ldexp per output.
+// Entries more than 2^17 below their row's largest lose low bits of lo to
+// fp16's smallest spacing, at most 2^-39 of the row's largest value each. A row with an
+// infinity or a NaN is marked instead, and every output it touches is summed in
+// plain fp32 from the original operands (split_exact_outputs).
+//
+// Two kernels. split_rows_kernel writes both operands' hi and lo planes in the
+// order the product reads them: 1 KiB fragments of 32 rows x 16 k, a lane's
+// eight fp16 contiguous, so that the product moves them with 16-byte accesses
+// through LDS and straight into the MFMA operands, with no transposition and no
+// bank conflicts. split_gemm_kernel is the tiled product.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "scan_ops.hpp"
+
+namespace kla {
+
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+constexpr int kSplitRows = 32;                       // rows of a fragment
+constexpr int kSplitK = 32;                          // k of a pair of fragments (a chunk)
+constexpr int kSplitChunk = kSplitRows * kSplitK * 2;   // fp16 of a chunk: 2 k halves x 2 planes x 512
+constexpr int kSplitExp = 14;                        // scaled rows lie in [2^14, 2^15)
+constexpr int kSplitMarked = 1 << 20;                // row exponent of a row with an infinity or NaN
+
+struct SplitOperand {
+  const float *src;    // [rows, k], row stride ld
+  int64_t ld, rows;
+  _Float16 *dst;       // [ceil(rows / 32)][chunks][2 k halves][2 planes][64 lanes][8]
+  int *exps;           // [ceil(rows / 32) * 32]: s = src * 2^(kSplitExp - exp), or kSplitMarked
+  int64_t blocks;      // ceil(rows / 32)
+};
+
+struct SplitParams {
+  SplitOperand op[2];
+  int64_t k;
+  int64_t chunks;      // ceil(k / 32)
+};
+
+// One workgroup takes 32 rows. Lane l of a wave holds, for each of the wave's
+// chunks, the 16 values k = 32 chunk + 16 (l / 32) + 0..15 of row l % 32 (64
+// contiguous bytes: the two halves of a wave read whole 128-byte lines), and
+// fragment f of the chunk is its values 8 f .. 8 f + 7. Which k a lane's eight
+// values are does not matter to the product as long as both operands agree.
+// NC > 0: the chunks of a wave stay in registers between the row maximum and
+// the conversion (at most NC of them); NC = 0 reads the rows twice.
+constexpr int kSplitThreads = 512;
+
+// Four floats at any 4-byte boundary: global loads of gfx950 need no more, so
+// rows of odd length ([512, 1365]) load as widely as aligned ones.
+typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ void split_load16(float (&x)[16], const float *row, int64_t k0, int64_t k) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f32x4_any_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int64_t at = k0 + 4 * i;
+    if (at + 4 <= k) {
+      v = *reinterpret_cast<const f32x4_any_t *>(row + at);
+    } else {
+      if (at < k) v.x = row[at];
+      if (at + 1 < k) v.y = row[at + 1];
+      if (at + 2 < k) v.z = row[at + 2];
+    }
+    x[4 * i] = v.x;
+    x[4 * i + 1] = v.y;
+    x[4 * i + 2] = v.z;
+    x[4 * i + 3] = v.w;
+  }
+}
+
+template <int NC>
+__global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p) {
+  constexpr int NWV = kSplitThreads / kWave;
+  __shared__ uint32_t s_max[NWV][kSplitRows];
+  const bool second = static_cast<int64_t>(blockIdx.x) >= p.op[0].blocks;
+  const SplitOperand &op = p.op[second ? 1 : 0];
+  const int64_t blk = static_cast<int64_t>(blockIdx.x) - (second ? p.op[0].blocks : 0);
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid % kWave, wave = tid / kWave;
+  const int r = lane % kSplitRows, half = lane / kSplitRows;
+  const int64_t row = blk * kSplitRows + r;
+  const bool in = row < op.rows;
+  const float *src = op.src + (in ? row : 0) * op.ld;
+
+  constexpr int HELD = NC > 0 ? NC : 1;
+  float x[HELD][16];
+  uint32_t top = 0;
+  auto scan = [&](const float (&v)[16]) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t b = __float_as_uint(v[i]) & 0x7fffffffu;
+      top = b > top ? b : top;
+    }
+  };
+  if constexpr (NC > 0) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      split_load16(x[i], src, (wave + static_cast<int64_t>(i) * NWV) * kSplitK + 16 * half, in ? p.k : 0);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) scan(x[i]);
+  } else {
+    for (int64_t ch = wave; ch < p.chunks; ch += NWV) {
+      split_load16(x[0], src, ch * kSplitK + 16 * half, in ? p.k : 0);
+      scan(x[0]);
+    }
+  }
+  const uint32_t other = __shfl_xor(top, 32);
+  top = other > top ? other : top;
+  if (half == 0) s_max[wave][r] = top;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NWV; ++w) top = s_max[w][r] > top ? s_max[w][r] : top;
+  const bool marked = top >= 0x7f800000u;
+  // The exponent of the row's largest magnitude (that of 1 for a row of zeros).
+  int ex = 0;
+  if (!marked && top != 0) ex = __builtin_amdgcn_frexp_expf(__uint_as_float(top)) - 1;
+  if (wave == 0 && half == 0) op.exps[row] = marked ? kSplitMarked : ex;
+
+  const int shift = kSplitExp - ex;
+  auto put = [&](const float (&v)[16], int64_t ch) {
+    _Float16 *out = op.dst + (blk * p.chunks + ch) * kSplitChunk + lane * 8;
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      f16x8_t hi, lo;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float s = marked ? 0.0f : ldexpf(v[8 * f + i], shift);
+        hi[i] = static_cast<_Float16>(s);
+        lo[i] = static_cast<_Float16>(s - static_cast<float>(hi[i]));
+      }
+      *reinterpret_cast<f16x8_t *>(out + (2 * f) * 512) = hi;
+      *reinterpret_cast<f16x8_t *>(out + (2 * f + 1) * 512) = lo;
+    }
+  };
+  if constexpr (NC > 0) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int64_t ch = wave + static_cast<int64_t>(i) * NWV;
+      if (ch < p.chunks) put(x[i], ch);
+    }
+  } else {
+    for (int64_t ch = wave; ch < p.chunks; ch += NWV) {
+      split_load16(x[0], src, ch * kSplitK + 16 * half, in ? p.k : 0);
+      put(x[0], ch);
+    }
+  }
+}
+
+struct SplitGemmParams {
+  const _Float16 *xs, *ws;       // split planes of x (tokens) and W (features)
+  const int *xe, *we;            // row exponents
+  const float *x, *w, *bias;     // the fp32 operands (marked rows), bias [n] or NULL
+  float *y;                      // [rows, n], row stride ldy
+  int64_t ldx, ldw, ldy, rows, n, k, chunks;
+  int64_t xblocks, wblocks;      // 32-row blocks of x and of W
+  int64_t tiles_n, tiles_t;      // output tiles over features and tokens
+};
+
+// Outputs of the tile that a marked row touches, one at a time in plain fp32.
+template <int TN, int TT>
+__device__ __forceinline__ void split_exact_outputs(const SplitGemmParams &p, int64_t n0, int64_t t0) {
+  for (int e = static_cast<int>(threadIdx.x); e < TN * TT; e += static_cast<int>(blockDim.x)) {
+    const int64_t n = n0 + e % TN, t = t0 + e / TN;
+    if (n >= p.n || t >= p.rows) continue;
+    if (p.xe[t] != kSplitMarked && p.we[n] != kSplitMarked) continue;
+    const float *a = p.x + t * p.ldx, *b = p.w + n * p.ldw;
+    float s = 0.0f;
+    for (int64_t i = 0; i < p.k; ++i) s = fmaf(a[i], b[i], s);
+    if (p.bias) s += p.bias[n];
+    p.y[t * p.ldy + n] = s;
+  }
+}
+
+typedef __attribute__((address_space(3))) void *lds_ptr_t;
+
+// An array's address in LDS.
+__device__ __forceinline__ uint32_t lds_address(f16x8_t *p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)p));
+}
+
+// One fragment from memory to LDS address `dst`, 16 bytes a lane in lane order
+// (`src` and `dst` the same in every lane). Written out, because the compiler cannot tell the
+// stages of a kernel apart and would wait for every load in flight before each
+// read of LDS; the caller holds the waits. No register is loaded, the address
+// registers are read as the load issues, and m0 (the LDS address) is put back.
+__device__ __forceinline__ void fragment_to_lds(const char *src, uint32_t lane_off, uint32_t dst) {
+#ifdef __OPTIMIZE__
+  uint32_t m0;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+               : "=&s"(m0)
+               : "s"(dst), "v"(lane_off), "s"(src)
+               : "memory");
+#else
+  // (An unoptimised build keeps no value in a scalar register.)
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + lane_off),
+                                   (lds_ptr_t)static_cast<uintptr_t>(dst), 16, 0, 0);
+#endif
+}
+
+// WAVN x WAVT waves, each FN x FT fragments of 32 features x 32 tokens. W is
+// the MFMA's A operand, so a lane ends with four consecutive features of one
+// token (D[8 (i / 4) + 4 (lane / 32) + i % 4][lane % 32]) and stores them as one
+// 16-byte word. Chunks of 32 k go straight from memory into ST stages of LDS,
+// ST - 1 chunks ahead of the products.
+//
+// Bound by the matrix cores, which draw the clock down at this load (torch's
+// bf16 product of 8192^3 reaches 1.32 PFLOP/s here; 382 TFLOP/s of fp32 product
+// are 1.15 of fp16). Both kernels / the library's fp32 product, us:
+//   8188 x 4096, k 2048   360 + 43 /  967      4096 x 50304, k 512  745 + 36 / 1528
+//   8188 x 1024, k 2048    96 + 39 /  258      4096 x 2048, k 1024   53 + 11 /  124
+//   2048 x 2048, k 1024    32 + 10 /   72       256 x 2048, k 512     8 +  8 /   20
+// Through registers instead of straight into LDS, one chunk ahead: 426 us for the
+// first; with the compiler's waits (every load before each read of LDS) 397.
+template <int WAVN, int WAVT, int FN, int FT, int ST, int OCC>
+__global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(SplitGemmParams p) {
+  constexpr int NW = WAVN * WAVT;
+  constexpr int BN = WAVN * FN, BT = WAVT * FT;          // 32-row blocks of the tile
+  constexpr int TN = BN * kSplitRows, TT = BT * kSplitRows;
+  constexpr int FRAGS = (BN + BT) * 4;                   // 1 KiB fragments of a chunk (2 halves x 2 planes)
+  constexpr int LD = FRAGS / NW;
+  static_assert(FRAGS % NW == 0, "whole fragments per wave");
+  static_assert(ST >= 2 && ST <= 4, "2 to 4 stages");
+  // One array per stage: a stage's reads then wait for that stage's loads only.
+  __shared__ f16x8_t s_0[FRAGS * 64], s_1[FRAGS * 64], s_2[ST > 2 ? FRAGS * 64 : 1], s_3[ST > 3 ? FRAGS * 64 : 1];
+  __shared__ __align__(16) int s_we[TN];
+  __shared__ __align__(16) float s_bias[TN];
+  __shared__ int s_xe[TT];
+
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wn = wave % WAVN, wt = wave / WAVN;
+
+  // Workgroup i runs on XCD i % 8; give each XCD a contiguous run of tiles, and
+  // walk those in bands of 8 feature tiles so that the tiles in flight on an XCD
+  // share operand rows in its L2.
+  int64_t idx = blockIdx.x;
+  const int64_t total = p.tiles_n * p.tiles_t;
+  if (total % 8 == 0) idx = (idx % 8) * (total / 8) + idx / 8;
+  constexpr int64_t BAND = 8;
+  const int64_t band = idx / (BAND * p.tiles_t);
+  const int64_t width = p.tiles_n - band * BAND < BAND ? p.tiles_n - band * BAND : BAND;
+  const int64_t rest = idx - band * BAND * p.tiles_t;
+  const int64_t tn = band * BAND + rest % width, tt = rest / width;
+
+  // Fragment wave + j NW of the tile's FRAGS: block / 4, half and plane % 4.
+  const char *from[LD];
+#pragma unroll
+  for (int j = 0; j < LD; ++j) {
+    const int e = wave + j * NW;
+    const int b = e / 4;
+    const bool isw = b < BN;
+    int64_t blk = isw ? tn * BN + b : tt * BT + (b - BN);
+    const int64_t last = (isw ? p.wblocks : p.xblocks) - 1;
+    blk = blk < last ? blk : last;      // rows past the end: any block, never stored
+    from[j] = reinterpret_cast<const char *>((isw ? p.ws : p.xs) + blk * p.chunks * kSplitChunk) + (e % 4) * 1024;
+  }
+  const uint32_t lane_off = static_cast<uint32_t>(lane) * 16;
+  auto load = [&](f16x8_t *stage, int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < LD; ++j)
+      fragment_to_lds(from[j] + static_cast<int64_t>(c) * (kSplitChunk * 2), lane_off,
+                      lds_address(stage) + (wave + j * NW) * 1024);
+  };
+
+  f32x16_t acc[FN][FT];
+#pragma unroll
+  for (int a = 0; a < FN; ++a)
+#pragma unroll
+    for (int b = 0; b < FT; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.0f;
+
+  auto products = [&](const f16x8_t *stage) __attribute__((always_inline)) {
+    const f16x8_t *sw = stage + wn * FN * 256 + lane;
+    const f16x8_t *sx = stage + (BN + wt * FT) * 256 + lane;
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      f16x8_t wh[FN], wl[FN], xh[FT], xl[FT];
+#pragma unroll
+      for (int a = 0; a < FN; ++a) {
+        wh[a] = sw[a * 256 + (2 * f) * 64];
+        wl[a] = sw[a * 256 + (2 * f + 1) * 64];
+      }
+#pragma unroll
+      for (int b = 0; b < FT; ++b) {
+        xh[b] = sx[b * 256 + (2 * f) * 64];
+        xl[b] = sx[b * 256 + (2 * f + 1) * 64];
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int a = 0; a < FN; ++a)
+#pragma unroll
+          for (int b = 0; b < FT; ++b)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(q == 0 ? wl[a] : wh[a], q == 1 ? xl[b] : xh[b],
+                                                               acc[a][b], 0, 0, 0);
+    }
+  };
+  const int chunks = static_cast<int>(p.chunks);
+  // Chunk c: wait for its loads (those of the ST - 2 chunks after it stay in
+  // flight) and for every wave to be done with the chunk before it, refill that
+  // chunk's stage, multiply. Past the end the last chunk is loaded again, so
+  // that the count in flight is the same for every chunk.
+  auto turn = [&](int c, f16x8_t *stage, f16x8_t *refill) __attribute__((always_inline)) {
+    constexpr int kInFlight = LD * (ST - 2);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kInFlight) : "memory");
+    load(refill, c + ST - 1 < chunks ? c + ST - 1 : chunks - 1);
+    products(stage);
+  };
+  load(s_0, 0);
+  if constexpr (ST > 2) load(s_1, chunks > 1 ? 1 : chunks - 1);
+  if constexpr (ST > 3) load(s_2, chunks > 2 ? 2 : chunks - 1);
+  // The tile's row exponents and bias, for the epilogue (they arrive with the first chunks).
+  const int64_t n0 = tn * TN, t0 = tt * TT;
+  bool marked = false;
+  for (int i = tid; i < TN + TT; i += NW * kWave) {
+    const bool isn = i < TN;
+    const int64_t r = isn ? n0 + i : t0 + (i - TN);
+    const bool in = r < (isn ? p.n : p.rows);
+    const int e = in ? (isn ? p.we : p.xe)[r] : 0;
+    marked = marked || e == kSplitMarked;
+    if (isn) {
+      s_we[i] = e - 2 * kSplitExp;
+      s_bias[i] = in && p.bias ? p.bias[r] : 0.0f;
+    } else {
+      s_xe[i - TN] = e;
+    }
+  }
+  int c = 0;
+  if constexpr (ST == 2) {
+    for (; c + 2 <= chunks; c += 2) {
+      turn(c, s_0, s_1);
+      turn(c + 1, s_1, s_0);
+    }
+    if (c < chunks) turn(c, s_0, s_1);
+  } else if constexpr (ST == 3) {
+    for (; c + 3 <= chunks; c += 3) {
+      turn(c, s_0, s_2);
+      turn(c + 1, s_1, s_0);
+      turn(c + 2, s_2, s_1);
+    }
+    if (c < chunks) turn(c, s_0, s_2);
+    if (c + 1 < chunks) turn(c + 1, s_1, s_0);
+  } else {
+    for (; c + 4 <= chunks; c += 4) {
+      turn(c, s_0, s_3);
+      turn(c + 1, s_1, s_0);
+      turn(c + 2, s_2, s_1);
+      turn(c + 3, s_3, s_2);
+    }
+    if (c < chunks) turn(c, s_0, s_3);
+    if (c + 1 < chunks) turn(c + 1, s_1, s_0);
+    if (c + 2 < chunks) turn(c + 2, s_2, s_1);
+  }
+  // No load into this workgroup's LDS may outlive it.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  const bool vec = p.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(p.y) % 16 == 0;
+#pragma unroll
+  for (int a = 0; a < FN; ++a)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int nl = (wn * FN + a) * kSplitRows + 8 * g + 4 * (lane / 32);
+      const int4 en = *reinterpret_cast<const int4 *>(s_we + nl);
+      const float4 bv = *reinterpret_cast<const float4 *>(s_bias + nl);
+      const int64_t n = n0 + nl;
+#pragma unroll
+      for (int b = 0; b < FT; ++b) {
+        const int tl = (wt * FT + b) * kSplitRows + lane % 32;
+        const int64_t t = t0 + tl;
+        const int ex = s_xe[tl];
+        const float4 v = make_float4(ldexpf(acc[a][b][4 * g], ex + en.x) + bv.x,
+                                     ldexpf(acc[a][b][4 * g + 1], ex + en.y) + bv.y,
+                                     ldexpf(acc[a][b][4 * g + 2], ex + en.z) + bv.z,
+                                     ldexpf(acc[a][b][4 * g + 3], ex + en.w) + bv.w);
+        if (t < p.rows) {
+          float *out = p.y + t * p.ldy + n;
+          if (vec && n + 4 <= p.n) {
+            *reinterpret_cast<float4 *>(out) = v;
+          } else {
+            if (n < p.n) out[0] = v.x;
+            if (n + 1 < p.n) out[1] = v.y;
+            if (n + 2 < p.n) out[2] = v.z;
+            if (n + 3 < p.n) out[3] = v.w;
+          }
+        }
+      }
+    }
+  // Marked rows or columns: their outputs once more, from the operands. (The
+  // barrier orders the two stores.)
+  if (__syncthreads_or(marked)) split_exact_outputs<TN, TT>(p, n0, t0);
+}
+
+}  // namespace kla

@@ -51,6 +51,16 @@ def _hip_inference(backend: str, *tensors: torch.Tensor) -> bool:
     return _step_on_hip(backend, tensors[0])
 
 
+def _project(backend: str, mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """mod(x); in inference on a hip-family ``backend`` the split fp32 product where it
+    applies (kla.ops.hip.linear.plain_linear)."""
+    if x.dtype == torch.float32 and _hip_inference(backend, x, *mod.parameters()):
+        from kla.ops.hip.linear import plain_linear
+
+        return plain_linear(mod, x)
+    return mod(x)
+
+
 class RMSNorm(nn.Module):
     """x * rsqrt(mean(x^2) + eps) * weight, computed in float32.
 
@@ -166,11 +176,11 @@ class MLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.kind == "swiglu":
-            h = self.w12(x)
+            h = _project(self.backend, self.w12, x)
             if h.dtype in (torch.float32, torch.bfloat16) and _hip_inference(self.backend, h):
                 from kla.ops.hip.model_ops import swiglu_hip
 
-                return self.w3(swiglu_hip(h))
+                return _project(self.backend, self.w3, swiglu_hip(h))
             gate, up = h.chunk(2, dim=-1)
             return self.w3(F.silu(gate) * up)
-        return self.w2(F.gelu(self.w1(x)))
+        return _project(self.backend, self.w2, F.gelu(_project(self.backend, self.w1, x)))

@@ -157,6 +157,7 @@ class KLALayer(nn.Module):
             # Inference at few tokens: value and variance columns as one hipBLASLt
             # product, k and q with their norm and clip as one HIP kernel (a 2S-row
             # tail would otherwise set hipBLASLt's tile for the whole product).
+            from kla.ops.hip.linear import linear_f32, linear_f32_ok
             from kla.ops.hip.sensors import qk_project_hip
 
             w, b = self.sensor_proj.weight, self.sensor_proj.bias
@@ -164,22 +165,23 @@ class KLALayer(nn.Module):
             B, L, _ = z.shape
             k, q = qk_project_hip(z.reshape(B * L, z.shape[-1]), w[n1:], None if b is None else b[n1:], S,
                                   norm=cfg.qk_norm, clip=cfg.clip_value)
-            v, log_var = torch.split(F.linear(z, w[:n1], None if b is None else b[:n1]),
-                                     [self._w_value, self._w_var], dim=-1)
+            b1 = None if b is None else b[:n1]
+            product = linear_f32 if linear_f32_ok(z, w[:n1], b1) else F.linear
+            v, log_var = torch.split(product(z, w[:n1], b1), [self._w_value, self._w_var], dim=-1)
             if self._value_rank == "conv":
                 v = z
             elif self.value_expand is not None:
-                v = self.value_expand(v)
+                v = self._expand(self.value_expand, v)
             if self.var_expand is not None:
-                log_var = self.var_expand(log_var)
+                log_var = self._expand(self.var_expand, log_var)
             return v, log_var, k.view(B, L, S), q.view(B, L, S)
         v, log_var, k, q = self._linear_split(self.sensor_proj, z, [self._w_value, self._w_var, S, S])
         if self._value_rank == "conv":
             v = z
         elif self.value_expand is not None:
-            v = self.value_expand(v)
+            v = self._expand(self.value_expand, v)
         if self.var_expand is not None:
-            log_var = self.var_expand(log_var)
+            log_var = self._expand(self.var_expand, log_var)
         if self._qk_on_hip(k):
             # Norm, clip and .float() of both as one HIP kernel each way (same values).
             from kla.ops.hip.sensors import qk_sensors_hip
@@ -257,21 +259,29 @@ class KLALayer(nn.Module):
 
     def _linear(self, mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
         """mod(x); on a hip-family backend with a gradient to carry, the projection
-        whose weight gradient is split over the tokens (kla.ops.hip.linear)."""
-        if torch.is_grad_enabled() and _step_on_hip(self.config.backend, x):
-            from kla.ops.hip.linear import linear
+        whose weight gradient is split over the tokens, and without one the split
+        fp32 product where it applies (kla.ops.hip.linear)."""
+        if _step_on_hip(self.config.backend, x):
+            from kla.ops.hip.linear import linear, plain_linear
 
-            return linear(mod, x)
+            return linear(mod, x) if torch.is_grad_enabled() else plain_linear(mod, x)
         return mod(x)
+
+    def _expand(self, mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
+        """mod(x) for the low-rank value and variance maps; without a gradient on a
+        hip-family backend as :meth:`_linear`."""
+        return mod(x) if torch.is_grad_enabled() else self._linear(mod, x)
 
     def _linear_split(self, mod: nn.Linear, x: torch.Tensor, sizes: list[int]):
         """self._split(mod(x), sizes); on a hip-family backend with a gradient to
         carry, the projection and the split as one (kla.ops.hip.linear), and
-        otherwise the product in row blocks where the pieces allow it
-        (kla.ops.hip.linear.split_blocks)."""
+        otherwise the split fp32 product, or the product in row blocks where the
+        pieces allow it (kla.ops.hip.linear.plain_linear, split_blocks)."""
         if _step_on_hip(self.config.backend, x):
-            from kla.ops.hip.linear import linear_split, split_blocks
+            from kla.ops.hip.linear import _bare, linear_f32_ok, linear_split, plain_linear, split_blocks
 
+            if not torch.is_grad_enabled() and _bare(mod) and linear_f32_ok(x, mod.weight, mod.bias):
+                return torch.split(plain_linear(mod, x), sizes, dim=-1)
             pieces = linear_split(mod, x, sizes) if torch.is_grad_enabled() else None
             if pieces is None and not (torch.is_grad_enabled() and x.requires_grad):
                 pieces = split_blocks(mod, x, sizes)

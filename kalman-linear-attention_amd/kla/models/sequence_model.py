@@ -16,7 +16,7 @@ import torch
 import torch.nn as nn
 
 from kla.configs import KLAConfig, ModelConfig
-from kla.layers.common import MLP, RMSNorm
+from kla.layers.common import MLP, RMSNorm, _project
 from kla.layers.kla_layer import KLALayer
 from kla.models.readout import MarginalReadout
 
@@ -137,7 +137,7 @@ class SequenceModel(MarginalReadout, nn.Module):
                                      norm_weight=self.norm_f.weight, eps=self.norm_f.eps)
             logits = logits.reshape(*x.shape[:-1], logits.shape[-1])
         else:
-            logits = self.lm_head(self.norm_f(x))
+            logits = _project(self.norm_f.backend, self.lm_head, self.norm_f(x))
         cap = self.config.logit_softcap
         return logits if cap is None else cap * torch.tanh(logits / cap)
 
@@ -191,7 +191,7 @@ class SequenceModel(MarginalReadout, nn.Module):
     def _head(self, x: torch.Tensor) -> torch.Tensor:
         """Last channel mixer + final norm + LM head + softcap, as log-probabilities."""
         x = self._last_block.channel(x)
-        logits = self.lm_head(self.norm_f(x)).float()
+        logits = _project(self.norm_f.backend, self.lm_head, self.norm_f(x)).float()
         cap = self.config.logit_softcap
         if cap is not None:
             logits = cap * torch.tanh(logits / cap)

@@ -19,7 +19,7 @@ import torch
 # one the ABI tests run against); by default the in-tree libkla_hip.so.
 LIB_PATH = os.environ.get("KLA_HIP_LIB") or os.path.join(
     os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)))), "lib", "libkla_hip.so")
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 KLA_OK = 0
 KLA_ERR_INVALID_ARG = 1
@@ -96,6 +96,9 @@ _SIGNATURES = {
     "kla_argmax_workspace_bytes": (ctypes.c_size_t, [_i64, _i64]),
     "kla_rows_linear_fwd": (ctypes.c_int, [ctypes.c_int, _p, _i64, _p, _i64, _p, _p, ctypes.c_float, _p, _i64, _p,
                                            _i64, _i64, _i64, _i64, _i64, _p]),
+    "kla_linear_f32_workspace_bytes": (ctypes.c_size_t, [_i64] * 3),
+    "kla_linear_f32_fwd": (ctypes.c_int, [_p, _i64, _p, _i64, _p, _p, _i64, _i64, _i64, _i64, _p, ctypes.c_size_t,
+                                          _p]),
     "kla_gate_skip_bwd": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _p, _p, _p, _i64, _p, _i64, _p, ctypes.c_int,
                                          ctypes.c_int] + [_p] * 4 + [_i64] * 2 + [_p, ctypes.c_size_t, _p]),
     "kla_causal_conv_bwd": (ctypes.c_int, [ctypes.c_int, _p, _p, _i64, _i64, _p, _p, _p, ctypes.c_int, _p, _p, _p,

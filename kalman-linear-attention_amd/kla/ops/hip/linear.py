@@ -24,16 +24,22 @@ taken in row blocks of whole 256-row tiles plus the rest (``sensor_proj``'s
 4128 rows: 4096 + 32), each block one forward product and one split weight
 gradient, so a ragged last tile row does not slow the whole product (C4's
 sensor_proj forward 304 -> 231 us, weight gradient 370 -> 294 us on MI355X).
+
+:func:`linear_f32` is the fp32 product of inference over a sequence, on the fp16
+matrix cores from split operands (``kla_linear_f32_fwd``); :func:`plain_linear`
+takes it for an ``nn.Linear`` where :func:`linear_f32_ok` holds.
 """
 
 from __future__ import annotations
 
 import functools
+from typing import Optional
 
 import torch
 import torch.nn.functional as F
 
 from kla.ops.hip import _lib
+from kla.ops.hip.scans import _require_device
 from kla.ops.hip.split import _Like, cat_cols_hip
 
 # At most this many token chunks per weight gradient, each at least this long.
@@ -260,3 +266,83 @@ def linear_split(mod: torch.nn.Linear, x: torch.Tensor, sizes: list[int]):
         return None
     with torch.autocast("cuda", enabled=False):
         return _SplitLinear.apply(*ops, list(sizes))
+
+
+# ------------------------------------------------------------- fp32 inference
+
+# Fewest rows for linear_f32. Its two kernels take 7.5 + 8 us at least; the library
+# product of 256 to 512 rows takes 19 us (x [256, 512], W [2048, 512]: 15.2 against
+# 20; x [2048, 512], W [2048, 512]: 28 against 42), and below 256 rows the two meet.
+F32_MIN_ROWS = 256
+
+
+@_lib.hip_op("kla_hip::linear_f32")
+def _linear_f32_op(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+    k = x.shape[-1]
+    n = w.shape[0]
+    x2 = x.reshape(-1, k)
+    rows = x2.shape[0]
+    lib = _lib.lib()
+    nbytes = lib.kla_linear_f32_workspace_bytes(rows, n, k)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    y = torch.empty(x.shape[:-1] + (n,), dtype=torch.float32, device=x.device)
+    _lib.check("kla_linear_f32_fwd", lib.kla_linear_f32_fwd(
+        x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), _lib.ptr(bias), y.data_ptr(), n, rows, n, k,
+        ws.data_ptr(), nbytes, _lib.stream(x.device)))
+    return y
+
+
+@_linear_f32_op.register_fake
+def _(x, w, bias):
+    return x.new_empty(x.shape[:-1] + (w.shape[0],))
+
+
+def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``F.linear(x, w, bias)`` for fp32 x [..., k], w [n, k] (k > 0), bias [n] on one
+    ROCm GPU, on the fp16 matrix cores from split operands: fp32 sums of exact
+    products, no larger an error than the fp32 product's (measured against float64
+    at k = 512, 1024, 2048: 0.63 of it). No gradient."""
+    if x.dtype != torch.float32 or w.dtype != torch.float32 or (bias is not None and bias.dtype != torch.float32):
+        raise TypeError("linear_f32: x, w and bias must be float32")
+    k = x.shape[-1] if x.dim() else 0
+    if w.dim() != 2 or w.shape[1] != k or k == 0 or (bias is not None and tuple(bias.shape) != (w.shape[0],)):
+        raise ValueError(f"linear_f32: x {tuple(x.shape)}, w {tuple(w.shape)}, "
+                         f"bias {None if bias is None else tuple(bias.shape)}")
+    _require_device(x, w, bias)
+    if x.stride(-1) != 1 or (x.dim() > 1 and x.stride(-2) < k):
+        x = x.contiguous()
+    if w.stride(1) != 1 or w.stride(0) < k:
+        w = w.contiguous()
+    if bias is not None and bias.stride(0) != 1:
+        bias = bias.contiguous()
+    return _lib.call(_linear_f32_op, x, w, bias)
+
+
+def linear_f32_ok(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
+    """Whether ``F.linear(x, w, bias)`` of a hip-family module runs as
+    :func:`linear_f32`: fp32 on a ROCm GPU outside autocast, no gradient to carry,
+    and at least F32_MIN_ROWS rows."""
+    k = w.shape[-1]
+    if (x.dtype != torch.float32 or w.dtype != torch.float32 or not x.is_cuda or k == 0 or w.shape[0] == 0
+            or x.numel() < F32_MIN_ROWS * k or x.shape[-1] != k or w.device != x.device):
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)):
+        return False
+    return not torch.is_autocast_enabled("cuda") and (bias is None or bias.dtype == torch.float32)
+
+
+def _bare(mod: torch.nn.Module) -> bool:
+    """Whether calling ``mod`` is F.linear on its weight and bias and nothing else: an
+    nn.Linear itself, not a subclass (nor a parametrised one), with no hooks and
+    plain parameters."""
+    hooks = torch.nn.modules.module
+    return (type(mod) is torch.nn.Linear and not (mod._forward_hooks or mod._forward_pre_hooks
+                                                  or hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
+            and type(mod.weight) in (torch.Tensor, torch.nn.Parameter))
+
+
+def plain_linear(mod: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``mod(x)`` for a hip-family module's nn.Linear, as :func:`linear_f32` where it applies."""
+    if _bare(mod) and linear_f32_ok(x, mod.weight, mod.bias):
+        return linear_f32(x, mod.weight, mod.bias)
+    return mod(x)

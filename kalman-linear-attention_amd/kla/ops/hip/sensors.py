@@ -94,11 +94,11 @@ def qk_sensors_hip(k: torch.Tensor, q: torch.Tensor, *, norm: bool, clip: float 
 
 
 # Token counts below which the k, q columns of the sensor projection run as
-# kla_rows_linear_qk_fwd: at 2048 tokens (k = 1024, S = 16) its product, norm and
-# clip take ~9 us against ~19 us for hipBLASLt's 32-row product alone (plus the
-# qk sensor kernel); at 32768 tokens hipBLASLt's product is the faster (23
-# against 68 us).
-QK_PROJECT_MAX_TOKENS = 8192
+# kla_rows_linear_qk_fwd, apart from the value and variance columns: with the split
+# fp32 product (kla.ops.hip.linear.linear_f32) for those, a layer's forward of width
+# 512 takes 292 us at 4096 tokens against 299 with one product for all columns and
+# the sensor kernel after it, and 1133 against 1116 us at 8188 tokens of width 1024.
+QK_PROJECT_MAX_TOKENS = 6144
 
 
 def qk_project_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, S: int, *, norm: bool,
