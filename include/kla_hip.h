@@ -321,6 +321,28 @@ int kla_adjoint_ends(const float *maps, const float *dlam_fin, const float *deta
                      int64_t batch, int64_t chunks, int64_t M, int64_t S, hipStream_t stream);
 
 /*
+ * The time split in one call, forward and backward, at any sequence length:
+ * chunks of chunk_steps steps (a multiple of 16 below steps), the last one
+ * shorter. The values of kla_fused_scan_sensors_fwd / _bwd on whole sequences up
+ * to the rounding of the chunk maps; same operands (dlam0, deta0 may be NULL). A
+ * backward needs the checkpoints of a forward over the same batch and steps,
+ * split or not. workspace: 256-byte aligned, at least
+ * kla_fused_split_workspace_bytes, contents not kept.
+ */
+size_t kla_fused_split_workspace_bytes(int64_t batch, int64_t steps, int64_t M, int64_t S, int64_t chunk_steps,
+                                       int backward);
+int kla_fused_split_fwd(const kla_sensors *sensors, const float *k, const float *q, const float *a, const float *p,
+                        const float *lam0, const float *eta0, float *y, float *y_var, float *lam_fin, float *eta_fin,
+                        float *ck_lam, float *ck_eta, int decode_from_prior, int64_t batch, int64_t steps, int64_t M,
+                        int64_t S, int64_t chunk_steps, void *workspace, size_t workspace_bytes, hipStream_t stream);
+int kla_fused_split_bwd(const float *dy, const float *dy_var, const float *dlam_fin, const float *deta_fin,
+                        const kla_sensors *sensors, const float *k, const float *q, const float *a, const float *p,
+                        const float *ck_lam, const float *ck_eta, void *dv, void *dobs, float *dk, float *dq,
+                        float *da, float *dp, float *dlam0, float *deta0, int decode_from_prior, int64_t batch,
+                        int64_t steps, int64_t M, int64_t S, int64_t chunk_steps, void *workspace,
+                        size_t workspace_bytes, hipStream_t stream);
+
+/*
  * One O(1) decode step of the filter for every (b, m, s) lane: kla_step
  * (reference src/kla/ops/kla_ops.py:293-331), phi floored at 1e-12 as there.
  * v, lambda_v, y, y_var [batch, M]; k, q [batch, S]; a, p [M, S]; lam, eta,

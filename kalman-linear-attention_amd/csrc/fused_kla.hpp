@@ -52,7 +52,25 @@ struct FusedGeom {
   int64_t batch, steps, M, S;
   int64_t groups;   // ceil(M / CH): channel groups (workgroups) per batch row
   int64_t n_ck;     // ceil(steps / kCkpt)
+  // A time split runs the chunks of a sequence of `steps` steps as batch rows
+  // (`batch` counts them): chunk_steps each, a multiple of kCkpt, the last one
+  // shorter. chunks = 1 and chunk_steps = steps: whole sequences.
+  int64_t chunks, chunk_steps;
 };
+
+// What batch row b of the grid covers: `steps` steps from row `row0` of the
+// [B L, .] tensors, and checkpoints from `ck0` of the [B n_ck, .] ones.
+struct FusedSpan {
+  int64_t row0, steps, ck0, n_ck;
+};
+
+__device__ __forceinline__ FusedSpan fused_span(const FusedGeom &g, int64_t b) {
+  if (g.chunks == 1) return FusedSpan{b * g.steps, g.steps, b * g.n_ck, g.n_ck};
+  const int64_t seq = b / g.chunks, t0 = (b % g.chunks) * g.chunk_steps;
+  const int64_t left = g.steps - t0;
+  const int64_t steps = left < g.chunk_steps ? left : g.chunk_steps;
+  return FusedSpan{seq * g.steps + t0, steps, seq * g.n_ck + t0 / kCkpt, (steps + kCkpt - 1) / kCkpt};
+}
 
 // The [B, L, M] sensor inputs v and the precision operand: rows of stride ld
 // (element (b, t, m) at (b * L + t) * ld + m, so they can be column slices of
@@ -585,7 +603,8 @@ __global__ void __launch_bounds__(kFusedThreads)
   __shared__ float s_y[2][WPC][CH][TB + kPad], s_yv[2][WPC][CH][TB + kPad];
 
   const FusedLane ln = fused_lane<SP>(g);
-  const int64_t M = g.M, S = g.S, L = g.steps;
+  const FusedSpan span = fused_span(g, ln.b);
+  const int64_t M = g.M, S = g.S, L = span.steps, row0 = span.row0;
   const int64_t m0 = (xcd_block() % g.groups) * CH;
   const int c = static_cast<int>(ln.m - m0);
   const int64_t ms = ln.m * S + ln.s;
@@ -600,17 +619,17 @@ __global__ void __launch_bounds__(kFusedThreads)
   float eta = (ln.active && prm.eta0) ? prm.eta0[bms] : 0.0f;
 
   const SensorIn &sn = prm.sn;
-  const float *kbase = prm.k + ln.b * L * S;
-  const float *qbase = prm.q + ln.b * L * S;
-  float *ybase = prm.y + ln.b * L * M + m0;
-  float *yvbase = VAR ? prm.yvar + ln.b * L * M + m0 : nullptr;
+  const float *kbase = prm.k + row0 * S;
+  const float *qbase = prm.q + row0 * S;
+  float *ybase = prm.y + row0 * M + m0;
+  float *yvbase = VAR ? prm.yvar + row0 * M + m0 : nullptr;
 
   TileRegs<TB, CH> rv, rl;
   TileRegs<TB, SP> rk, rq;
   auto load = [&](int64_t t0) {
     const int64_t rows = L - t0;
-    tile_load_sensor<TB, CH, BF16>(rv, sensor_at<BF16>(sn.v, ln.b * L + t0, m0, sn.ld_v), sn.ld_v, rows, cols_m);
-    tile_load_sensor<TB, CH, BF16>(rl, sensor_at<BF16>(sn.lv, ln.b * L + t0, m0, sn.ld_lv), sn.ld_lv, rows, cols_m);
+    tile_load_sensor<TB, CH, BF16>(rv, sensor_at<BF16>(sn.v, row0 + t0, m0, sn.ld_v), sn.ld_v, rows, cols_m);
+    tile_load_sensor<TB, CH, BF16>(rl, sensor_at<BF16>(sn.lv, row0 + t0, m0, sn.ld_lv), sn.ld_lv, rows, cols_m);
     tile_load<TB, SP>(rk, kbase + t0 * S, S, rows, S);
     tile_load<TB, SP>(rq, qbase + t0 * S, S, rows, S);
   };
@@ -626,7 +645,7 @@ __global__ void __launch_bounds__(kFusedThreads)
   };
 
   // Checkpoint of the state entering step t: ck[((b * n_ck + t / kCkpt) * M + m) * S + s].
-  const int64_t ck_off = (ln.b * g.n_ck * M + ln.m) * S + ln.s;
+  const int64_t ck_off = (span.ck0 * M + ln.m) * S + ln.s;
   const int64_t ck_stride = M * S;
   static_assert(TB % kCkpt == 0, "checkpoints must fall on half-block boundaries");
 
@@ -781,7 +800,8 @@ __global__ void __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per
   constexpr bool kFullBlocks = SP >= 16 && SP <= 64 && !PRIOR && !VAR;
 
   const FusedLane ln = fused_lane<SP>(g);
-  const int64_t M = g.M, S = g.S, L = g.steps;
+  const FusedSpan span = fused_span(g, ln.b);
+  const int64_t M = g.M, S = g.S, L = span.steps, row0 = span.row0;
   const int64_t grp = xcd_block() % g.groups;
   const int64_t m0 = grp * CH;
   const int c = static_cast<int>(ln.m - m0);
@@ -802,14 +822,14 @@ __global__ void __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per
   float ge = (ln.active && prm.deta_fin) ? prm.deta_fin[bms] : 0.0f;   // adjoint of eta_t
   float acc_a = 0.0f, acc_a2 = 0.0f, acc_p = 0.0f;
 
-  const int64_t offM = ln.b * L * M + m0, offS = ln.b * L * S;
+  const int64_t offM = row0 * M + m0, offS = row0 * S;
   const SensorIn &sn = prm.sn;
   TileRegs<TB, CH> rv, rl, rdy, rdyv;
   TileRegs<TB, SP> rk, rq;
   auto load = [&](int64_t t0) {
     const int64_t rows = L - t0;
-    tile_load_sensor<TB, CH, BF16>(rv, sensor_at<BF16>(sn.v, ln.b * L + t0, m0, sn.ld_v), sn.ld_v, rows, cols_m);
-    tile_load_sensor<TB, CH, BF16>(rl, sensor_at<BF16>(sn.lv, ln.b * L + t0, m0, sn.ld_lv), sn.ld_lv, rows, cols_m);
+    tile_load_sensor<TB, CH, BF16>(rv, sensor_at<BF16>(sn.v, row0 + t0, m0, sn.ld_v), sn.ld_v, rows, cols_m);
+    tile_load_sensor<TB, CH, BF16>(rl, sensor_at<BF16>(sn.lv, row0 + t0, m0, sn.ld_lv), sn.ld_lv, rows, cols_m);
     tile_load<TB, CH>(rdy, prm.dy + offM + t0 * M, M, rows, cols_m);
     if constexpr (VAR) tile_load<TB, CH>(rdyv, prm.dyvar + offM + t0 * M, M, rows, cols_m);
     tile_load<TB, SP>(rk, prm.k + offS + t0 * S, S, rows, S);
@@ -861,12 +881,12 @@ __global__ void __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per
 #pragma unroll
         for (int w = 0; w < NW / WPC; ++w) sum += s_red[RB == 1 ? 0 : buf][which][j][w][s];
         float *part = which == 0 ? prm.part_k : prm.part_q;
-        part[((ln.b * L + t) * g.groups + grp) * S + s] = sum;
+        part[((row0 + t) * g.groups + grp) * S + s] = sum;
       }
     }
   };
 
-  const int64_t n_ck = g.n_ck;
+  const int64_t n_ck = span.n_ck;
   // The checkpoint entering a block is read one block ahead, with the block's
   // tiles: a load issued just before the replay would make the replay wait for
   // every load still in flight (memory counters retire in order), the next
@@ -874,7 +894,7 @@ __global__ void __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per
   float ck_l = 1.0f, ck_e = 0.0f;
   auto load_ck = [&](int64_t blk) {
     if (ln.active) {
-      const int64_t ci = ((ln.b * n_ck + blk) * M + ln.m) * S + ln.s;
+      const int64_t ci = ((span.ck0 + blk) * M + ln.m) * S + ln.s;
       ck_l = prm.ck_lam[ci];
       ck_e = prm.ck_eta[ci];
     }
@@ -1252,9 +1272,11 @@ __global__ void reduce_groups_kernel(const float *__restrict__ in, float *__rest
 // ============================================= time-split forward (inference)
 //
 // With few chains (batch * M * S) the lane-serial forward leaves CUs idle. For a
-// forward without a backward the sequence can be cut into `chunks` equal pieces
-// run side by side: a [B, L, .] tensor viewed as [B * chunks, L / chunks, .] is
-// the same memory, with sequence b's chunk c at b' = b * chunks + c.
+// forward without a backward the sequence can be cut into `chunks` pieces run
+// side by side, sequence b's chunk c as batch row b' = b * chunks + c: equal
+// pieces are the same memory viewed as [B * chunks, L / chunks, .], and a length
+// that equal pieces do not divide takes chunk_steps each with a shorter last one
+// (FusedGeom).
 //
 // The state entering each chunk comes from one pass over the chunks and one
 // walk along them. In homogeneous coordinates lam = N / D, eta = W / D a step of
@@ -1286,7 +1308,8 @@ __global__ void __launch_bounds__(kFusedThreads) fused_chunk_map_kernel(ChunkMap
   __shared__ __align__(16) float s_k[KQB][SP][TB + kPad];
 
   const FusedLane ln = fused_lane<SP>(g);
-  const int64_t M = g.M, S = g.S, L = g.steps;
+  const FusedSpan span = fused_span(g, ln.b);
+  const int64_t M = g.M, S = g.S, L = span.steps, row0 = span.row0;
   const int64_t m0 = (xcd_block() % g.groups) * CH;
   const int c = static_cast<int>(ln.m - m0);
   const int64_t ms = ln.m * S + ln.s;
@@ -1298,13 +1321,13 @@ __global__ void __launch_bounds__(kFusedThreads) fused_chunk_map_kernel(ChunkMap
   const A2 a2 = split_a2(a_s);
 
   const SensorIn &sn = prm.sn;
-  const float *kbase = prm.k + ln.b * L * S;
+  const float *kbase = prm.k + row0 * S;
   TileRegs<TB, CH> rv, rl;
   TileRegs<TB, SP> rk;
   auto load = [&](int64_t t0) {
     const int64_t rows = L - t0;
-    tile_load_sensor<TB, CH, BF16>(rv, sensor_at<BF16>(sn.v, ln.b * L + t0, m0, sn.ld_v), sn.ld_v, rows, cols_m);
-    tile_load_sensor<TB, CH, BF16>(rl, sensor_at<BF16>(sn.lv, ln.b * L + t0, m0, sn.ld_lv), sn.ld_lv, rows, cols_m);
+    tile_load_sensor<TB, CH, BF16>(rv, sensor_at<BF16>(sn.v, row0 + t0, m0, sn.ld_v), sn.ld_v, rows, cols_m);
+    tile_load_sensor<TB, CH, BF16>(rl, sensor_at<BF16>(sn.lv, row0 + t0, m0, sn.ld_lv), sn.ld_lv, rows, cols_m);
     tile_load<TB, SP>(rk, kbase + t0 * S, S, rows, S);
   };
   auto stage = [&](int buf) {
@@ -1459,7 +1482,8 @@ __global__ void __launch_bounds__(kFusedThreads) fused_adjoint_map_kernel(Adjoin
   __shared__ __align__(16) float s_k2[kK2 ? KQB : 1][kK2 ? SP : 1][TB + kPad];
 
   const FusedLane ln = fused_lane<SP>(g);
-  const int64_t M = g.M, S = g.S, L = g.steps;
+  const FusedSpan span = fused_span(g, ln.b);
+  const int64_t M = g.M, S = g.S, L = span.steps, row0 = span.row0;
   const int64_t m0 = (xcd_block() % g.groups) * CH;
   const int c = static_cast<int>(ln.m - m0);
   const int64_t ms = ln.m * S + ln.s;
@@ -1471,14 +1495,14 @@ __global__ void __launch_bounds__(kFusedThreads) fused_adjoint_map_kernel(Adjoin
   const A2 a2s = split_a2(a_s);
   const float a2 = a2s.hi;
 
-  const int64_t offM = ln.b * L * M + m0, offS = ln.b * L * S;
+  const int64_t offM = row0 * M + m0, offS = row0 * S;
   const SensorIn &sn = prm.sn;
   TileRegs<TB, CH> rv, rl, rdy, rdyv;
   TileRegs<TB, SP> rk, rq;
   auto load = [&](int64_t t0) {
     const int64_t rows = L - t0;
-    tile_load_sensor<TB, CH, BF16>(rv, sensor_at<BF16>(sn.v, ln.b * L + t0, m0, sn.ld_v), sn.ld_v, rows, cols_m);
-    tile_load_sensor<TB, CH, BF16>(rl, sensor_at<BF16>(sn.lv, ln.b * L + t0, m0, sn.ld_lv), sn.ld_lv, rows, cols_m);
+    tile_load_sensor<TB, CH, BF16>(rv, sensor_at<BF16>(sn.v, row0 + t0, m0, sn.ld_v), sn.ld_v, rows, cols_m);
+    tile_load_sensor<TB, CH, BF16>(rl, sensor_at<BF16>(sn.lv, row0 + t0, m0, sn.ld_lv), sn.ld_lv, rows, cols_m);
     tile_load<TB, CH>(rdy, prm.dy + offM + t0 * M, M, rows, cols_m);
     if constexpr (VAR) tile_load<TB, CH>(rdyv, prm.dyvar + offM + t0 * M, M, rows, cols_m);
     tile_load<TB, SP>(rk, prm.k + offS + t0 * S, S, rows, S);
@@ -1501,13 +1525,13 @@ __global__ void __launch_bounds__(kFusedThreads) fused_adjoint_map_kernel(Adjoin
   // The chunk's map so far (identity): the adjoint entering the chunk from the
   // right, x, becomes [[P, Q], [0, A]] x + (ul, ue) before the steps walked.
   float P = 1.0f, Q = 0.0f, A = 1.0f, ul = 0.0f, ue = 0.0f;
-  const int64_t n_ck = g.n_ck;
+  const int64_t n_ck = span.n_ck;
   // Checkpoints are read one block ahead, with the block's tiles (as in
   // fused_kla_bwd_kernel: a load just before the replay waits for all in flight).
   float ck_l = 1.0f, ck_e = 0.0f;
   auto load_ck = [&](int64_t blk) {
     if (ln.active) {
-      const int64_t ci = ((ln.b * n_ck + blk) * M + ln.m) * S + ln.s;
+      const int64_t ci = ((span.ck0 + blk) * M + ln.m) * S + ln.s;
       ck_l = prm.ck_lam[ci];
       ck_e = prm.ck_eta[ci];
     }
@@ -1649,6 +1673,18 @@ __global__ void __launch_bounds__(256) adjoint_ends_kernel(const float *__restri
     ge = fmaf(pqa.z, ge, rest.x);
     gl = gl_new;
   }
+}
+
+// dlam0, deta0 [batch, n] (NULL: not wanted) from every chunk's [batch, chunks, n]:
+// the first chunk's.
+__global__ void __launch_bounds__(256) first_chunks_kernel(const float *__restrict__ gl, const float *__restrict__ ge,
+                                                           float *__restrict__ dlam0, float *__restrict__ deta0,
+                                                           int64_t batch, int64_t chunks, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= batch * n) return;
+  const int64_t row = (i / n) * chunks * n + i % n;
+  if (dlam0) dlam0[i] = gl[row];
+  if (deta0) deta0[i] = ge[row];
 }
 
 }  // namespace kla

@@ -276,13 +276,25 @@ FusedGeom fused_geom(int64_t batch, int64_t steps, int64_t M, int64_t S) {
   const int64_t ch = kFusedThreads / sp_of(S);
   g.groups = (M + ch - 1) / ch;
   g.n_ck = (steps + kCkpt - 1) / kCkpt;
+  g.chunks = 1;
+  g.chunk_steps = steps;
   return g;
 }
 
-// Partials of the fused backward: part_k, part_q [B, L, G, S]; part_a, part_p [B, M, S]
-// (kHuge when that saturates).
-int64_t fused_workspace_floats(const FusedGeom &g) {
-  return sadd(smul(2, smul(smul(g.batch, g.steps), smul(g.groups, g.S))), smul(2, smul(g.batch, smul(g.M, g.S))));
+// fused_geom of `batch` sequences cut into chunks of chunk_steps steps (a
+// multiple of kCkpt, below steps): one grid row per chunk.
+FusedGeom split_geom(int64_t batch, int64_t steps, int64_t M, int64_t S, int64_t chunk_steps) {
+  FusedGeom g = fused_geom(batch, steps, M, S);
+  g.chunks = (steps + chunk_steps - 1) / chunk_steps;
+  g.chunk_steps = chunk_steps;
+  g.batch = batch * g.chunks;
+  return g;
+}
+
+// Partials of the fused backward over `seqs` sequences: part_k, part_q [B, L, G, S];
+// part_a, part_p [B * chunks, M, S] (kHuge when that saturates).
+int64_t fused_workspace_floats(const FusedGeom &g, int64_t seqs) {
+  return sadd(smul(2, smul(smul(seqs, g.steps), smul(g.groups, g.S))), smul(2, smul(g.batch, smul(g.M, g.S))));
 }
 
 int check_fused_shape(const char *fn, int64_t batch, int64_t steps, int64_t M, int64_t S) {
@@ -438,6 +450,84 @@ int record_kernel_event(const char *fn, int kernel, int which, hipStream_t strea
   return ev ? hip_status(fn, hipEventRecord(ev, stream)) : KLA_OK;
 }
 
+int fused_fwd_launch(const char *fn, const FusedFwdParams &prm, const FusedGeom &g, int decode_from_prior,
+                     hipStream_t stream) {
+  const int64_t grid = smul(g.batch, g.groups);
+  if (grid >= (1ll << 31)) return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
+  int rc = record_kernel_event(fn, KLA_KERNEL_FUSED_FWD, 0, stream);
+  if (rc != KLA_OK) return rc;
+  rc = with_sp(g.S, [&](auto sp) {
+    constexpr int SP = decltype(sp)::value;
+    auto run = [&](auto prior, auto bf16, auto var) {
+      hipLaunchKernelGGL(
+          (fused_kla_fwd_kernel<SP, decltype(prior)::value, decltype(bf16)::value, decltype(var)::value>),
+          dim3(static_cast<uint32_t>(grid)), dim3(kFusedThreads), 0, stream, prm, g);
+    };
+    with_flags(run, decode_from_prior != 0, prm.sn.bf16 != 0, prm.yvar != nullptr);
+    return hip_status(fn, hipGetLastError());
+  });
+  if (rc != KLA_OK) return rc;
+  return record_kernel_event(fn, KLA_KERNEL_FUSED_FWD, 1, stream);
+}
+
+int chunk_maps_launch(const char *fn, const ChunkMapParams &prm, const FusedGeom &g, hipStream_t stream) {
+  const int64_t grid = smul(g.batch, g.groups);
+  if (grid >= (1ll << 31)) return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
+  return with_sp(g.S, [&](auto sp) {
+    constexpr int SP = decltype(sp)::value;
+    if (prm.sn.bf16)
+      hipLaunchKernelGGL((fused_chunk_map_kernel<SP, true>), dim3(static_cast<uint32_t>(grid)), dim3(kFusedThreads),
+                         0, stream, prm, g);
+    else
+      hipLaunchKernelGGL((fused_chunk_map_kernel<SP, false>), dim3(static_cast<uint32_t>(grid)), dim3(kFusedThreads),
+                         0, stream, prm, g);
+    return hip_status(fn, hipGetLastError());
+  });
+}
+
+int adjoint_maps_launch(const char *fn, const AdjointMapParams &prm, const FusedGeom &g, int decode_from_prior,
+                        hipStream_t stream) {
+  const int64_t grid = smul(g.batch, g.groups);
+  if (grid >= (1ll << 31)) return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
+  return with_sp(g.S, [&](auto sp) {
+    constexpr int SP = decltype(sp)::value;
+    auto run = [&](auto prior, auto bf16, auto var) {
+      hipLaunchKernelGGL(
+          (fused_adjoint_map_kernel<SP, decltype(prior)::value, decltype(bf16)::value, decltype(var)::value>),
+          dim3(static_cast<uint32_t>(grid)), dim3(kFusedThreads), 0, stream, prm, g);
+    };
+    with_flags(run, decode_from_prior != 0, prm.sn.bf16 != 0, prm.dyvar != nullptr);
+    return hip_status(fn, hipGetLastError());
+  });
+}
+
+void chunk_starts_launch(const float *maps, const float *lam0, const float *eta0, float *lam_start, float *eta_start,
+                         float *lam_end, float *eta_end, int64_t batch, int64_t chunks, int64_t n, hipStream_t stream) {
+  hipLaunchKernelGGL(chunk_starts_kernel, dim3(static_cast<uint32_t>((batch * n + 255) / 256)), dim3(256), 0, stream,
+                     maps, lam0, eta0, lam_start, eta_start, lam_end, eta_end, batch, chunks, n);
+}
+
+void adjoint_ends_launch(const float *maps, const float *dlam_fin, const float *deta_fin, float *gl_end,
+                         float *ge_end, int64_t batch, int64_t chunks, int64_t n, hipStream_t stream) {
+  hipLaunchKernelGGL(adjoint_ends_kernel, dim3(static_cast<uint32_t>((batch * n + 255) / 256)), dim3(256), 0, stream,
+                     maps, dlam_fin, deta_fin, gl_end, ge_end, batch, chunks, n);
+}
+
+// Floats of scratch a split over `chunks` chunks takes beside the backward's
+// partials: the maps [B * chunks, M, S, 8] and two states a chunk.
+int64_t split_scratch_floats(int64_t batch, int64_t chunks, int64_t M, int64_t S) {
+  return smul(10, smul(smul(batch, chunks), smul(M, S)));
+}
+
+// The chunk length of a split call, checked.
+int check_split(const char *fn, int64_t batch, int64_t steps, int64_t M, int64_t S, int64_t chunk_steps) {
+  const int rc = check_fused_shape(fn, batch, steps, M, S);
+  if (rc != KLA_OK) return rc;
+  if (chunk_steps <= 0 || chunk_steps % kCkpt || chunk_steps >= steps)
+    return fail(KLA_ERR_INVALID_ARG, "%s: chunk_steps must be a positive multiple of %d below steps", fn, kCkpt);
+  return KLA_OK;
+}
+
 int fused_fwd(const char *fn, const SensorIn &sn, const float *k, const float *q, const float *a, const float *p,
               const float *lam0, const float *eta0, float *y, float *y_var, float *lam_fin, float *eta_fin,
               float *ck_lam, float *ck_eta, int decode_from_prior, int64_t batch, int64_t steps, int64_t M,
@@ -453,30 +543,14 @@ int fused_fwd(const char *fn, const SensorIn &sn, const float *k, const float *q
     return fail(KLA_ERR_INVALID_ARG, "%s: pass both checkpoint buffers or neither", fn);
   if (!all_aligned(4, {k, q, a, p, lam0, eta0, y, y_var, lam_fin, eta_fin, ck_lam, ck_eta}))
     return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
-  const FusedGeom g = fused_geom(batch, steps, M, S);
-  const int64_t grid = batch * g.groups;
-  if (grid >= (1ll << 31)) return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
   const FusedFwdParams prm{sn, k, q, a, p, lam0, eta0, y, y_var, lam_fin, eta_fin, ck_lam, ck_eta};
-  if ((rc = record_kernel_event(fn, KLA_KERNEL_FUSED_FWD, 0, stream)) != KLA_OK) return rc;
-  rc = with_sp(S, [&](auto sp) {
-    constexpr int SP = decltype(sp)::value;
-    auto run = [&](auto prior, auto bf16, auto var) {
-      hipLaunchKernelGGL(
-          (fused_kla_fwd_kernel<SP, decltype(prior)::value, decltype(bf16)::value, decltype(var)::value>),
-          dim3(static_cast<uint32_t>(grid)), dim3(kFusedThreads), 0, stream, prm, g);
-    };
-    with_flags(run, decode_from_prior != 0, sn.bf16 != 0, y_var != nullptr);
-    return hip_status(fn, hipGetLastError());
-  });
-  if (rc != KLA_OK) return rc;
-  return record_kernel_event(fn, KLA_KERNEL_FUSED_FWD, 1, stream);
+  return fused_fwd_launch(fn, prm, fused_geom(batch, steps, M, S), decode_from_prior, stream);
 }
-
 int fused_bwd(const char *fn, const float *dy, const float *dy_var, const float *dlam_fin, const float *deta_fin,
               const SensorIn &sn, const float *k, const float *q, const float *a, const float *p,
               const float *ck_lam, const float *ck_eta, void *dv, void *dlambda_v, float *dk, float *dq, float *da,
               float *dp, float *dlam0, float *deta0, int decode_from_prior, int64_t batch, int64_t steps, int64_t M,
-              int64_t S, void *workspace, size_t workspace_bytes, hipStream_t stream) {
+              int64_t S, int64_t chunk_steps, void *workspace, size_t workspace_bytes, hipStream_t stream) {
   int rc = check_fused_shape(fn, batch, steps, M, S);
   if (rc != KLA_OK) return rc;
   if (M == 0 || S == 0) return KLA_OK;
@@ -488,22 +562,22 @@ int fused_bwd(const char *fn, const float *dy, const float *dy_var, const float 
     return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
   if (misaligned_bytes(dv, sn.bf16 ? 2 : 4) || misaligned_bytes(dlambda_v, sn.bf16 ? 2 : 4))
     return fail(KLA_ERR_ALIGN, "%s: sensor gradient not aligned to its element size", fn);
-  const FusedGeom g = fused_geom(batch, steps, M, S);
+  const FusedGeom g = chunk_steps ? split_geom(batch, steps, M, S, chunk_steps) : fused_geom(batch, steps, M, S);
   if (workspace == nullptr) return fail(KLA_ERR_WORKSPACE, "%s: workspace is NULL", fn);
   if (misaligned_bytes(workspace, 256)) return fail(KLA_ERR_WORKSPACE, "%s: workspace not 256-byte aligned", fn);
-  const int64_t need_floats = fused_workspace_floats(g);
+  const int64_t need_floats = fused_workspace_floats(g, batch);
   if (need_floats >= kHuge / 4) return fail(KLA_ERR_INVALID_ARG, "%s: problem too large", fn);
   const size_t need = static_cast<size_t>(need_floats) * sizeof(float);
   if (workspace_bytes < need)
     return fail(KLA_ERR_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes, need);
-  const int64_t grid = batch * g.groups;
+  const int64_t grid = smul(g.batch, g.groups);
   if (grid >= (1ll << 31)) return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
 
   float *ws = static_cast<float *>(workspace);
   float *part_k = ws;
   float *part_q = part_k + batch * steps * g.groups * S;
   float *part_a = part_q + batch * steps * g.groups * S;
-  float *part_p = part_a + batch * M * S;
+  float *part_p = part_a + g.batch * M * S;
   if (batch > 0) {
     const FusedBwdParams prm{dy, dy_var, dlam_fin, deta_fin, sn, k, q, a, p, ck_lam, ck_eta,
                              dv, dlambda_v, dlam0, deta0, part_k, part_q, part_a, part_p};
@@ -534,8 +608,8 @@ int fused_bwd(const char *fn, const float *dy, const float *dy_var, const float 
     if ((rc = reduce(part_k, dk, batch * steps, g.groups, S)) != KLA_OK) return rc;
     if ((rc = reduce(part_q, dq, batch * steps, g.groups, S)) != KLA_OK) return rc;
   }
-  if ((rc = reduce(part_a, da, 1, batch, M * S)) != KLA_OK) return rc;
-  return reduce(part_p, dp, 1, batch, M * S);
+  if ((rc = reduce(part_a, da, 1, g.batch, M * S)) != KLA_OK) return rc;
+  return reduce(part_p, dp, 1, g.batch, M * S);
 }
 
 int check_tail(const char *fn, int dtype, const void *res, int64_t ld_res, const void *gate, int64_t ld_gate,
@@ -844,7 +918,7 @@ int64_t kla_fused_checkpoints(int64_t steps) { return steps < 0 ? 0 : (steps + k
 
 size_t kla_fused_workspace_bytes(int64_t batch, int64_t steps, int64_t M, int64_t S) {
   if (check_fused_shape("kla_fused_workspace_bytes", batch, steps, M, S) != KLA_OK) return 0;
-  const int64_t floats = fused_workspace_floats(fused_geom(batch, steps, M, S));
+  const int64_t floats = fused_workspace_floats(fused_geom(batch, steps, M, S), batch);
   if (floats >= kHuge / 4) {
     fail(KLA_ERR_INVALID_ARG, "kla_fused_workspace_bytes: problem too large");
     return 0;
@@ -886,7 +960,7 @@ int kla_fused_scan_bwd(const float *dy, const float *dy_var, const float *dlam_f
   const char *fn = "kla_fused_scan_bwd";
   if (!all_aligned(4, {v, lambda_v})) return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
   return fused_bwd(fn, dy, dy_var, dlam_fin, deta_fin, dense_sensors(v, lambda_v, M), k, q, a, p, ck_lam, ck_eta,
-                   dv, dlambda_v, dk, dq, da, dp, dlam0, deta0, decode_from_prior, batch, steps, M, S, workspace,
+                   dv, dlambda_v, dk, dq, da, dp, dlam0, deta0, decode_from_prior, batch, steps, M, S, 0, workspace,
                    workspace_bytes, stream);
 }
 
@@ -902,7 +976,7 @@ int kla_fused_scan_sensors_bwd(const float *dy, const float *dy_var, const float
   const int rc = sensors_from(fn, sensors, M, &sn);
   if (rc != KLA_OK) return rc;
   return fused_bwd(fn, dy, dy_var, dlam_fin, deta_fin, sn, k, q, a, p, ck_lam, ck_eta, dv, dobs, dk, dq, da, dp,
-                   dlam0, deta0, decode_from_prior, batch, steps, M, S, workspace, workspace_bytes, stream);
+                   dlam0, deta0, decode_from_prior, batch, steps, M, S, 0, workspace, workspace_bytes, stream);
 }
 
 int kla_fused_chunk_maps(const kla_sensors *sensors, const float *k, const float *a, const float *p, float *maps,
@@ -918,20 +992,7 @@ int kla_fused_chunk_maps(const kla_sensors *sensors, const float *k, const float
     return fail(KLA_ERR_INVALID_ARG, "%s: the sensors and k must not be NULL", fn);
   if (!all_aligned(4, {k, a, p})) return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
   if (!all_aligned(16, {maps})) return fail(KLA_ERR_ALIGN, "%s: maps not 16-byte aligned", fn);
-  const FusedGeom g = fused_geom(batch, steps, M, S);
-  const int64_t grid = smul(batch, g.groups);
-  if (grid >= (1ll << 31)) return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
-  const ChunkMapParams prm{sn, k, a, p, maps};
-  return with_sp(S, [&](auto sp) {
-    constexpr int SP = decltype(sp)::value;
-    if (sn.bf16)
-      hipLaunchKernelGGL((fused_chunk_map_kernel<SP, true>), dim3(static_cast<uint32_t>(grid)), dim3(kFusedThreads),
-                         0, stream, prm, g);
-    else
-      hipLaunchKernelGGL((fused_chunk_map_kernel<SP, false>), dim3(static_cast<uint32_t>(grid)), dim3(kFusedThreads),
-                         0, stream, prm, g);
-    return hip_status(fn, hipGetLastError());
-  });
+  return chunk_maps_launch(fn, ChunkMapParams{sn, k, a, p, maps}, fused_geom(batch, steps, M, S), stream);
 }
 
 int kla_chunk_starts(const float *maps, const float *lam0, const float *eta0, float *lam_start, float *eta_start,
@@ -954,6 +1015,100 @@ int kla_chunk_starts(const float *maps, const float *lam0, const float *eta0, fl
   return hip_status(fn, hipGetLastError());
 }
 
+size_t kla_fused_split_workspace_bytes(int64_t batch, int64_t steps, int64_t M, int64_t S, int64_t chunk_steps,
+                                       int backward) {
+  if (check_split("kla_fused_split_workspace_bytes", batch, steps, M, S, chunk_steps) != KLA_OK) return 0;
+  const FusedGeom g = split_geom(batch, steps, M, S, chunk_steps);
+  int64_t floats = split_scratch_floats(batch, g.chunks, M, S);
+  if (backward) floats = sadd(sadd(floats, smul(2, smul(g.batch, smul(M, S)))), sadd(fused_workspace_floats(g, batch), 4));
+  if (floats >= kHuge / 4) {
+    fail(KLA_ERR_INVALID_ARG, "kla_fused_split_workspace_bytes: problem too large");
+    return 0;
+  }
+  return std::max<size_t>(256, static_cast<size_t>(floats) * sizeof(float));
+}
+
+int kla_fused_split_fwd(const kla_sensors *sensors, const float *k, const float *q, const float *a, const float *p,
+                        const float *lam0, const float *eta0, float *y, float *y_var, float *lam_fin, float *eta_fin,
+                        float *ck_lam, float *ck_eta, int decode_from_prior, int64_t batch, int64_t steps, int64_t M,
+                        int64_t S, int64_t chunk_steps, void *workspace, size_t workspace_bytes, hipStream_t stream) {
+  const char *fn = "kla_fused_split_fwd";
+  int rc = check_split(fn, batch, steps, M, S, chunk_steps);
+  if (rc != KLA_OK) return rc;
+  SensorIn sn;
+  if ((rc = sensors_from(fn, sensors, M, &sn)) != KLA_OK) return rc;
+  if (batch == 0 || M == 0 || S == 0) return KLA_OK;
+  if (!sn.v || !sn.lv || !k || !q || !a || !p || !y || !lam_fin || !eta_fin)
+    return fail(KLA_ERR_INVALID_ARG, "%s: the sensors, k, q, a, p, y, lam_fin and eta_fin must not be NULL", fn);
+  if ((ck_lam == nullptr) != (ck_eta == nullptr))
+    return fail(KLA_ERR_INVALID_ARG, "%s: pass both checkpoint buffers or neither", fn);
+  if (!all_aligned(4, {k, q, a, p, lam0, eta0, y, y_var, lam_fin, eta_fin, ck_lam, ck_eta}))
+    return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
+  const FusedGeom g = split_geom(batch, steps, M, S, chunk_steps);
+  const int64_t floats = split_scratch_floats(batch, g.chunks, M, S);
+  if (floats >= kHuge / 4) return fail(KLA_ERR_INVALID_ARG, "%s: problem too large", fn);
+  if (!workspace || misaligned_bytes(workspace, 256) || workspace_bytes < static_cast<size_t>(floats) * sizeof(float))
+    return fail(KLA_ERR_WORKSPACE, "%s: a 256-byte aligned workspace of %lld bytes is needed", fn,
+                (long long)floats * 4);
+  const int64_t lanes = g.batch * M * S;
+  if (smul(batch, M * S) >= (1ll << 39)) return fail(KLA_ERR_INVALID_ARG, "%s: problem too large", fn);
+  float *maps = static_cast<float *>(workspace);
+  float *lam_st = maps + 8 * lanes, *eta_st = maps + 9 * lanes;
+  if ((rc = chunk_maps_launch(fn, ChunkMapParams{sn, k, a, p, maps}, g, stream)) != KLA_OK) return rc;
+  chunk_starts_launch(maps, lam0, eta0, lam_st, eta_st, lam_fin, eta_fin, batch, g.chunks, M * S, stream);
+  if ((rc = hip_status(fn, hipGetLastError())) != KLA_OK) return rc;
+  // Every chunk's final state lands in the maps, which nothing reads any more.
+  const FusedFwdParams prm{sn, k, q, a, p, lam_st, eta_st, y, y_var, maps, maps + lanes, ck_lam, ck_eta};
+  return fused_fwd_launch(fn, prm, g, decode_from_prior, stream);
+}
+
+int kla_fused_split_bwd(const float *dy, const float *dy_var, const float *dlam_fin, const float *deta_fin,
+                        const kla_sensors *sensors, const float *k, const float *q, const float *a, const float *p,
+                        const float *ck_lam, const float *ck_eta, void *dv, void *dobs, float *dk, float *dq,
+                        float *da, float *dp, float *dlam0, float *deta0, int decode_from_prior, int64_t batch,
+                        int64_t steps, int64_t M, int64_t S, int64_t chunk_steps, void *workspace,
+                        size_t workspace_bytes, hipStream_t stream) {
+  const char *fn = "kla_fused_split_bwd";
+  int rc = check_split(fn, batch, steps, M, S, chunk_steps);
+  if (rc != KLA_OK) return rc;
+  SensorIn sn;
+  if ((rc = sensors_from(fn, sensors, M, &sn)) != KLA_OK) return rc;
+  if (batch == 0 || M == 0 || S == 0)
+    return fail(KLA_ERR_INVALID_ARG, "%s: an empty problem has nothing to split", fn);
+  if (!dy || !sn.v || !sn.lv || !k || !q || !a || !p || !ck_lam || !ck_eta)
+    return fail(KLA_ERR_INVALID_ARG, "%s: dy, the sensors, k, q, a, p and the checkpoints must not be NULL", fn);
+  if (!all_aligned(4, {dy, dy_var, dlam_fin, deta_fin, k, q, a, p, ck_lam, ck_eta, dlam0, deta0}))
+    return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
+  const FusedGeom g = split_geom(batch, steps, M, S, chunk_steps);
+  const int64_t lanes = g.batch * M * S;
+  const int64_t parts = fused_workspace_floats(g, batch);
+  const int64_t floats = sadd(sadd(split_scratch_floats(batch, g.chunks, M, S), smul(2, lanes)), sadd(parts, 4));
+  if (floats >= kHuge / 4) return fail(KLA_ERR_INVALID_ARG, "%s: problem too large", fn);
+  if (!workspace || misaligned_bytes(workspace, 256) || workspace_bytes < static_cast<size_t>(floats) * sizeof(float))
+    return fail(KLA_ERR_WORKSPACE, "%s: a 256-byte aligned workspace of %lld bytes is needed", fn,
+                (long long)floats * 4);
+  if (smul(batch, M * S) >= (1ll << 39)) return fail(KLA_ERR_INVALID_ARG, "%s: problem too large", fn);
+  // The partials first (256-byte aligned), then the maps, rounded up to 16 bytes.
+  float *ws = static_cast<float *>(workspace);
+  float *maps = ws + (parts + 3) / 4 * 4;
+  float *gl_end = maps + 8 * lanes, *ge_end = gl_end + lanes, *gl0 = ge_end + lanes, *ge0 = gl0 + lanes;
+  const AdjointMapParams amp{dy, dy_var, sn, k, q, a, p, ck_lam, ck_eta, maps};
+  if ((rc = adjoint_maps_launch(fn, amp, g, decode_from_prior, stream)) != KLA_OK) return rc;
+  adjoint_ends_launch(maps, dlam_fin, deta_fin, gl_end, ge_end, batch, g.chunks, M * S, stream);
+  if ((rc = hip_status(fn, hipGetLastError())) != KLA_OK) return rc;
+  rc = fused_bwd(fn, dy, dy_var, gl_end, ge_end, sn, k, q, a, p, ck_lam, ck_eta, dv, dobs, dk, dq, da, dp, gl0, ge0,
+                 decode_from_prior, batch, steps, M, S, chunk_steps, ws, static_cast<size_t>(parts) * sizeof(float),
+                 stream);
+  if (rc != KLA_OK) return rc;
+  // The initial state's gradients are the first chunks'.
+  if (dlam0 || deta0) {
+    hipLaunchKernelGGL(first_chunks_kernel, dim3(static_cast<uint32_t>((batch * M * S + 255) / 256)), dim3(256), 0,
+                       stream, gl0, ge0, dlam0, deta0, batch, g.chunks, M * S);
+    return hip_status(fn, hipGetLastError());
+  }
+  return KLA_OK;
+}
+
 int kla_fused_adjoint_maps(const float *dy, const float *dy_var, const kla_sensors *sensors, const float *k,
                            const float *q, const float *a, const float *p, const float *ck_lam, const float *ck_eta,
                            float *maps, int decode_from_prior, int64_t batch, int64_t steps, int64_t M, int64_t S,
@@ -970,20 +1125,8 @@ int kla_fused_adjoint_maps(const float *dy, const float *dy_var, const kla_senso
   if (!all_aligned(4, {dy, dy_var, k, q, a, p, ck_lam, ck_eta}))
     return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
   if (!all_aligned(16, {maps})) return fail(KLA_ERR_ALIGN, "%s: maps not 16-byte aligned", fn);
-  const FusedGeom g = fused_geom(batch, steps, M, S);
-  const int64_t grid = smul(batch, g.groups);
-  if (grid >= (1ll << 31)) return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
   const AdjointMapParams prm{dy, dy_var, sn, k, q, a, p, ck_lam, ck_eta, maps};
-  return with_sp(S, [&](auto sp) {
-    constexpr int SP = decltype(sp)::value;
-    auto run = [&](auto prior, auto bf16, auto var) {
-      hipLaunchKernelGGL(
-          (fused_adjoint_map_kernel<SP, decltype(prior)::value, decltype(bf16)::value, decltype(var)::value>),
-          dim3(static_cast<uint32_t>(grid)), dim3(kFusedThreads), 0, stream, prm, g);
-    };
-    with_flags(run, decode_from_prior != 0, sn.bf16 != 0, dy_var != nullptr);
-    return hip_status(fn, hipGetLastError());
-  });
+  return adjoint_maps_launch(fn, prm, fused_geom(batch, steps, M, S), decode_from_prior, stream);
 }
 
 int kla_adjoint_ends(const float *maps, const float *dlam_fin, const float *deta_fin, float *gl_end, float *ge_end,

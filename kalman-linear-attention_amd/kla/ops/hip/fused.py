@@ -97,21 +97,56 @@ def train_chunks(B: int, L: int, M: int, S: int, cus: int) -> int:
     return nc
 
 
+def ragged_chunk(B: int, L: int, M: int, S: int, cus: int, nc: int, train: bool) -> int:
+    """Steps of a chunk where the equal split into ``nc`` chunks (time_chunks, or
+    train_chunks with ``train``) ended because 2 nc does not divide L (into whole
+    checkpoint blocks with ``train``), though the grid still leaves CUs idle: chunks
+    of this many steps, the last one shorter (0: keep the equal split). A multiple of
+    16 near MIN_CHUNK or above, with which the grid reaches what the equal planners
+    aim at. One sequence of 1021 steps (M 1024, S 16) runs 86 us whole and 38 us in
+    eight chunks on MI355X."""
+    if L % ((32 if train else 2) * nc) == 0:
+        return 0
+    sp, base = _grid(B, M, S)
+    if base == 0 or base >= (1 if train else _split_below(sp)) * cus:
+        return 0
+    most = -(-2 * cus // base) if train else SPLIT_TO * cus // base
+    want = min(most, (L + MIN_CHUNK // 2) // MIN_CHUNK)
+    if want <= nc:
+        return 0
+    steps = -(-L // (16 * want)) * 16
+    return steps if MIN_CHUNK <= steps < L else 0
+
+
+def _plan(B: int, L: int, M: int, S: int, dev: torch.device, train: bool) -> tuple[int, int]:
+    """(chunks, steps of a chunk) of the time split: (1, L) for none."""
+    cus = _cus(dev.index or 0)
+    nc = train_chunks(B, L, M, S, cus) if train else time_chunks(B, L, M, S, cus)
+    steps = ragged_chunk(B, L, M, S, cus, nc, train)
+    return (-(-L // steps), steps) if steps else (nc, L // nc)
+
+
 def _split_forward(sn, k, q, a, p, lam0, eta0, y, y_var, lam_fin, eta_fin, decode_from_prior, B, L, M, S, nc,
-                   dev, ck_lam=None, ck_eta=None):
-    """The time-split forward: kla_fused_chunk_maps on the [B * nc, L / nc] view,
-    kla_chunk_starts, then the fused forward on the view from those starts (with
-    the checkpoints when given: [B, n_ck, M, S] is the view's [B * nc, n_ck / nc,
-    M, S] when L / nc is a multiple of 16). Writes lam_fin, eta_fin [B, M, S], the
-    state after each sequence's last chunk (from the chunk maps, by
-    kla_chunk_starts). The maps and the chunk starts share one buffer; every
-    chunk's final state (unused) then lands in the maps' part, no longer read."""
+                   dev, ck_lam=None, ck_eta=None, steps=None):
+    """The time-split forward in ``nc`` chunks of ``steps`` steps (default L / nc),
+    with the checkpoints when given. Writes lam_fin, eta_fin [B, M, S], the state
+    after each sequence's last chunk. Chunks of whole checkpoint blocks are one call,
+    kla_fused_split_fwd; equal chunks of another length run kla_fused_chunk_maps on
+    the [B * nc, L / nc] view, kla_chunk_starts, then the fused forward on the view
+    from those starts, with the maps and the chunk starts in one buffer (every
+    chunk's final state, unused, then lands in the maps' part, no longer read)."""
     lib, pt = _lib.lib(), _lib.ptr
     stream = _lib.stream(dev)
-    Bp, Lc = B * nc, L // nc
+    Bp, Lc = B * nc, steps or L // nc
     lanes = Bp * M * S
-    buf = torch.empty(10 * lanes, dtype=_F32, device=dev)   # maps [Bp, M, S, 8], then two [Bp, M, S]
+    buf = torch.empty(10 * max(lanes, 7), dtype=_F32, device=dev)   # maps [Bp, M, S, 8], then two [Bp, M, S]
     maps = pt(buf)
+    if Lc % 16 == 0 and Lc < L:
+        _lib.check("kla_fused_split_fwd", lib.kla_fused_split_fwd(
+            ctypes.byref(sn), pt(k), pt(q), pt(a), pt(p), pt(lam0), pt(eta0), pt(y), pt(y_var), pt(lam_fin),
+            pt(eta_fin), pt(ck_lam), pt(ck_eta), int(decode_from_prior), B, L, M, S, Lc, maps, 4 * buf.numel(),
+            stream))
+        return
     lam_st, eta_st = maps + 32 * lanes, maps + 36 * lanes
     _lib.check("kla_fused_chunk_maps", lib.kla_fused_chunk_maps(
         ctypes.byref(sn), pt(k), pt(a), pt(p), maps, Bp, Lc, M, S, stream))
@@ -122,29 +157,18 @@ def _split_forward(sn, k, q, a, p, lam0, eta0, y, y_var, lam_fin, eta_fin, decod
         pt(ck_lam), pt(ck_eta), int(decode_from_prior), Bp, Lc, M, S, stream))
 
 
-def _split_backward(bwd, dy, dy_var, dlam_fin, deta_fin, sn, k, q, a, p, ck_lam, ck_eta, decode_from_prior,
-                    B, L, M, S, nc, dev):
-    """The time-split backward: kla_fused_adjoint_maps on the [B * nc, L / nc]
-    view, kla_adjoint_ends, then ``bwd(batch, steps, dlam_fin, deta_fin, dlam0,
-    deta0, workspace, nbytes)`` -- the backward entry point on the view, with every
-    chunk's adjoint entering from its end. Returns (dlam0, deta0) [B, M, S], the
-    first chunks' initial-state gradients."""
+def _split_backward(dy, dy_var, dlam_fin, deta_fin, sn, k, q, a, p, ck_lam, ck_eta, dv, dobs, dk, dq, da, dp, dlam0,
+                    deta0, decode_from_prior, B, L, M, S, steps, dev):
+    """The time-split backward in chunks of ``steps`` steps (whole checkpoint blocks),
+    one call: each chunk's adjoint map, the adjoint entering every chunk from its end,
+    then the backward of every chunk from there."""
     lib, pt = _lib.lib(), _lib.ptr
-    stream = _lib.stream(dev)
-    Bp, Lc = B * nc, L // nc
-    f32 = dict(dtype=_F32, device=dev)
-    maps = torch.empty(Bp, M, S, 8, **f32)
-    _lib.check("kla_fused_adjoint_maps", lib.kla_fused_adjoint_maps(
-        pt(dy), pt(dy_var), ctypes.byref(sn), pt(k), pt(q), pt(a), pt(p), pt(ck_lam), pt(ck_eta), pt(maps),
-        int(decode_from_prior), Bp, Lc, M, S, stream))
-    gl_end, ge_end = torch.empty(B, nc, M, S, **f32), torch.empty(B, nc, M, S, **f32)
-    _lib.check("kla_adjoint_ends", lib.kla_adjoint_ends(
-        pt(maps), pt(dlam_fin), pt(deta_fin), pt(gl_end), pt(ge_end), B, nc, M, S, stream))
-    dlam0, deta0 = torch.empty(B, nc, M, S, **f32), torch.empty(B, nc, M, S, **f32)
-    nbytes = int(lib.kla_fused_workspace_bytes(Bp, Lc, M, S))
-    ws, _ = _lib.scratch(nbytes, dev)
-    bwd(Bp, Lc, gl_end, ge_end, dlam0, deta0, ws, nbytes)
-    return dlam0[:, 0].contiguous(), deta0[:, 0].contiguous()
+    nbytes = int(lib.kla_fused_split_workspace_bytes(B, L, M, S, steps, 1))
+    ws, stream = _lib.scratch(nbytes, dev)
+    _lib.check("kla_fused_split_bwd", lib.kla_fused_split_bwd(
+        pt(dy), pt(dy_var), pt(dlam_fin), pt(deta_fin), ctypes.byref(sn), pt(k), pt(q), pt(a), pt(p), pt(ck_lam),
+        pt(ck_eta), pt(dv), pt(dobs), pt(dk), pt(dq), pt(da), pt(dp), pt(dlam0), pt(deta0), int(decode_from_prior),
+        B, L, M, S, steps, pt(ws), ws.numel(), stream))
 
 
 def _dense_sensors(v: torch.Tensor, lambda_v: torch.Tensor) -> "_lib.Sensors":
@@ -216,12 +240,11 @@ def _fwd_one(v, lambda_v, k, q, a, p, lam0, eta0, decode_from_prior, save, dev, 
     if B * M * S == 0:
         # No lanes: the read-outs sum over no state lanes (zero where B, L, M leave entries).
         return y.zero_(), y_var.zero_(), lam_fin, eta_fin
-    cus = _cus(dev.index or 0)
-    nc = train_chunks(B, L, M, S, cus) if save else time_chunks(B, L, M, S, cus)
+    nc, steps = _plan(B, L, M, S, dev, save)
     if nc > 1:
         _split_forward(_dense_sensors(v, lambda_v), k, q, a, p, lam0, eta0, y, y_var, lam_fin, eta_fin,
                        decode_from_prior, B, L, M, S, nc, dev,
-                       ck_lam=ck_lam if save else None, ck_eta=ck_eta if save else None)
+                       ck_lam=ck_lam if save else None, ck_eta=ck_eta if save else None, steps=steps)
         return y, y_var, lam_fin, eta_fin
     stream = _lib.stream(dev)
     pt = _lib.ptr
@@ -285,23 +308,18 @@ def _bwd_one(dy, dy_var, dlam_fin, deta_fin, v, lambda_v, k, q, a, p, ck_lam, ck
         for t in (dv, dlv, dk, dq, da, dp):
             t.zero_()
         return dv, dlv, dk, dq, da, dp, dlam0, deta0
-    pt = _lib.ptr
-
-    def bwd(batch, steps, lam_fin_grad, eta_fin_grad, lam0_grad, eta0_grad, ws, nbytes):
-        stream = _lib.stream(dev)
-        _lib.check("kla_fused_scan_bwd", _lib.lib().kla_fused_scan_bwd(
-            pt(dy), pt(dy_var), pt(lam_fin_grad), pt(eta_fin_grad), pt(v), pt(lambda_v), pt(k), pt(q), pt(a),
-            pt(p), pt(ck_lam), pt(ck_eta), pt(dv), pt(dlv), pt(dk), pt(dq), pt(da), pt(dp), pt(lam0_grad),
-            pt(eta0_grad), int(decode_from_prior), batch, steps, M, S, pt(ws), nbytes, stream))
-
-    nc = train_chunks(B, L, M, S, _cus(dev.index or 0))
+    nc, steps = _plan(B, L, M, S, dev, True)
     if nc > 1:
-        dlam0, deta0 = _split_backward(bwd, dy, dy_var, dlam_fin, deta_fin, _dense_sensors(v, lambda_v), k, q, a,
-                                       p, ck_lam, ck_eta, decode_from_prior, B, L, M, S, nc, dev)
+        _split_backward(dy, dy_var, dlam_fin, deta_fin, _dense_sensors(v, lambda_v), k, q, a, p, ck_lam, ck_eta, dv,
+                        dlv, dk, dq, da, dp, dlam0, deta0, decode_from_prior, B, L, M, S, steps, dev)
         return dv, dlv, dk, dq, da, dp, dlam0, deta0
+    pt = _lib.ptr
     nbytes = int(_lib.lib().kla_fused_workspace_bytes(B, L, M, S))
-    ws, _ = _lib.scratch(nbytes, dev)
-    bwd(B, L, dlam_fin, deta_fin, dlam0, deta0, ws, ws.numel())
+    ws, stream = _lib.scratch(nbytes, dev)
+    _lib.check("kla_fused_scan_bwd", _lib.lib().kla_fused_scan_bwd(
+        pt(dy), pt(dy_var), pt(dlam_fin), pt(deta_fin), pt(v), pt(lambda_v), pt(k), pt(q), pt(a), pt(p), pt(ck_lam),
+        pt(ck_eta), pt(dv), pt(dlv), pt(dk), pt(dq), pt(da), pt(dp), pt(dlam0), pt(deta0), int(decode_from_prior),
+        B, L, M, S, pt(ws), ws.numel(), stream))
     return dv, dlv, dk, dq, da, dp, dlam0, deta0
 
 
@@ -455,12 +473,11 @@ def _sensors_fwd_op(v: torch.Tensor, obs: torch.Tensor, k: torch.Tensor, q: torc
         # No lanes: the read-outs sum over no state lanes (zero where B, L, M leave entries).
         return y.zero_(), y_var.zero_(), lam_fin, eta_fin, ck_lam, ck_eta
     sn = _sensor_desc(v, obs, lds, log_var, obs_var_min, obs_var_max)
-    cus = _cus(dev.index or 0)
-    nc = train_chunks(B, L, M, S, cus) if save else time_chunks(B, L, M, S, cus)
+    nc, steps = _plan(B, L, M, S, dev, save)
     if nc > 1:
         _split_forward(sn, k, q, a, p, lam0, eta0, y, y_var if with_var else None, lam_fin, eta_fin,
                        decode_from_prior, B, L, M, S, nc, dev,
-                       ck_lam=ck_lam if save else None, ck_eta=ck_eta if save else None)
+                       ck_lam=ck_lam if save else None, ck_eta=ck_eta if save else None, steps=steps)
         return y, y_var, lam_fin, eta_fin, ck_lam, ck_eta
     pt = _lib.ptr
     _lib.check("kla_fused_scan_sensors_fwd", _lib.lib().kla_fused_scan_sensors_fwd(
@@ -508,23 +525,18 @@ def _sensors_bwd_op(dy: torch.Tensor, dy_var: Optional[torch.Tensor], dlam_fin: 
             t.zero_()
         return dv, dobs, dk, dq, da, dp, dlam0, deta0
     sn = _sensor_desc(v, obs, lds, log_var, obs_var_min, obs_var_max)
-    pt = _lib.ptr
-
-    def bwd(batch, steps, lam_fin_grad, eta_fin_grad, lam0_grad, eta0_grad, ws, nbytes):
-        stream = _lib.stream(dev)
-        _lib.check("kla_fused_scan_sensors_bwd", _lib.lib().kla_fused_scan_sensors_bwd(
-            pt(dy), pt(dy_var), pt(lam_fin_grad), pt(eta_fin_grad), ctypes.byref(sn), pt(k), pt(q), pt(a), pt(p),
-            pt(ck_lam), pt(ck_eta), pt(dv), pt(dobs), pt(dk), pt(dq), pt(da), pt(dp), pt(lam0_grad),
-            pt(eta0_grad), int(decode_from_prior), batch, steps, M, S, pt(ws), nbytes, stream))
-
-    nc = train_chunks(B, L, M, S, _cus(dev.index or 0))
+    nc, steps = _plan(B, L, M, S, dev, True)
     if nc > 1:
-        dlam0, deta0 = _split_backward(bwd, dy, dy_var, dlam_fin, deta_fin, sn, k, q, a, p, ck_lam, ck_eta,
-                                       decode_from_prior, B, L, M, S, nc, dev)
+        _split_backward(dy, dy_var, dlam_fin, deta_fin, sn, k, q, a, p, ck_lam, ck_eta, dv, dobs, dk, dq, da, dp,
+                        dlam0, deta0, decode_from_prior, B, L, M, S, steps, dev)
         return dv, dobs, dk, dq, da, dp, dlam0, deta0
+    pt = _lib.ptr
     nbytes = int(_lib.lib().kla_fused_workspace_bytes(B, L, M, S))
-    ws, _ = _lib.scratch(nbytes, dev)
-    bwd(B, L, dlam_fin, deta_fin, dlam0, deta0, ws, ws.numel())
+    ws, stream = _lib.scratch(nbytes, dev)
+    _lib.check("kla_fused_scan_sensors_bwd", _lib.lib().kla_fused_scan_sensors_bwd(
+        pt(dy), pt(dy_var), pt(dlam_fin), pt(deta_fin), ctypes.byref(sn), pt(k), pt(q), pt(a), pt(p), pt(ck_lam),
+        pt(ck_eta), pt(dv), pt(dobs), pt(dk), pt(dq), pt(da), pt(dp), pt(dlam0), pt(deta0), int(decode_from_prior),
+        B, L, M, S, pt(ws), ws.numel(), stream))
     return dv, dobs, dk, dq, da, dp, dlam0, deta0
 
 
