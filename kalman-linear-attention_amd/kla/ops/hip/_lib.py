@@ -202,29 +202,73 @@ def stream(device: torch.device) -> int:
 
 def hip_op(name: str):
     """Decorator: ``torch.library.custom_op(name, mutates_args=())`` that keeps the
-    undecorated function as ``op.direct``."""
+    undecorated function as ``op.direct`` and what its ``register_autograd`` was given
+    as ``op.autograd`` (setup_context, backward)."""
     def wrap(fn):
         op = torch.library.custom_op(name, mutates_args=())(fn)
-        op.direct = fn
+        register = op.register_autograd
+
+        def register_autograd(backward, /, *, setup_context):
+            op.autograd = (setup_context, backward)
+            register(backward, setup_context=setup_context)
+
+        op.direct, op.autograd, op.register_autograd = fn, None, register_autograd
         return op
     return wrap
+
+
+class _Recorded(torch.autograd.Function):
+    """``op(*args)`` with its gradient, recorded as torch.library records it (the same
+    function, setup_context and backward) without the dispatcher's layers around
+    each: a small Moebius scan and its gradient 81 -> 66 us, the host time of a
+    training layer's forward (2 x 500, width 384, fp32) 540 -> 390 us, interleaved
+    runs on one MI355X host."""
+
+    @staticmethod
+    def forward(ctx, *args):
+        *args, op = args
+        out = op.direct(*args)
+        op.autograd[0](ctx, tuple(args), out)
+        ctx.op = op
+        return out
+
+    @staticmethod
+    def backward(ctx, *grads):
+        return (*ctx.op.autograd[1](ctx, *grads), None)
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
+def _eager() -> bool:
+    """Whether nothing but autograd watches the call: no compile, export or jit trace,
+    no functorch transform, no forward-mode level, no dispatch or function mode."""
+    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack())
+
+
 def call(op, *args):
     """``op(*args)``, run without the dispatcher where it adds nothing: outside
     torch.compile / export tracing, every tensor argument a plain tensor or
-    parameter (no fake or other subclass), and no autograd to record (grad mode
-    off, or no tensor argument requires grad). The same function runs either way."""
+    parameter (no fake or other subclass), and either no autograd to record (grad
+    mode off, or no tensor argument requires grad) or autograd alone (_eager), which
+    then records the op's own backward (_Recorded). The same functions run either way."""
     if torch.compiler.is_compiling():
         return op(*args)
     grad = torch.is_grad_enabled()
+    record = False
     for a in args:
-        if isinstance(a, torch.Tensor) and (type(a) not in _PLAIN or (grad and a.requires_grad)):
-            return op(*args)
-    return op.direct(*args)
+        if isinstance(a, torch.Tensor):
+            if type(a) not in _PLAIN:
+                return op(*args)
+            record = record or (grad and a.requires_grad)
+    if not record:
+        return op.direct(*args)
+    if op.autograd is None or not _eager():
+        return op(*args)
+    return _Recorded.apply(*args, op)
 
 
 # ----------------------------------------------------------------- workspace
