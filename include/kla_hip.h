@@ -620,21 +620,33 @@ int kla_rows_linear_conv_fwd(const float *x, int64_t ldx, const float *w, int64_
                              float *window_out, int64_t conv_n, int conv_k, int activation, hipStream_t stream);
 
 /*
- * y = x W^T + bias in fp32 over many rows: x [rows, k] (row stride ldx), W [n, k]
- * (ldw), bias [n] or NULL, y [rows, n] (ldy). The product runs on the fp16 matrix
- * cores over operands split into two fp16 planes (scaled per row), summed in
- * fp32: no larger an error than an fp32 product's, at about 2.5 times its rate.
- * Rows holding an infinity or a NaN give what fp32 arithmetic gives. No
- * gradient; deterministic (fixed-order sums). workspace: 256-byte aligned, at
- * least kla_linear_f32_workspace_bytes, contents not kept.
+ * A linear layer over many rows in fp32, with what surrounds it in a block:
+ *   xn  = norm_w ? (x * rsqrt(mean(x^2) + eps)) * norm_w : x      (per row of k)
+ *   acc = xn W^T + bias                 W [n_w, k] rows ldw apart, bias [n_w] or NULL
+ *   y   = acc | res + acc | silu(acc[:, j]) * acc[:, glu_off + j]  by epilogue
+ *         (KLA_ROWS_PLAIN, _RESIDUAL, _SWIGLU; W holds n rows, n + glu_off with SwiGLU)
+ * x [rows, k] and res, y [rows, n] with row strides ld*. The product
+ * runs on the fp16 matrix cores over operands split into two fp16 planes (scaled
+ * per row), summed in fp32: no larger an error than an fp32 product's, at about
+ * 2.5 times its rate. Rows holding an infinity or a NaN give what fp32 arithmetic
+ * gives. No gradient; deterministic (fixed-order sums). workspace: 256-byte
+ * aligned, at least kla_linear_f32_workspace_bytes, contents not kept.
  * Replaces, in inference over a sequence, the nn.Linear calls of KLALayer
- * (reference src/kla/layers/kla_layer.py:61, :88, :127), MLP (src/kla/layers/
- * common.py:99-123) and the LM head (src/kla/models/sequence_model.py:169).
+ * (reference src/kla/layers/kla_layer.py:61, :88, :127), MLP and RMSNorm
+ * (src/kla/layers/common.py:45-55, :99-123), the block's residual adds
+ * (src/kla/models/sequence_model.py:71-87) and the LM head (:169).
  */
-size_t kla_linear_f32_workspace_bytes(int64_t rows, int64_t n, int64_t k);
-int kla_linear_f32_fwd(const float *x, int64_t ldx, const float *w, int64_t ldw, const float *bias, float *y,
-                       int64_t ldy, int64_t rows, int64_t n, int64_t k, void *workspace, size_t workspace_bytes,
-                       hipStream_t stream);
+typedef struct kla_linear_f32_args {
+  int epilogue;
+  float eps;
+  const float *x, *w, *bias, *norm_w, *res;
+  float *y;
+  int64_t ldx, ldw, ldres, ldy;
+  int64_t rows, n, k, glu_off;
+} kla_linear_f32_args;
+
+size_t kla_linear_f32_workspace_bytes(int64_t rows, int64_t n, int64_t k, int epilogue);
+int kla_linear_f32_fwd(const kla_linear_f32_args *args, void *workspace, size_t workspace_bytes, hipStream_t stream);
 
 #ifdef __cplusplus
 }

@@ -1664,25 +1664,86 @@ int rows_linear_launch(const char *fn, int epi, RowsLinearParams &p, hipStream_t
   return hip_status(fn, hipGetLastError());
 }
 
-// The split fp32 product (split_gemm.hpp). Workspace: the planes of x and of W,
-// then their row exponents.
-int64_t linear_f32_bytes(int64_t rows, int64_t n, int64_t k) {
-  const int64_t blocks = sadd(sadd(rows, kSplitRows - 1) / kSplitRows, sadd(n, kSplitRows - 1) / kSplitRows);
+// The split fp32 product (split_gemm.hpp). Workspace: the planes of x and of W (two
+// sets of 32-row blocks with SwiGLU), then their row exponents.
+int64_t linear_f32_wblocks(int64_t n, bool swiglu) {
+  const int64_t b = sadd(n, kSplitRows - 1) / kSplitRows;
+  return swiglu ? smul(2, b) : b;
+}
+
+int64_t linear_f32_bytes(int64_t rows, int64_t n, int64_t k, bool swiglu) {
+  const int64_t blocks = sadd(sadd(rows, kSplitRows - 1) / kSplitRows, linear_f32_wblocks(n, swiglu));
   const int64_t planes = smul(smul(blocks, sadd(k, kSplitK - 1) / kSplitK), kSplitChunk * 2);
   return sadd(planes, smul(blocks, kSplitRows * 4));
 }
 
-int linear_f32_launch(const char *fn, const float *x, int64_t ldx, const float *w, int64_t ldw, const float *bias,
-                      float *y, int64_t ldy, int64_t rows, int64_t n, int64_t k, void *workspace,
-                      hipStream_t stream) {
+template <bool NORM>
+void split_rows_launch(const SplitParams &sp, hipStream_t stream) {
+  const dim3 grid(static_cast<uint32_t>(sp.op[0].blocks + sp.op[1].blocks)), block(kSplitThreads);
+  const int64_t per_wave = (sp.chunks + kSplitThreads / kWave - 1) / (kSplitThreads / kWave);
+  if (per_wave <= 2)
+    hipLaunchKernelGGL((split_rows_kernel<2, NORM>), grid, block, 0, stream, sp);
+  else if (per_wave <= 4)
+    hipLaunchKernelGGL((split_rows_kernel<4, NORM>), grid, block, 0, stream, sp);
+  else if (per_wave <= 8)
+    hipLaunchKernelGGL((split_rows_kernel<8, NORM>), grid, block, 0, stream, sp);
+  else
+    hipLaunchKernelGGL((split_rows_kernel<0, NORM>), grid, block, 0, stream, sp);
+}
+
+template <int EPI>
+void split_gemm_launch(SplitGemmParams g, hipStream_t stream) {
+  // The widest tile that still gives every CU two workgroups (512 on 256 CUs):
+  // a workgroup alone on a CU waits out its barriers, and 128 x 128 moves half
+  // the operand bytes per product of 64 x 64. Measured (us, k = 1024): 4096 x
+  // 2048 outputs 53 (128 x 128) / 58 (128 x 64) / 62 (64 x 64), 2048 x 2048
+  // 33.2 / 31.5 / 33.5, 2048 x 512 25.0 / 17.4 / 12.1. (SwiGLU needs two blocks
+  // of W a wave, which 64 x 64 does not have.)
+  constexpr int64_t kFill = 2 * 256;
+  auto tiles = [&](int bn, int bt) { return ((g.wblocks + bn - 1) / bn) * ((g.xblocks + bt - 1) / bt); };
+  auto go = [&](auto kernel, int bn, int bt) {
+    g.tiles_n = (g.wblocks + bn - 1) / bn;
+    g.tiles_t = (g.xblocks + bt - 1) / bt;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(g.tiles_n * g.tiles_t)), dim3(4 * kWave), 0, stream, g);
+  };
+  if (tiles(4, 4) >= kFill) return go(split_gemm_kernel<EPI, 2, 2, 2, 2, 2, 2>, 4, 4);
+  if constexpr (EPI != kGemmSwiglu) {
+    if (tiles(4, 2) < kFill) return go(split_gemm_kernel<EPI, 2, 2, 1, 1, 3, 3>, 2, 2);
+  }
+  go(split_gemm_kernel<EPI, 2, 2, 2, 1, 2, 3>, 4, 2);
+}
+
+int linear_f32(const char *fn, const kla_linear_f32_args &a, void *workspace, size_t workspace_bytes,
+               hipStream_t stream) {
+  if (a.rows < 0 || a.n < 0 || a.k <= 0 || a.glu_off < 0)
+    return fail(KLA_ERR_INVALID_ARG, "%s: negative size or no columns", fn);
+  if (a.epilogue != KLA_ROWS_PLAIN && a.epilogue != KLA_ROWS_RESIDUAL && a.epilogue != KLA_ROWS_SWIGLU)
+    return fail(KLA_ERR_INVALID_ARG, "%s: unknown epilogue %d", fn, a.epilogue);
+  if (a.rows == 0 || a.n == 0) return KLA_OK;
+  const bool swiglu = a.epilogue == KLA_ROWS_SWIGLU, residual = a.epilogue == KLA_ROWS_RESIDUAL;
+  if (!a.x || !a.w || !a.y) return fail(KLA_ERR_INVALID_ARG, "%s: x, w and y must not be NULL", fn);
+  if (residual && !a.res) return fail(KLA_ERR_INVALID_ARG, "%s: the residual epilogue needs res", fn);
+  if (swiglu && a.glu_off < a.n)
+    return fail(KLA_ERR_INVALID_ARG, "%s: glu_off %lld below n %lld (the halves overlap)", fn, (long long)a.glu_off,
+                (long long)a.n);
+  if (a.ldx < a.k || a.ldw < a.k || a.ldy < a.n || (residual && a.ldres < a.n))
+    return fail(KLA_ERR_INVALID_ARG, "%s: a row stride is below its row length", fn);
+  if (!all_aligned(4, {a.x, a.w, a.bias, a.norm_w, a.res, a.y}))
+    return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
+  const int64_t need = linear_f32_bytes(a.rows, a.n, a.k, swiglu);
+  if (!workspace || need >= kHuge || static_cast<int64_t>(workspace_bytes) < need)
+    return fail(KLA_ERR_WORKSPACE, "%s: a workspace of %lld bytes is needed", fn, (long long)need);
+  if (misaligned_bytes(workspace, 256)) return fail(KLA_ERR_WORKSPACE, "%s: workspace not 256-byte aligned", fn);
+
   SplitGemmParams g{};
-  g.x = x, g.w = w, g.bias = bias, g.y = y;
-  g.ldx = ldx, g.ldw = ldw, g.ldy = ldy;
-  g.rows = rows, g.n = n, g.k = k;
-  g.chunks = (k + kSplitK - 1) / kSplitK;
-  g.xblocks = (rows + kSplitRows - 1) / kSplitRows;
-  g.wblocks = (n + kSplitRows - 1) / kSplitRows;
-  if (g.chunks >= (1ll << 30) || g.xblocks + g.wblocks >= (1ll << 31) || smul(2 * g.xblocks, 2 * g.wblocks) >= (1ll << 31))
+  g.w = a.w, g.bias = a.bias, g.res = a.res, g.y = a.y;
+  g.ldw = a.ldw, g.ldres = a.ldres, g.ldy = a.ldy;
+  g.rows = a.rows, g.n = a.n, g.k = a.k, g.glu_off = a.glu_off;
+  g.chunks = (a.k + kSplitK - 1) / kSplitK;
+  g.xblocks = (a.rows + kSplitRows - 1) / kSplitRows;
+  g.wblocks = linear_f32_wblocks(a.n, swiglu);
+  if (g.chunks >= (1ll << 30) || g.xblocks + g.wblocks >= (1ll << 31) ||
+      smul(2 * g.xblocks, 2 * g.wblocks) >= (1ll << 31))
     return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
   _Float16 *xs = static_cast<_Float16 *>(workspace);
   _Float16 *ws = xs + g.xblocks * g.chunks * kSplitChunk;
@@ -1691,39 +1752,22 @@ int linear_f32_launch(const char *fn, const float *x, int64_t ldx, const float *
   g.xs = xs, g.ws = ws, g.xe = xe, g.we = we;
 
   SplitParams sp{};
-  sp.op[0] = SplitOperand{x, ldx, rows, xs, xe, g.xblocks};
-  sp.op[1] = SplitOperand{w, ldw, n, ws, we, g.wblocks};
-  sp.k = k;
+  sp.op[0] = SplitOperand{a.x, a.ldx, a.rows, xs, xe, g.xblocks};
+  sp.op[1] = SplitOperand{a.w, a.ldw, a.n, ws, we, g.wblocks};
+  sp.k = a.k;
   sp.chunks = g.chunks;
-  const dim3 sgrid(static_cast<uint32_t>(g.xblocks + g.wblocks)), sblock(kSplitThreads);
-  const int64_t per_wave = (g.chunks + kSplitThreads / kWave - 1) / (kSplitThreads / kWave);
-  if (per_wave <= 2)
-    hipLaunchKernelGGL(split_rows_kernel<2>, sgrid, sblock, 0, stream, sp);
-  else if (per_wave <= 4)
-    hipLaunchKernelGGL(split_rows_kernel<4>, sgrid, sblock, 0, stream, sp);
-  else if (per_wave <= 8)
-    hipLaunchKernelGGL(split_rows_kernel<8>, sgrid, sblock, 0, stream, sp);
+  if (swiglu) sp.glu_off = a.glu_off, sp.glu_rows = a.n;
+  sp.norm_w = a.norm_w, sp.eps = a.eps;
+  if (a.norm_w)
+    split_rows_launch<true>(sp, stream);
   else
-    hipLaunchKernelGGL(split_rows_kernel<0>, sgrid, sblock, 0, stream, sp);
-
-  // The widest tile that still gives every CU two workgroups (512 on 256 CUs):
-  // a workgroup alone on a CU waits out its barriers, and 128 x 128 moves half
-  // the operand bytes per product of 64 x 64. Measured (us, k = 1024): 4096 x
-  // 2048 outputs 53 (128 x 128) / 58 (128 x 64) / 62 (64 x 64), 2048 x 2048
-  // 33.2 / 31.5 / 33.5, 2048 x 512 25.0 / 17.4 / 12.1.
-  constexpr int64_t kFill = 2 * 256;
-  auto tiles = [&](int tn, int tt) { return ((n + tn - 1) / tn) * ((rows + tt - 1) / tt); };
-  auto go = [&](auto kernel, int tn, int tt) {
-    g.tiles_n = (n + tn - 1) / tn;
-    g.tiles_t = (rows + tt - 1) / tt;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(g.tiles_n * g.tiles_t)), dim3(4 * kWave), 0, stream, g);
-  };
-  if (tiles(128, 128) >= kFill)
-    go(split_gemm_kernel<2, 2, 2, 2, 2, 2>, 128, 128);
-  else if (tiles(128, 64) >= kFill)
-    go(split_gemm_kernel<2, 2, 2, 1, 2, 3>, 128, 64);
+    split_rows_launch<false>(sp, stream);
+  if (swiglu)
+    split_gemm_launch<kGemmSwiglu>(g, stream);
+  else if (residual)
+    split_gemm_launch<kGemmResidual>(g, stream);
   else
-    go(split_gemm_kernel<2, 2, 1, 1, 3, 3>, 64, 64);
+    split_gemm_launch<kGemmPlain>(g, stream);
   return hip_status(fn, hipGetLastError());
 }
 
@@ -1820,27 +1864,16 @@ int kla_rows_linear_conv_fwd(const float *x, int64_t ldx, const float *w, int64_
   return rows_linear_launch(fn, kEpiConv, p, stream);
 }
 
-size_t kla_linear_f32_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
+size_t kla_linear_f32_workspace_bytes(int64_t rows, int64_t n, int64_t k, int epilogue) {
   if (rows <= 0 || n <= 0 || k <= 0) return 0;
-  const int64_t bytes = linear_f32_bytes(rows, n, k);
+  const int64_t bytes = linear_f32_bytes(rows, n, k, epilogue == KLA_ROWS_SWIGLU);
   return bytes >= kHuge ? 0 : static_cast<size_t>(bytes);
 }
 
-int kla_linear_f32_fwd(const float *x, int64_t ldx, const float *w, int64_t ldw, const float *bias, float *y,
-                       int64_t ldy, int64_t rows, int64_t n, int64_t k, void *workspace, size_t workspace_bytes,
-                       hipStream_t stream) {
+int kla_linear_f32_fwd(const kla_linear_f32_args *args, void *workspace, size_t workspace_bytes, hipStream_t stream) {
   const char *fn = "kla_linear_f32_fwd";
-  if (rows < 0 || n < 0 || k <= 0) return fail(KLA_ERR_INVALID_ARG, "%s: negative size or no columns", fn);
-  if (rows == 0 || n == 0) return KLA_OK;
-  if (!x || !w || !y) return fail(KLA_ERR_INVALID_ARG, "%s: x, w and y must not be NULL", fn);
-  if (ldx < k || ldw < k || ldy < n) return fail(KLA_ERR_INVALID_ARG, "%s: a row stride is below its row length", fn);
-  if (misaligned(x) || misaligned(w) || misaligned(bias) || misaligned(y))
-    return fail(KLA_ERR_ALIGN, "%s: fp32 operand not 4-byte aligned", fn);
-  const int64_t need = linear_f32_bytes(rows, n, k);
-  if (!workspace || need >= kHuge || static_cast<int64_t>(workspace_bytes) < need)
-    return fail(KLA_ERR_WORKSPACE, "%s: a workspace of %lld bytes is needed", fn, (long long)need);
-  if (misaligned_bytes(workspace, 256)) return fail(KLA_ERR_WORKSPACE, "%s: workspace not 256-byte aligned", fn);
-  return linear_f32_launch(fn, x, ldx, w, ldw, bias, y, ldy, rows, n, k, workspace, stream);
+  if (!args) return fail(KLA_ERR_INVALID_ARG, "%s: args must not be NULL", fn);
+  return linear_f32(fn, *args, workspace, workspace_bytes, stream);
 }
 
 int kla_gather_rows(int dtype, const void *table, int64_t ld_table, int64_t vocab, const int64_t *ids, void *out,

@@ -16,8 +16,18 @@
 // magnitude into [2^14, 2^15); the scales go back in with one ldexp per output.
 // Entries more than 2^17 below their row's largest lose low bits of lo to
 // fp16's smallest spacing, at most 2^-39 of the row's largest value each. A row with an
-// infinity or a NaN is marked instead, and every output it touches is summed in
-// plain fp32 from the original operands (split_exact_outputs).
+// infinity or a NaN is marked instead and its planes hold the two halves of the
+// fp32 words, from which every output it touches is summed in plain fp32
+// (split_exact_outputs).
+//
+// What surrounds a product in a block is folded in: before it the RMSNorm of x's
+// rows (formed as the rows are split, never stored in fp32: 13.1 us at 4096 x 512
+// with W [2730, 512], against 7.2 + 11.9 apart), after it the residual add (22 us
+// against 21 + 5.4) or the MLP's SwiGLU (whose gate and up features lie in
+// neighbouring 32-row blocks of the split W, so one wave holds both: 42 us against
+// 66 + 13.6). The layer's skip and gate before out_proj stay a kernel of their own:
+// formed here their three operands' loads wait on one another, 29 us at 2048 x
+// 1024 against 9 + 11 apart.
 //
 // Two kernels. split_rows_kernel writes both operands' hi and lo planes in the
 // order the product reads them: 1 KiB fragments of 32 rows x 16 k, a lane's
@@ -29,6 +39,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "causal_conv.hpp"
 #include "scan_ops.hpp"
 
 namespace kla {
@@ -45,15 +56,21 @@ constexpr int kSplitMarked = 1 << 20;                // row exponent of a row wi
 struct SplitOperand {
   const float *src;    // [rows, k], row stride ld
   int64_t ld, rows;
-  _Float16 *dst;       // [ceil(rows / 32)][chunks][2 k halves][2 planes][64 lanes][8]
-  int *exps;           // [ceil(rows / 32) * 32]: s = src * 2^(kSplitExp - exp), or kSplitMarked
-  int64_t blocks;      // ceil(rows / 32)
+  _Float16 *dst;       // [blocks][chunks][2 k halves][2 planes][64 lanes][8]
+  int *exps;           // [blocks * 32]: s = src * 2^(kSplitExp - exp), or kSplitMarked
+  int64_t blocks;      // 32-row blocks
 };
 
 struct SplitParams {
-  SplitOperand op[2];
+  SplitOperand op[2];  // x, W
   int64_t k;
   int64_t chunks;      // ceil(k / 32)
+  // NORM: x -> (x * rsqrt(mean(x^2) + eps)) * norm_w
+  const float *norm_w;
+  float eps;
+  // Nonzero: W's blocks alternate between rows 32 i .. (gate) and glu_off + 32 i ..
+  // (up) of two halves of glu_rows rows.
+  int64_t glu_off, glu_rows;
 };
 
 // One workgroup takes 32 rows. Lane l of a wave holds, for each of the wave's
@@ -62,7 +79,8 @@ struct SplitParams {
 // fragment f of the chunk is its values 8 f .. 8 f + 7. Which k a lane's eight
 // values are does not matter to the product as long as both operands agree.
 // NC > 0: the chunks of a wave stay in registers between the row maximum and
-// the conversion (at most NC of them); NC = 0 reads the rows twice.
+// the conversion (at most NC of them); NC = 0 reads the rows twice. It moves 8
+// bytes an element (read, written), at 3.6 to 4.5 TB/s from 4096 rows on.
 constexpr int kSplitThreads = 512;
 
 // Four floats at any 4-byte boundary: global loads of gfx950 need no more, so
@@ -88,65 +106,107 @@ __device__ __forceinline__ void split_load16(float (&x)[16], const float *row, i
   }
 }
 
-template <int NC>
+template <int NC, bool NORM>
 __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p) {
   constexpr int NWV = kSplitThreads / kWave;
   __shared__ uint32_t s_max[NWV][kSplitRows];
+  __shared__ float s_sum[NORM ? NWV : 1][kSplitRows];
   const bool second = static_cast<int64_t>(blockIdx.x) >= p.op[0].blocks;
   const SplitOperand &op = p.op[second ? 1 : 0];
   const int64_t blk = static_cast<int64_t>(blockIdx.x) - (second ? p.op[0].blocks : 0);
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid % kWave, wave = tid / kWave;
   const int r = lane % kSplitRows, half = lane / kSplitRows;
-  const int64_t row = blk * kSplitRows + r;
-  const bool in = row < op.rows;
-  const float *src = op.src + (in ? row : 0) * op.ld;
+  int64_t row = blk * kSplitRows + r;
+  bool in = row < op.rows;
+  if (second && p.glu_off) {
+    row = (blk / 2) * kSplitRows + r;
+    in = row < p.glu_rows;
+    row += blk % 2 ? p.glu_off : 0;
+  }
+  const int64_t src_row = in ? row : 0, kin = in ? p.k : 0;
+  const float *src = op.src + src_row * op.ld;
+  const bool norm = NORM && !second;
+
+  auto load = [&](float (&v)[16], int64_t ch) { split_load16(v, src, ch * kSplitK + 16 * half, kin); };
 
   constexpr int HELD = NC > 0 ? NC : 1;
   float x[HELD][16];
-  uint32_t top = 0;
-  auto scan = [&](const float (&v)[16]) {
+  uint32_t top = 0;     // the largest magnitude's bits (of x norm_w, before the row's scale, with the norm)
+  float squares = 0.0f;
+  auto scan = [&](const float (&v)[16], int64_t ch) {
+    float w[16];
+    if (norm) split_load16(w, p.norm_w, ch * kSplitK + 16 * half, kin);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const uint32_t b = __float_as_uint(v[i]) & 0x7fffffffu;
+      uint32_t b = __float_as_uint(v[i]) & 0x7fffffffu;
+      if (norm) {
+        squares = fmaf(v[i], v[i], squares);
+        const uint32_t c = __float_as_uint(v[i] * w[i]) & 0x7fffffffu;
+        b = b >= 0x7f800000u ? b : c;
+      }
       top = b > top ? b : top;
     }
   };
   if constexpr (NC > 0) {
 #pragma unroll
-    for (int i = 0; i < NC; ++i)
-      split_load16(x[i], src, (wave + static_cast<int64_t>(i) * NWV) * kSplitK + 16 * half, in ? p.k : 0);
+    for (int i = 0; i < NC; ++i) load(x[i], wave + static_cast<int64_t>(i) * NWV);
 #pragma unroll
-    for (int i = 0; i < NC; ++i) scan(x[i]);
+    for (int i = 0; i < NC; ++i) scan(x[i], wave + static_cast<int64_t>(i) * NWV);
   } else {
     for (int64_t ch = wave; ch < p.chunks; ch += NWV) {
-      split_load16(x[0], src, ch * kSplitK + 16 * half, in ? p.k : 0);
-      scan(x[0]);
+      load(x[0], ch);
+      scan(x[0], ch);
     }
   }
   const uint32_t other = __shfl_xor(top, 32);
   top = other > top ? other : top;
   if (half == 0) s_max[wave][r] = top;
+  if constexpr (NORM) {
+    squares += __shfl_xor(squares, 32);
+    if (half == 0) s_sum[wave][r] = squares;
+  }
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < NWV; ++w) top = s_max[w][r] > top ? s_max[w][r] : top;
+  float scale = 1.0f;
+  if constexpr (NORM) {
+    if (norm) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NWV; ++w) ss += s_sum[w][r];
+      scale = rsqrtf(ss / static_cast<float>(p.k) + p.eps);
+    }
+  }
+  // (With the norm the bound on the row's largest magnitude may round up to a power
+  // of two: |s| then stays below 2^15 (1 + 2^-22).)
   const bool marked = top >= 0x7f800000u;
+  float bound = __uint_as_float(top);
+  if (NORM && !marked) bound *= scale;
   // The exponent of the row's largest magnitude (that of 1 for a row of zeros).
   int ex = 0;
-  if (!marked && top != 0) ex = __builtin_amdgcn_frexp_expf(__uint_as_float(top)) - 1;
-  if (wave == 0 && half == 0) op.exps[row] = marked ? kSplitMarked : ex;
+  if (!marked && bound != 0.0f) ex = __builtin_amdgcn_frexp_expf(bound) - 1;
+  if (wave == 0 && half == 0) op.exps[blk * kSplitRows + r] = marked ? kSplitMarked : ex;
 
   const int shift = kSplitExp - ex;
   auto put = [&](const float (&v)[16], int64_t ch) {
     _Float16 *out = op.dst + (blk * p.chunks + ch) * kSplitChunk + lane * 8;
+    float w[16];
+    if (norm) split_load16(w, p.norm_w, ch * kSplitK + 16 * half, kin);
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
       f16x8_t hi, lo;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float s = marked ? 0.0f : ldexpf(v[8 * f + i], shift);
+        const float u = norm ? (v[8 * f + i] * scale) * w[8 * f + i] : v[8 * f + i];
+        const float s = ldexpf(u, shift);
         hi[i] = static_cast<_Float16>(s);
         lo[i] = static_cast<_Float16>(s - static_cast<float>(hi[i]));
+        if (marked) {
+          const uint32_t b = __float_as_uint(u);
+          hi[i] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(b >> 16));
+          lo[i] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(b));
+        }
       }
       *reinterpret_cast<f16x8_t *>(out + (2 * f) * 512) = hi;
       *reinterpret_cast<f16x8_t *>(out + (2 * f + 1) * 512) = lo;
@@ -160,34 +220,70 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
     }
   } else {
     for (int64_t ch = wave; ch < p.chunks; ch += NWV) {
-      split_load16(x[0], src, ch * kSplitK + 16 * half, in ? p.k : 0);
+      load(x[0], ch);
       put(x[0], ch);
     }
   }
 }
 
+enum SplitEpilogue { kGemmPlain = 0, kGemmResidual = 1, kGemmSwiglu = 2 };
+
 struct SplitGemmParams {
   const _Float16 *xs, *ws;       // split planes of x (tokens) and W (features)
   const int *xe, *we;            // row exponents
-  const float *x, *w, *bias;     // the fp32 operands (marked rows), bias [n] or NULL
+  const float *w, *bias;         // W itself (row stride ldw; marked rows), bias by W's rows or NULL
+  const float *res;              // [rows, n], row stride ldres (kGemmResidual)
   float *y;                      // [rows, n], row stride ldy
-  int64_t ldx, ldw, ldy, rows, n, k, chunks;
+  int64_t ldw, ldres, ldy, rows, n, k, chunks;
+  int64_t glu_off;               // kGemmSwiglu: W row of the up half of output column 0
   int64_t xblocks, wblocks;      // 32-row blocks of x and of W
-  int64_t tiles_n, tiles_t;      // output tiles over features and tokens
+  int64_t tiles_n, tiles_t;      // output tiles over W's blocks and tokens
 };
 
-// Outputs of the tile that a marked row touches, one at a time in plain fp32.
-template <int TN, int TT>
+// Element (row of the split operand, k) in fp32: as it was in a marked row, else the
+// sum of its planes with the row's scale.
+__device__ __forceinline__ float split_element(const _Float16 *planes, int64_t chunks, int e, int64_t row, int64_t k) {
+  const int64_t at = ((row / kSplitRows) * chunks + k / kSplitK) * kSplitChunk + 2 * ((k % 16) / 8) * 512 +
+                     ((k % kSplitK) / 16 * 32 + row % kSplitRows) * 8 + k % 8;
+  const _Float16 hi = planes[at], lo = planes[at + 512];
+  if (e == kSplitMarked)
+    return __uint_as_float(static_cast<uint32_t>(__builtin_bit_cast(uint16_t, hi)) << 16 |
+                           __builtin_bit_cast(uint16_t, lo));
+  return ldexpf(static_cast<float>(hi) + static_cast<float>(lo), e - kSplitExp);
+}
+
+// silu(g) u, as the MLP forms it.
+__device__ __forceinline__ float swiglu_value(float g, float u) { return activation(kActSilu, g) * u; }
+
+// Outputs of the tile that a marked row touches, one at a time in plain fp32: n0 and
+// TN count W's blocks' rows (two a column with SwiGLU).
+template <int EPI, int TN, int TT>
 __device__ __forceinline__ void split_exact_outputs(const SplitGemmParams &p, int64_t n0, int64_t t0) {
-  for (int e = static_cast<int>(threadIdx.x); e < TN * TT; e += static_cast<int>(blockDim.x)) {
-    const int64_t n = n0 + e % TN, t = t0 + e / TN;
-    if (n >= p.n || t >= p.rows) continue;
-    if (p.xe[t] != kSplitMarked && p.we[n] != kSplitMarked) continue;
-    const float *a = p.x + t * p.ldx, *b = p.w + n * p.ldw;
+  auto dot = [&](int64_t t, int64_t w_row) {
+    const int xe = p.xe[t];
+    const float *w = p.w + w_row * p.ldw;
     float s = 0.0f;
-    for (int64_t i = 0; i < p.k; ++i) s = fmaf(a[i], b[i], s);
-    if (p.bias) s += p.bias[n];
-    p.y[t * p.ldy + n] = s;
+    for (int64_t i = 0; i < p.k; ++i) s = fmaf(split_element(p.xs, p.chunks, xe, t, i), w[i], s);
+    return s;
+  };
+  constexpr int COLS = EPI == kGemmSwiglu ? TN / 2 : TN;
+  for (int e = static_cast<int>(threadIdx.x); e < COLS * TT; e += static_cast<int>(blockDim.x)) {
+    const int64_t t = t0 + e / COLS;
+    const int64_t n = (EPI == kGemmSwiglu ? n0 / 2 : n0) + e % COLS;
+    if (n >= p.n || t >= p.rows) continue;
+    const int64_t wr = EPI == kGemmSwiglu ? (n / 32) * 64 + n % 32 : n;
+    const bool m = p.xe[t] == kSplitMarked || p.we[wr] == kSplitMarked;
+    float v;
+    if constexpr (EPI == kGemmSwiglu) {
+      if (!m && p.we[wr + 32] != kSplitMarked) continue;
+      const float g = dot(t, n) + (p.bias ? p.bias[n] : 0.0f);
+      v = swiglu_value(g, dot(t, p.glu_off + n) + (p.bias ? p.bias[p.glu_off + n] : 0.0f));
+    } else {
+      if (!m) continue;
+      v = dot(t, n) + (p.bias ? p.bias[n] : 0.0f);
+      if constexpr (EPI == kGemmResidual) v = p.res[t * p.ldres + n] + v;
+    }
+    p.y[t * p.ldy + n] = v;
   }
 }
 
@@ -231,7 +327,7 @@ __device__ __forceinline__ void fragment_to_lds(const char *src, uint32_t lane_o
 //   2048 x 2048, k 1024    32 + 10 /   72       256 x 2048, k 512     8 +  8 /   20
 // Through registers instead of straight into LDS, one chunk ahead: 426 us for the
 // first; with the compiler's waits (every load before each read of LDS) 397.
-template <int WAVN, int WAVT, int FN, int FT, int ST, int OCC>
+template <int EPI, int WAVN, int WAVT, int FN, int FT, int ST, int OCC>
 __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(SplitGemmParams p) {
   constexpr int NW = WAVN * WAVT;
   constexpr int BN = WAVN * FN, BT = WAVT * FT;          // 32-row blocks of the tile
@@ -337,12 +433,13 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   for (int i = tid; i < TN + TT; i += NW * kWave) {
     const bool isn = i < TN;
     const int64_t r = isn ? n0 + i : t0 + (i - TN);
-    const bool in = r < (isn ? p.n : p.rows);
-    const int e = in ? (isn ? p.we : p.xe)[r] : 0;
+    const int e = r < (isn ? p.wblocks : p.xblocks) * kSplitRows ? (isn ? p.we : p.xe)[r] : 0;
     marked = marked || e == kSplitMarked;
     if (isn) {
+      int64_t col = r;
+      if constexpr (EPI == kGemmSwiglu) col = (r / 64) * 32 + r % 32;
       s_we[i] = e - 2 * kSplitExp;
-      s_bias[i] = in && p.bias ? p.bias[r] : 0.0f;
+      s_bias[i] = p.bias && col < p.n ? p.bias[EPI == kGemmSwiglu && r / 32 % 2 ? p.glu_off + col : col] : 0.0f;
     } else {
       s_xe[i - TN] = e;
     }
@@ -377,25 +474,49 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   const bool vec = p.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(p.y) % 16 == 0;
+  const bool vec_res = EPI == kGemmResidual && p.ldres % 4 == 0 && reinterpret_cast<uintptr_t>(p.res) % 16 == 0;
+  static_assert(EPI != kGemmSwiglu || FN % 2 == 0, "a wave holds a gate block with its up block");
+  constexpr int STEP = EPI == kGemmSwiglu ? 2 : 1;
 #pragma unroll
-  for (int a = 0; a < FN; ++a)
+  for (int a = 0; a < FN; a += STEP)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int nl = (wn * FN + a) * kSplitRows + 8 * g + 4 * (lane / 32);
       const int4 en = *reinterpret_cast<const int4 *>(s_we + nl);
       const float4 bv = *reinterpret_cast<const float4 *>(s_bias + nl);
-      const int64_t n = n0 + nl;
+      const int64_t n = EPI == kGemmSwiglu ? n0 / 2 + (wn * FN + a) / 2 * kSplitRows + 8 * g + 4 * (lane / 32) : n0 + nl;
 #pragma unroll
       for (int b = 0; b < FT; ++b) {
         const int tl = (wt * FT + b) * kSplitRows + lane % 32;
         const int64_t t = t0 + tl;
         const int ex = s_xe[tl];
-        const float4 v = make_float4(ldexpf(acc[a][b][4 * g], ex + en.x) + bv.x,
-                                     ldexpf(acc[a][b][4 * g + 1], ex + en.y) + bv.y,
-                                     ldexpf(acc[a][b][4 * g + 2], ex + en.z) + bv.z,
-                                     ldexpf(acc[a][b][4 * g + 3], ex + en.w) + bv.w);
+        float4 v = make_float4(ldexpf(acc[a][b][4 * g], ex + en.x) + bv.x,
+                               ldexpf(acc[a][b][4 * g + 1], ex + en.y) + bv.y,
+                               ldexpf(acc[a][b][4 * g + 2], ex + en.z) + bv.z,
+                               ldexpf(acc[a][b][4 * g + 3], ex + en.w) + bv.w);
+        if constexpr (EPI == kGemmSwiglu) {
+          const int4 eu = *reinterpret_cast<const int4 *>(s_we + nl + kSplitRows);
+          const float4 bu = *reinterpret_cast<const float4 *>(s_bias + nl + kSplitRows);
+          const f32x16_t &u = acc[a + 1][b];
+          v = make_float4(swiglu_value(v.x, ldexpf(u[4 * g], ex + eu.x) + bu.x),
+                          swiglu_value(v.y, ldexpf(u[4 * g + 1], ex + eu.y) + bu.y),
+                          swiglu_value(v.z, ldexpf(u[4 * g + 2], ex + eu.z) + bu.z),
+                          swiglu_value(v.w, ldexpf(u[4 * g + 3], ex + eu.w) + bu.w));
+        }
         if (t < p.rows) {
           float *out = p.y + t * p.ldy + n;
+          if constexpr (EPI == kGemmResidual) {
+            const float *res = p.res + t * p.ldres + n;
+            if (vec_res && n + 4 <= p.n) {
+              const float4 x = *reinterpret_cast<const float4 *>(res);
+              v = make_float4(x.x + v.x, x.y + v.y, x.z + v.z, x.w + v.w);
+            } else {
+              if (n < p.n) v.x = res[0] + v.x;
+              if (n + 1 < p.n) v.y = res[1] + v.y;
+              if (n + 2 < p.n) v.z = res[2] + v.z;
+              if (n + 3 < p.n) v.w = res[3] + v.w;
+            }
+          }
           if (vec && n + 4 <= p.n) {
             *reinterpret_cast<float4 *>(out) = v;
           } else {
@@ -409,7 +530,7 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
     }
   // Marked rows or columns: their outputs once more, from the operands. (The
   // barrier orders the two stores.)
-  if (__syncthreads_or(marked)) split_exact_outputs<TN, TT>(p, n0, t0);
+  if (__syncthreads_or(marked)) split_exact_outputs<EPI, TN, TT>(p, n0, t0);
 }
 
 }  // namespace kla

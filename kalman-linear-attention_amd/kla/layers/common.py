@@ -174,6 +174,24 @@ class MLP(nn.Module):
         h = rows_linear_hip(x2, self.w12.weight, self.w12.bias, norm_weight=norm.weight, eps=norm.eps, swiglu=True)
         return rows_linear_hip(h, self.w3.weight, self.w3.bias, residual=x2).reshape(x.shape)
 
+    def block_forward_hip(self, x: torch.Tensor, norm: "RMSNorm") -> torch.Tensor | None:
+        """``x + self(norm(x))`` as two split fp32 products, the norm and the SwiGLU folded
+        into the first, the residual into the second (kla.ops.hip.linear.linear_f32),
+        or None where that does not serve: not a SwiGLU MLP in fp32 inference on a hip
+        backend over enough rows. The same operations as the torch lines."""
+        if self.kind != "swiglu" or x.dtype != torch.float32 or not _hip_inference(
+                self.backend, x, *self.parameters(), *norm.parameters()):
+            return None
+        from kla.ops.hip.linear import linear_f32, norm_args, product_ok, unhooked
+
+        w12, w3 = self.w12, self.w3
+        args = norm_args(norm, x)
+        if args is None or not unhooked(self, MLP) or not product_ok(w12, x) or w12.weight.shape[0] % 2 \
+                or not unhooked(w3, nn.Linear) or any(p.dtype != torch.float32 for p in w3.parameters()):
+            return None
+        h = linear_f32(x, w12.weight, w12.bias, norm=args, swiglu=True)
+        return linear_f32(h, w3.weight, w3.bias, residual=x)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.kind == "swiglu":
             h = _project(self.backend, self.w12, x)

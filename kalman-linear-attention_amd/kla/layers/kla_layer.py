@@ -257,31 +257,37 @@ class KLALayer(nn.Module):
             return split_last(t, sizes)
         return torch.split(t, sizes, dim=-1)
 
-    def _linear(self, mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
+    def _linear(self, mod: nn.Linear, x: torch.Tensor, residual=None) -> torch.Tensor:
         """mod(x); on a hip-family backend with a gradient to carry, the projection
         whose weight gradient is split over the tokens, and without one the split
-        fp32 product where it applies (kla.ops.hip.linear)."""
+        fp32 product where it applies (kla.ops.hip.linear). ``residual``: plus that,
+        folded into the split product."""
         if _step_on_hip(self.config.backend, x):
-            from kla.ops.hip.linear import linear, plain_linear
+            from kla.ops.hip.linear import linear, linear_f32, product_ok
 
-            return linear(mod, x) if torch.is_grad_enabled() else plain_linear(mod, x)
-        return mod(x)
+            if not torch.is_grad_enabled() and product_ok(mod, x) and (residual is None or residual.dtype == x.dtype):
+                return linear_f32(x, mod.weight, mod.bias, residual=residual)
+            out = linear(mod, x) if torch.is_grad_enabled() else mod(x)
+        else:
+            out = mod(x)
+        return out if residual is None else residual + out
 
     def _expand(self, mod: nn.Linear, x: torch.Tensor) -> torch.Tensor:
         """mod(x) for the low-rank value and variance maps; without a gradient on a
         hip-family backend as :meth:`_linear`."""
         return mod(x) if torch.is_grad_enabled() else self._linear(mod, x)
 
-    def _linear_split(self, mod: nn.Linear, x: torch.Tensor, sizes: list[int]):
+    def _linear_split(self, mod: nn.Linear, x: torch.Tensor, sizes: list[int], norm=None):
         """self._split(mod(x), sizes); on a hip-family backend with a gradient to
         carry, the projection and the split as one (kla.ops.hip.linear), and
         otherwise the split fp32 product, or the product in row blocks where the
-        pieces allow it (kla.ops.hip.linear.plain_linear, split_blocks)."""
+        pieces allow it (kla.ops.hip.linear.linear_f32, split_blocks). ``norm``: the
+        (weight, eps) of an RMSNorm of x first (given only where :meth:`block_norm` holds)."""
         if _step_on_hip(self.config.backend, x):
-            from kla.ops.hip.linear import _bare, linear_f32_ok, linear_split, plain_linear, split_blocks
+            from kla.ops.hip.linear import linear_f32, linear_split, product_ok, split_blocks
 
-            if not torch.is_grad_enabled() and _bare(mod) and linear_f32_ok(x, mod.weight, mod.bias):
-                return torch.split(plain_linear(mod, x), sizes, dim=-1)
+            if not torch.is_grad_enabled() and product_ok(mod, x):
+                return torch.split(linear_f32(x, mod.weight, mod.bias, norm=norm), sizes, dim=-1)
             pieces = linear_split(mod, x, sizes) if torch.is_grad_enabled() else None
             if pieces is None and not (torch.is_grad_enabled() and x.requires_grad):
                 pieces = split_blocks(mod, x, sizes)
@@ -454,18 +460,49 @@ class KLALayer(nn.Module):
         out = rows_linear_hip(y[:, 0], self.out_proj.weight, self.out_proj.bias, residual=x2)
         return out.unsqueeze(1), KLALayerState(conv=conv_state, ssm=ssm_state)
 
+    def block_norm(self, x: torch.Tensor, norm: nn.Module):
+        """(weight, eps) of ``norm`` where :meth:`block_forward_hip` serves ``x +
+        self(norm(x))``, else None: fp32 inference on a hip backend over enough rows for
+        the split product, no variance to return, and plain, unhooked modules."""
+        if torch.is_grad_enabled() or x.dtype != torch.float32 or self.config.return_variance:
+            return None
+        if not _step_on_hip(self.config.backend, x):
+            return None
+        from kla.ops.hip.linear import norm_args, product_ok, unhooked
+
+        if not (unhooked(self, KLALayer) and product_ok(self.in_proj, x) and unhooked(self.out_proj, nn.Linear)
+                and all(p.dtype == torch.float32 for p in self.out_proj.parameters())):
+            return None
+        return norm_args(norm, x)
+
+    def block_forward_hip(self, x: torch.Tensor, norm, state: KLALayerState | None, emit_state: bool):
+        """(``x + self(rms_norm(x))``, new state or None) over a sequence, with the norm
+        (weight, eps) folded into in_proj and the residual into out_proj where they run
+        as split products (kla.ops.hip.linear.linear_f32). The same operations."""
+        out = self._forward(x, state, emit_state, norm=norm, residual=x)
+        return out if emit_state else (out, None)
+
     def forward(self, x: torch.Tensor, state: KLALayerState | None = None, return_state: bool = False):
         """x [B, L, d_model] -> out, or (out, new_state) when a state is passed or requested.
 
         ``out`` is y, or (y, y_var) when ``config.return_variance``.
         """
+        return self._forward(x, state, return_state)
+
+    def _forward(self, x, state, return_state, norm=None, residual=None):
+        """forward; with ``norm`` (weight, eps) and ``residual``, ``residual +
+        forward(rms_norm(x))`` (see block_forward_hip)."""
         cfg = self.config
         L = x.shape[1]
         emit_state = return_state or state is not None
+        block_res = residual
 
         if cfg.use_gating:
-            z, gate = self._linear_split(self.in_proj, x, [self.d_inner, self.d_inner])
+            z, gate = self._linear_split(self.in_proj, x, [self.d_inner, self.d_inner], norm)
             projected = z
+        elif norm is not None:
+            (z,) = self._linear_split(self.in_proj, x, [self.d_inner], norm)
+            projected, gate = z, None
         else:
             z = projected = self._linear(self.in_proj, x)
             gate = None
@@ -511,7 +548,7 @@ class KLALayer(nn.Module):
                     if y_var is not None:
                         y_var = y_var * g.pow(2)
 
-        out = self._linear(self.out_proj, y)
+        out = self._linear(self.out_proj, y, block_res)
         result = (out, F.linear(y_var, self.out_proj.weight.pow(2))) if cfg.return_variance else out
         if emit_state:
             return result, KLALayerState(conv=conv_state, ssm=ssm_state)

@@ -16,7 +16,7 @@ import torch
 import torch.nn as nn
 
 from kla.configs import KLAConfig, ModelConfig
-from kla.layers.common import MLP, RMSNorm, _project
+from kla.layers.common import MLP, RMSNorm, _hip_inference
 from kla.layers.kla_layer import KLALayer
 from kla.models.readout import MarginalReadout
 
@@ -65,7 +65,17 @@ class Block(nn.Module):
 
     def channel(self, x: torch.Tensor) -> torch.Tensor:
         """Channel-mixing half: x + mlp(norm(x)) (identity when there is no MLP)."""
-        return x if self.mlp is None else x + self.mlp(self.mlp_norm(x))
+        if self.mlp is None:
+            return x
+        y = self.mlp.block_forward_hip(x, self.mlp_norm)
+        return x + self.mlp(self.mlp_norm(x)) if y is None else y
+
+    def _fold_norm(self, x: torch.Tensor):
+        """(weight, eps) of the mixer's pre-norm where KLALayer.block_forward_hip serves
+        ``x + mixer(norm(x))``, else None."""
+        if x.dim() != 3 or not x.is_cuda or type(self.mixer) is not KLALayer:
+            return None
+        return self.mixer.block_norm(x, self.mixer_norm)
 
     def forward(self, x: torch.Tensor, state=None, return_state: bool = False):
         emit_state = return_state or state is not None
@@ -79,7 +89,12 @@ class Block(nn.Module):
             else:
                 x = self.channel(x)
             return x, new_state
-        if emit_state:
+        norm = self._fold_norm(x)
+        if norm is not None:
+            # Inference over a sequence in fp32: the norm folded into in_proj, the residual
+            # into out_proj.
+            x, new_state = self.mixer.block_forward_hip(x, norm, state, emit_state)
+        elif emit_state:
             mixed, new_state = self.mixer(self.mixer_norm(x), state=state, return_state=True)
             if isinstance(mixed, tuple):
                 mixed = mixed[0]
@@ -137,17 +152,26 @@ class SequenceModel(MarginalReadout, nn.Module):
                                      norm_weight=self.norm_f.weight, eps=self.norm_f.eps)
             logits = logits.reshape(*x.shape[:-1], logits.shape[-1])
         else:
-            logits = _project(self.norm_f.backend, self.lm_head, self.norm_f(x))
+            logits = self._head_product(x)
         cap = self.config.logit_softcap
         return logits if cap is None else cap * torch.tanh(logits / cap)
+
+    def _head_product(self, x: torch.Tensor) -> torch.Tensor:
+        """lm_head(norm_f(x)); in fp32 inference over a sequence on a hip backend one split
+        product with the norm folded in (kla.ops.hip.linear.linear_f32)."""
+        if x.dtype == torch.float32 and _hip_inference(self.norm_f.backend, x, self.lm_head.weight, self.norm_f.weight):
+            from kla.ops.hip.linear import linear_f32, norm_args, product_ok
+
+            norm = norm_args(self.norm_f, x)
+            if norm is not None and product_ok(self.lm_head, x):
+                return linear_f32(x, self.lm_head.weight, self.lm_head.bias, norm=norm)
+        return self.lm_head(self.norm_f(x))
 
     def _embed(self, input_ids: torch.Tensor) -> torch.Tensor:
         """Token embeddings; in inference on a hip backend one gather kernel
         (kla.ops.hip.model_ops.gather_rows_hip) instead of torch's index kernel."""
         w = self.embedding.weight
         if w.dtype in (torch.float32, torch.bfloat16) and input_ids.dtype == torch.int64:
-            from kla.layers.common import _hip_inference
-
             if _hip_inference(self.norm_f.backend, w):
                 from kla.ops.hip.model_ops import gather_rows_hip
 
@@ -160,8 +184,6 @@ class SequenceModel(MarginalReadout, nn.Module):
             return False
         if self.lm_head.weight.dtype != torch.float32 or self.norm_f.weight.dtype != torch.float32:
             return False
-        from kla.layers.common import _hip_inference
-
         return _hip_inference(self.norm_f.backend, x, self.lm_head.weight, self.norm_f.weight)
 
     def forward(self, input_ids: torch.Tensor, state: Optional[list] = None, return_state: bool = False):
@@ -191,7 +213,7 @@ class SequenceModel(MarginalReadout, nn.Module):
     def _head(self, x: torch.Tensor) -> torch.Tensor:
         """Last channel mixer + final norm + LM head + softcap, as log-probabilities."""
         x = self._last_block.channel(x)
-        logits = _project(self.norm_f.backend, self.lm_head, self.norm_f(x)).float()
+        logits = self._head_product(x).float()
         cap = self.config.logit_softcap
         if cap is not None:
             logits = cap * torch.tanh(logits / cap)
@@ -227,8 +249,6 @@ class SequenceModel(MarginalReadout, nn.Module):
 
     def _sample(self, logits: torch.Tensor, temperature: float, top_k: Optional[int]) -> torch.Tensor:
         if temperature <= 0:
-            from kla.layers.common import _hip_inference
-
             if logits.dtype == torch.float32 and logits.shape[-1] > 0 and _hip_inference(self.norm_f.backend, logits):
                 # Greedy choice as one kernel (torch.argmax's order: NaN first, ties to the lower id).
                 from kla.ops.hip.model_ops import argmax_rows_hip

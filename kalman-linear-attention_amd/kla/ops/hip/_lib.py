@@ -99,9 +99,8 @@ _SIGNATURES = {
     "kla_argmax_workspace_bytes": (ctypes.c_size_t, [_i64, _i64]),
     "kla_rows_linear_fwd": (ctypes.c_int, [ctypes.c_int, _p, _i64, _p, _i64, _p, _p, ctypes.c_float, _p, _i64, _p,
                                            _i64, _i64, _i64, _i64, _i64, _p]),
-    "kla_linear_f32_workspace_bytes": (ctypes.c_size_t, [_i64] * 3),
-    "kla_linear_f32_fwd": (ctypes.c_int, [_p, _i64, _p, _i64, _p, _p, _i64, _i64, _i64, _i64, _p, ctypes.c_size_t,
-                                          _p]),
+    "kla_linear_f32_workspace_bytes": (ctypes.c_size_t, [_i64] * 3 + [ctypes.c_int]),
+    "kla_linear_f32_fwd": (ctypes.c_int, [_p, _p, ctypes.c_size_t, _p]),
     "kla_gate_skip_bwd": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _p, _p, _p, _i64, _p, _i64, _p, ctypes.c_int,
                                          ctypes.c_int] + [_p] * 4 + [_i64] * 2 + [_p, ctypes.c_size_t, _p]),
     "kla_causal_conv_bwd": (ctypes.c_int, [ctypes.c_int, _p, _p, _i64, _i64, _p, _p, _p, ctypes.c_int, _p, _p, _p,
@@ -124,6 +123,14 @@ class DecodeConfig(ctypes.Structure):
         ("gate_activation", ctypes.c_int),
         ("skip_vector", ctypes.c_int),
     ]
+
+
+class LinearF32(ctypes.Structure):
+    """kla_linear_f32_args of include/kla_hip.h."""
+
+    _fields_ = ([("epilogue", ctypes.c_int), ("eps", ctypes.c_float)]
+                + [(n, ctypes.c_void_p) for n in ("x", "w", "bias", "norm_w", "res", "y")]
+                + [(n, _i64) for n in ("ldx", "ldw", "ldres", "ldy", "rows", "n", "k", "glu_off")])
 
 
 class Sensors(ctypes.Structure):

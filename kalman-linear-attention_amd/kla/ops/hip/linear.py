@@ -32,6 +32,7 @@ takes it for an ``nn.Linear`` where :func:`linear_f32_ok` holds.
 
 from __future__ import annotations
 
+import ctypes
 import functools
 from typing import Optional
 
@@ -276,46 +277,74 @@ def linear_split(mod: torch.nn.Linear, x: torch.Tensor, sizes: list[int]):
 F32_MIN_ROWS = 256
 
 
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """t [..., k] as [rows, k] with a unit column stride and rows at least k apart (a view
+    where the strides allow it)."""
+    t = t.reshape(-1, t.shape[-1])
+    return t if t.stride(1) == 1 and (t.shape[0] < 2 or t.stride(0) >= t.shape[1]) else t.contiguous()
+
+
+def _ld(t: Optional[torch.Tensor]) -> int:
+    """Row stride of a [rows, k] tensor of _rows (one row: its length)."""
+    return 0 if t is None else (t.stride(0) if t.shape[0] > 1 else t.shape[1])
+
+
 @_lib.hip_op("kla_hip::linear_f32")
-def _linear_f32_op(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
-    k = x.shape[-1]
-    n = w.shape[0]
-    x2 = x.reshape(-1, k)
+def _linear_f32_op(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], norm_w: Optional[torch.Tensor],
+                   eps: float, residual: Optional[torch.Tensor], swiglu: bool) -> torch.Tensor:
+    k, n = x.shape[-1], w.shape[0] // 2 if swiglu else w.shape[0]
+    x2, res2 = _rows(x), None if residual is None else _rows(residual)
     rows = x2.shape[0]
-    lib = _lib.lib()
-    nbytes = lib.kla_linear_f32_workspace_bytes(rows, n, k)
+    epi = _lib.KLA_ROWS_SWIGLU if swiglu else _lib.KLA_ROWS_PLAIN if residual is None else _lib.KLA_ROWS_RESIDUAL
+    lib, p = _lib.lib(), _lib.ptr
+    nbytes = lib.kla_linear_f32_workspace_bytes(rows, n, k, epi)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    y = torch.empty(x.shape[:-1] + (n,), dtype=torch.float32, device=x.device)
-    _lib.check("kla_linear_f32_fwd", lib.kla_linear_f32_fwd(
-        x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), _lib.ptr(bias), y.data_ptr(), n, rows, n, k,
-        ws.data_ptr(), nbytes, _lib.stream(x.device)))
-    return y
+    # SwiGLU's result feeds a product over its columns: rows padded to 16 bytes.
+    ld = -(-n // 4) * 4 if swiglu else n
+    y = torch.empty(x.shape[:-1] + (ld,), dtype=torch.float32, device=x.device)
+    args = _lib.LinearF32(
+        epilogue=epi, eps=eps, x=p(x2), w=p(w), bias=p(bias), norm_w=p(norm_w), res=p(res2), y=p(y), ldx=_ld(x2),
+        ldw=_ld(w), ldres=_ld(res2), ldy=ld, rows=rows, n=n, k=k, glu_off=n if swiglu else 0)
+    _lib.check("kla_linear_f32_fwd", lib.kla_linear_f32_fwd(ctypes.byref(args), p(ws), nbytes, _lib.stream(x.device)))
+    return y[..., :n] if ld != n else y
 
 
 @_linear_f32_op.register_fake
-def _(x, w, bias):
-    return x.new_empty(x.shape[:-1] + (w.shape[0],))
+def _(x, w, bias, norm_w, eps, residual, swiglu):
+    n = w.shape[0] // 2 if swiglu else w.shape[0]
+    ld = -(-n // 4) * 4 if swiglu else n
+    return x.new_empty(x.shape[:-1] + (ld,))[..., :n]
 
 
-def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, *,
+               norm: Optional[tuple[torch.Tensor, float]] = None, residual: Optional[torch.Tensor] = None,
+               swiglu: bool = False) -> torch.Tensor:
     """``F.linear(x, w, bias)`` for fp32 x [..., k], w [n, k] (k > 0), bias [n] on one
     ROCm GPU, on the fp16 matrix cores from split operands: fp32 sums of exact
     products, no larger an error than the fp32 product's (measured against float64
-    at k = 512, 1024, 2048: 0.63 of it). No gradient."""
-    if x.dtype != torch.float32 or w.dtype != torch.float32 or (bias is not None and bias.dtype != torch.float32):
-        raise TypeError("linear_f32: x, w and bias must be float32")
+    at k = 512, 1024, 2048: 0.63 of it). No gradient. Folded in where given:
+    ``norm`` (weight [k], eps), RMSNorm of x's rows before it; after it ``residual``
+    [..., n], ``residual + (...)``, or ``swiglu`` (w [2 H, k]), ``silu(a[..., :H]) *
+    a[..., H:]`` of the product a (a view of rows H rounded up to 4 apart).
+    """
     k = x.shape[-1] if x.dim() else 0
-    if w.dim() != 2 or w.shape[1] != k or k == 0 or (bias is not None and tuple(bias.shape) != (w.shape[0],)):
-        raise ValueError(f"linear_f32: x {tuple(x.shape)}, w {tuple(w.shape)}, "
-                         f"bias {None if bias is None else tuple(bias.shape)}")
-    _require_device(x, w, bias)
-    if x.stride(-1) != 1 or (x.dim() > 1 and x.stride(-2) < k):
-        x = x.contiguous()
-    if w.stride(1) != 1 or w.stride(0) < k:
+    n = w.shape[0] // 2 if swiglu else w.shape[0]
+    norm_w = norm[0] if norm else None
+    for name, t, shape in (("x", x, x.shape), ("w", w, (w.shape[0], k)), ("bias", bias, (w.shape[0],)),
+                           ("norm", norm_w, (k,)), ("residual", residual, (*x.shape[:-1], n))):
+        if t is None:
+            continue
+        if t.dtype != torch.float32:
+            raise TypeError(f"linear_f32: {name} must be float32, got {t.dtype}")
+        if tuple(t.shape) != tuple(shape):
+            raise ValueError(f"linear_f32: {name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
+    if k == 0 or (swiglu and (w.shape[0] % 2 or residual is not None)):
+        raise ValueError("linear_f32: no columns, or options that do not go together")
+    _require_device(x, w, bias, norm_w, residual)
+    if w.stride(1) != 1 or (w.shape[0] > 1 and w.stride(0) < k):
         w = w.contiguous()
-    if bias is not None and bias.stride(0) != 1:
-        bias = bias.contiguous()
-    return _lib.call(_linear_f32_op, x, w, bias)
+    bias, norm_w = (None if t is None else t.contiguous() for t in (bias, norm_w))
+    return _lib.call(_linear_f32_op, x, w, bias, norm_w, float(norm[1]) if norm else 0.0, residual, swiglu)
 
 
 def linear_f32_ok(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
@@ -331,18 +360,31 @@ def linear_f32_ok(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]
     return not torch.is_autocast_enabled("cuda") and (bias is None or bias.dtype == torch.float32)
 
 
-def _bare(mod: torch.nn.Module) -> bool:
-    """Whether calling ``mod`` is F.linear on its weight and bias and nothing else: an
-    nn.Linear itself, not a subclass (nor a parametrised one), with no hooks and
-    plain parameters."""
+def unhooked(mod: torch.nn.Module, kind: type) -> bool:
+    """Whether ``mod`` is a ``kind`` itself, not a subclass (nor a parametrised one), with
+    no forward hooks: calling it runs kind.forward and nothing else."""
     hooks = torch.nn.modules.module
-    return (type(mod) is torch.nn.Linear and not (mod._forward_hooks or mod._forward_pre_hooks
-                                                  or hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
-            and type(mod.weight) in (torch.Tensor, torch.nn.Parameter))
+    return (type(mod) is kind and not (mod._forward_hooks or mod._forward_pre_hooks or hooks._global_forward_hooks
+                                       or hooks._global_forward_pre_hooks))
+
+
+def product_ok(mod: torch.nn.Module, x: torch.Tensor) -> bool:
+    """Whether ``mod(x)`` is F.linear on plain parameters and runs as :func:`linear_f32`."""
+    return (unhooked(mod, torch.nn.Linear) and type(mod.weight) in (torch.Tensor, torch.nn.Parameter)
+            and linear_f32_ok(x, mod.weight, mod.bias))
 
 
 def plain_linear(mod: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
     """``mod(x)`` for a hip-family module's nn.Linear, as :func:`linear_f32` where it applies."""
-    if _bare(mod) and linear_f32_ok(x, mod.weight, mod.bias):
-        return linear_f32(x, mod.weight, mod.bias)
-    return mod(x)
+    return linear_f32(x, mod.weight, mod.bias) if product_ok(mod, x) else mod(x)
+
+
+def norm_args(norm: torch.nn.Module, x: torch.Tensor) -> Optional[tuple[torch.Tensor, float]]:
+    """(weight, eps) of an RMSNorm that :func:`linear_f32` can form in fp32 on x, else None."""
+    from kla.layers.common import RMSNorm
+
+    w = norm.weight if unhooked(norm, RMSNorm) else None
+    if w is None or type(w) not in (torch.Tensor, torch.nn.Parameter) or w.dtype != torch.float32 \
+            or tuple(w.shape) != tuple(x.shape[-1:]) or (torch.is_grad_enabled() and w.requires_grad):
+        return None
+    return w, norm.eps

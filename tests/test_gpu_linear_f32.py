@@ -87,7 +87,7 @@ def test_which_calls_take_it(cuda, monkeypatch):
     dtypes keep the module's own call."""
     calls = []
     orig = lin.linear_f32
-    monkeypatch.setattr(lin, "linear_f32", lambda *a: calls.append(1) or orig(*a))
+    monkeypatch.setattr(lin, "linear_f32", lambda *a, **kw: calls.append(1) or orig(*a, **kw))
     mod = torch.nn.Linear(64, 80).to(cuda)
     x = torch.randn(2, 200, 64, device=cuda)
 
@@ -147,3 +147,103 @@ def test_under_graph_capture_and_on_two_streams(cuda):
         torch.cuda.synchronize()
         assert torch.equal(out, want[i])
         assert torch.equal(lin.linear_f32(xs[i], w), want[i])
+
+
+def _folded(x, w, bias, opts):
+    """linear_f32's options in float64, and the operand of the product."""
+    xd = x.double()
+    if "norm" in opts:
+        nw, eps = opts["norm"]
+        xd = xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + eps) * nw.double()
+    a = xd @ w.double().t() + bias.double()
+    if opts.get("swiglu"):
+        h = w.shape[0] // 2
+        return F.silu(a[..., :h]) * a[..., h:], xd, a
+    return (a if "residual" not in opts else opts["residual"].double() + a), xd, a
+
+
+@pytest.mark.parametrize("rows,n,k", [(1, 2, 1), (33, 64, 31), (65, 66, 513), (300, 130, 1030), (70, 1366, 2060),
+                                      (1030, 2050, 64)])
+@pytest.mark.parametrize("what", ["norm", "norm+swiglu", "norm+residual", "swiglu", "residual"])
+def test_folded_options_match_float64(cuda, rows, n, k, what):
+    print(f"[linear_f32] {what} {rows} x {k} -> {n}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(rows + n + k)
+
+    def rn(*s):
+        return torch.randn(*s, device=cuda, generator=g)
+
+    x, w, bias, opts = rn(rows, k), rn(n, k) * k ** -0.5, rn(n), {}
+    if "norm" in what:
+        opts["norm"] = (1 + 0.1 * rn(k), 1e-5)
+    if "residual" in what:
+        opts["residual"] = rn(rows, n)
+    if "swiglu" in what:
+        opts["swiglu"] = True
+    got = lin.linear_f32(x, w, bias, **opts)
+    want, xd, a = _folded(x, w, bias, opts)
+    # The product's bound on the operand formed in fp32: the norm's few roundings
+    # (a sum of k squares among them) and hardware exp, 2^-21 of it each element.
+    prod = _bound(xd, w) + (2.0 ** -21 + k * 2.0 ** -25) * (xd.abs() @ w.double().abs().t()) + 2.0 ** -22 * a.abs()
+    if "swiglu" in opts:
+        h = n // 2
+        ga, ua = a[:, :h], a[:, h:]
+        # silu' <= 1.1; silu itself good to 2^-20 of its value plus its argument's error.
+        bound = 1.1 * prod[:, :h] * (ua.abs() + prod[:, h:]) + F.silu(ga).abs() * prod[:, h:] + 2.0 ** -20 * want.abs()
+    else:
+        bound = prod + 2.0 ** -22 * want.abs()
+    assert got.shape == want.shape
+    assert ((got.double() - want).abs() / (bound + 1e-30)).max().item() <= 1.0
+
+
+def test_folded_options_with_infinities_and_nans(cuda):
+    g = torch.Generator(device=cuda).manual_seed(8)
+    x, w, bias = (torch.randn(*s, device=cuda, generator=g) for s in ((100, 70), (96, 70), (96,)))
+    nw, res = torch.ones(70, device=cuda), torch.randn(100, 96, device=cuda, generator=g)
+    x[3, 4], x[64, 0], w[9, 2], x[5] = float("inf"), float("nan"), -float("inf"), 1e30
+    for opts in ({"norm": (nw, 1e-5), "swiglu": True}, {"norm": (nw, 1e-5), "residual": res}, {"residual": res}):
+        got, xw = lin.linear_f32(x, w, bias, **opts), x.clone()
+        if "norm" in opts:      # fp32 squares of 1e30 overflow, as torch's do: the row normalises to 0
+            xw[5] = 0
+        want = _folded(xw, w, bias, opts)[0]
+        rows = [i for i in range(100) if i not in (3, 64)]
+        cols = [i for i in range(want.shape[1]) if i != 9]
+        scale = want[rows][:, cols].abs().amax(1, keepdim=True)
+        assert ((got[rows][:, cols].double() - want[rows][:, cols]).abs() <= 1e-4 * scale).all()
+        for r in (3, 64):
+            assert torch.equal(torch.isfinite(got[r]), torch.isfinite(want[r].float())), (opts.keys(), r)
+        assert not torch.isfinite(got[rows, 9]).all()
+
+
+def test_blocks_fold_their_norms_and_residuals(cuda, monkeypatch):
+    """A block's prefill with the folded products against the same modules called one by
+    one (hooks on them), with and without a state; a hook keeps its module's own call."""
+    from kla import KLAConfig
+    from kla.configs import ModelConfig
+    from kla.models import Block
+
+    torch.manual_seed(0)
+    for cfg in (KLAConfig(backend="hip"), KLAConfig(backend="hip", use_gating=False, value_rank="conv", var_rank="dt"),
+                KLAConfig(backend="hip", lambda_skip_mode="vector", gating_activation="gelu", bias=True)):
+        block = Block(48, cfg, ModelConfig(d_model=48, mlp_ratio=3.0)).to(cuda)
+        x = torch.randn(3, 100, 48, device=cuda)
+        folded = []
+        orig = lin.linear_f32
+        monkeypatch.setattr(lin, "linear_f32", lambda *a, **kw: folded.append(set(kw)) or orig(*a, **kw))
+        with torch.no_grad():
+            y, st = block(x, return_state=True)
+            y2 = block(x)
+            assert any("norm" in f for f in folded) and any("swiglu" in f for f in folded)
+            assert torch.equal(y, y2)
+            folded.clear()
+            seen = []
+            hooks = [m.register_forward_hook(lambda m, a, o: seen.append(type(m).__name__)) for m in
+                     (block.mixer_norm, block.mlp_norm, block.mixer.in_proj, block.mixer.out_proj, block.mlp.w12)]
+            want, wst = block(x, return_state=True)
+            assert len(seen) == 5 and not any("norm" in f or "swiglu" in f for f in folded)
+            for h in hooks:
+                h.remove()
+            monkeypatch.setattr(lin, "linear_f32", orig)
+        # Two fp32 evaluations of one block, a few products deep.
+        assert torch.allclose(y, want, rtol=1e-4, atol=1e-5 * want.abs().max().item())
+        for a, b in zip((st.conv, *st.ssm), (wst.conv, *wst.ssm)):
+            assert torch.allclose(a, b, rtol=1e-4, atol=1e-5 * b.abs().max().item())
