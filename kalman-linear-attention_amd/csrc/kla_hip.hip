@@ -1693,12 +1693,16 @@ void split_rows_launch(const SplitParams &sp, hipStream_t stream) {
 
 template <int EPI>
 void split_gemm_launch(SplitGemmParams g, hipStream_t stream) {
-  // The widest tile that still gives every CU two workgroups (512 on 256 CUs):
-  // a workgroup alone on a CU waits out its barriers, and 128 x 128 moves half
-  // the operand bytes per product of 64 x 64. Measured (us, k = 1024): 4096 x
-  // 2048 outputs 53 (128 x 128) / 58 (128 x 64) / 62 (64 x 64), 2048 x 2048
-  // 33.2 / 31.5 / 33.5, 2048 x 512 25.0 / 17.4 / 12.1. (SwiGLU needs two blocks
-  // of W a wave, which 64 x 64 does not have.)
+  // The widest tile that still gives every CU two workgroups (512 on 256 CUs): a
+  // workgroup alone on a CU waits out its barriers, and a wider tile moves fewer
+  // operand bytes a product. Measured (us; tiles of W rows x tokens 256 x 128 / 128 x
+  // 128 / 128 x 64 / 64 x 64):
+  //   8188 x 4096, k 2048  329 / 341 / 378 / 441     4096 x 2048, k 1024  55 / 52 / 55 / 60
+  //   8188 x 4096, k 1024  183 / 190 / 203 / 236     2048 x 2048, k 1024  46 / 31 / 31 / 33
+  //   4096 x 50304, k 512  715 / 697 / 761 / 846     2048 x  512, k 1024  42 / 24 / 18 / 12
+  // 256 x 128 pays from four workgroups a CU and k = 1024 on, where its long prologue
+  // and epilogue are a small part. (SwiGLU needs two blocks of W a wave, which 64 x 64
+  // does not have.)
   constexpr int64_t kFill = 2 * 256;
   auto tiles = [&](int bn, int bt) { return ((g.wblocks + bn - 1) / bn) * ((g.xblocks + bt - 1) / bt); };
   auto go = [&](auto kernel, int bn, int bt) {
@@ -1706,11 +1710,12 @@ void split_gemm_launch(SplitGemmParams g, hipStream_t stream) {
     g.tiles_t = (g.xblocks + bt - 1) / bt;
     hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(g.tiles_n * g.tiles_t)), dim3(4 * kWave), 0, stream, g);
   };
-  if (tiles(4, 4) >= kFill) return go(split_gemm_kernel<EPI, 2, 2, 2, 2, 2, 2>, 4, 4);
+  if (tiles(8, 4) >= 2 * kFill && g.k >= 1024) return go(split_gemm_kernel<EPI, 2, 2, 4, 2, 1, 3, 2>, 8, 4);
+  if (tiles(4, 4) >= kFill) return go(split_gemm_kernel<EPI, 2, 2, 2, 2, 1, 3, 3>, 4, 4);
   if constexpr (EPI != kGemmSwiglu) {
-    if (tiles(4, 2) < kFill) return go(split_gemm_kernel<EPI, 2, 2, 1, 1, 3, 3>, 2, 2);
+    if (tiles(4, 2) < kFill) return go(split_gemm_kernel<EPI, 2, 2, 1, 1, 2, 3, 3>, 2, 2);
   }
-  go(split_gemm_kernel<EPI, 2, 2, 2, 1, 2, 3>, 4, 2);
+  go(split_gemm_kernel<EPI, 2, 2, 2, 1, 1, 4, 3>, 4, 2);
 }
 
 int linear_f32(const char *fn, const kla_linear_f32_args &a, void *workspace, size_t workspace_bytes,

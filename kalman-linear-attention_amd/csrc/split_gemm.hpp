@@ -316,23 +316,26 @@ __device__ __forceinline__ void fragment_to_lds(const char *src, uint32_t lane_o
 // WAVN x WAVT waves, each FN x FT fragments of 32 features x 32 tokens. W is
 // the MFMA's A operand, so a lane ends with four consecutive features of one
 // token (D[8 (i / 4) + 4 (lane / 32) + i % 4][lane % 32]) and stores them as one
-// 16-byte word. Chunks of 32 k go straight from memory into ST stages of LDS,
-// ST - 1 chunks ahead of the products.
+// 16-byte word. Steps of 16 KH k (KH halves of a chunk) go straight from memory
+// into ST stages of LDS, ST - 1 steps ahead of the products.
 //
-// Bound by the matrix cores, which draw the clock down at this load (torch's
-// bf16 product of 8192^3 reaches 1.32 PFLOP/s here; 382 TFLOP/s of fp32 product
-// are 1.15 of fp16). Both kernels / the library's fp32 product, us:
-//   8188 x 4096, k 2048   360 + 43 /  967      4096 x 50304, k 512  745 + 36 / 1528
-//   8188 x 1024, k 2048    96 + 39 /  258      4096 x 2048, k 1024   53 + 11 /  124
-//   2048 x 2048, k 1024    32 + 10 /   72       256 x 2048, k 512     8 +  8 /   20
-// Through registers instead of straight into LDS, one chunk ahead: 426 us for the
-// first; with the compiler's waits (every load before each read of LDS) 397.
-template <int EPI, int WAVN, int WAVT, int FN, int FT, int ST, int OCC>
+// Bound by the matrix cores and what feeds them: a wave alone keeps them half busy
+// (LDS reads and the barrier of a step), so two or three workgroups share a CU,
+// and this load draws the clock down (torch's bf16 product of 8192^3 reaches 1.32
+// PFLOP/s here; 417 TFLOP/s of fp32 product are 1.25 of fp16). Split + product /
+// the library's fp32 product, us:
+//   8188 x 4096, k 2048   46 + 329 /  961      4096 x 50304, k 512   36 + 697 / 1539
+//   8188 x 1024, k 2048   40 +  94 /  264      4096 x 2048, k 1024   11 +  52 /  124
+//   2048 x 2048, k 1024   10 +  31 /   67       256 x 2048, k 512     8 +   8 /   19
+// The first through registers instead of straight into LDS: 426; with the
+// compiler's waits (every load before each read of LDS) 397; 128 x 128 tiles with
+// whole chunks, two stages: 354, with half chunks, three stages: 341.
+template <int EPI, int WAVN, int WAVT, int FN, int FT, int KH, int ST, int OCC>
 __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(SplitGemmParams p) {
   constexpr int NW = WAVN * WAVT;
   constexpr int BN = WAVN * FN, BT = WAVT * FT;          // 32-row blocks of the tile
   constexpr int TN = BN * kSplitRows, TT = BT * kSplitRows;
-  constexpr int FRAGS = (BN + BT) * 4;                   // 1 KiB fragments of a chunk (2 halves x 2 planes)
+  constexpr int FRAGS = (BN + BT) * 2 * KH;               // 1 KiB fragments of a step (KH halves x 2 planes)
   constexpr int LD = FRAGS / NW;
   static_assert(FRAGS % NW == 0, "whole fragments per wave");
   static_assert(ST >= 2 && ST <= 4, "2 to 4 stages");
@@ -359,23 +362,23 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   const int64_t rest = idx - band * BAND * p.tiles_t;
   const int64_t tn = band * BAND + rest % width, tt = rest / width;
 
-  // Fragment wave + j NW of the tile's FRAGS: block / 4, half and plane % 4.
+  // Fragment wave + j NW of the tile's FRAGS: block / (2 KH), half and plane % (2 KH).
   const char *from[LD];
 #pragma unroll
   for (int j = 0; j < LD; ++j) {
     const int e = wave + j * NW;
-    const int b = e / 4;
+    const int b = e / (2 * KH);
     const bool isw = b < BN;
     int64_t blk = isw ? tn * BN + b : tt * BT + (b - BN);
     const int64_t last = (isw ? p.wblocks : p.xblocks) - 1;
     blk = blk < last ? blk : last;      // rows past the end: any block, never stored
-    from[j] = reinterpret_cast<const char *>((isw ? p.ws : p.xs) + blk * p.chunks * kSplitChunk) + (e % 4) * 1024;
+    from[j] = reinterpret_cast<const char *>((isw ? p.ws : p.xs) + blk * p.chunks * kSplitChunk) + (e % (2 * KH)) * 1024;
   }
   const uint32_t lane_off = static_cast<uint32_t>(lane) * 16;
   auto load = [&](f16x8_t *stage, int c) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < LD; ++j)
-      fragment_to_lds(from[j] + static_cast<int64_t>(c) * (kSplitChunk * 2), lane_off,
+      fragment_to_lds(from[j] + static_cast<int64_t>(c) * (kSplitChunk * KH), lane_off,
                       lds_address(stage) + (wave + j * NW) * 1024);
   };
 
@@ -388,20 +391,20 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
       for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.0f;
 
   auto products = [&](const f16x8_t *stage) __attribute__((always_inline)) {
-    const f16x8_t *sw = stage + wn * FN * 256 + lane;
-    const f16x8_t *sx = stage + (BN + wt * FT) * 256 + lane;
+    const f16x8_t *sw = stage + wn * FN * (128 * KH) + lane;
+    const f16x8_t *sx = stage + (BN + wt * FT) * (128 * KH) + lane;
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
+    for (int f = 0; f < KH; ++f) {
       f16x8_t wh[FN], wl[FN], xh[FT], xl[FT];
 #pragma unroll
       for (int a = 0; a < FN; ++a) {
-        wh[a] = sw[a * 256 + (2 * f) * 64];
-        wl[a] = sw[a * 256 + (2 * f + 1) * 64];
+        wh[a] = sw[a * (128 * KH) + (2 * f) * 64];
+        wl[a] = sw[a * (128 * KH) + (2 * f + 1) * 64];
       }
 #pragma unroll
       for (int b = 0; b < FT; ++b) {
-        xh[b] = sx[b * 256 + (2 * f) * 64];
-        xl[b] = sx[b * 256 + (2 * f + 1) * 64];
+        xh[b] = sx[b * (128 * KH) + (2 * f) * 64];
+        xl[b] = sx[b * (128 * KH) + (2 * f + 1) * 64];
       }
 #pragma unroll
       for (int q = 0; q < 3; ++q)
@@ -413,11 +416,11 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
                                                                acc[a][b], 0, 0, 0);
     }
   };
-  const int chunks = static_cast<int>(p.chunks);
-  // Chunk c: wait for its loads (those of the ST - 2 chunks after it stay in
-  // flight) and for every wave to be done with the chunk before it, refill that
-  // chunk's stage, multiply. Past the end the last chunk is loaded again, so
-  // that the count in flight is the same for every chunk.
+  const int chunks = static_cast<int>(p.chunks) * (2 / KH);
+  // Step c: wait for its loads (those of the ST - 2 steps after it stay in flight)
+  // and for every wave to be done with the step before it, refill that step's
+  // stage, multiply. Past the end the last step is loaded again, so that the count
+  // in flight is the same for every step.
   auto turn = [&](int c, f16x8_t *stage, f16x8_t *refill) __attribute__((always_inline)) {
     constexpr int kInFlight = LD * (ST - 2);
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kInFlight) : "memory");

@@ -30,7 +30,8 @@ def _check(got, x, w, bias=None):
 # (rows, n, k): single rows and columns, one off each tile (64, 128), the chunk's 32
 # and the register-held widths of the split (512, 1024, 2048), and each tile choice.
 SIZES = [(1, 1, 1), (1, 300, 31), (63, 65, 32), (64, 64, 33), (65, 129, 511), (255, 1365, 512), (257, 40, 513),
-         (300, 2080, 1025), (130, 70, 2049), (1025, 1030, 96), (2049, 2049, 40), (4100, 2100, 64)]
+         (300, 2080, 1025), (130, 70, 2049), (1025, 1030, 96), (2049, 2049, 40), (4100, 2100, 64),
+         (8100, 4200, 1024)]
 
 
 @pytest.mark.parametrize("rows,n,k", SIZES)
