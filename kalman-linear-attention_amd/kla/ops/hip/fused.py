@@ -97,14 +97,33 @@ def train_chunks(B: int, L: int, M: int, S: int, cus: int) -> int:
     return nc
 
 
+def _split_cost(L: int, steps: int, base: int, cus: int, train: bool) -> float:
+    """What a sequence of L steps in chunks of ``steps`` on ``base`` workgroups a chunk
+    takes, in steps of the whole walk on a grid that leaves CUs idle (0.083 us a step
+    forward, 0.32 us forward and backward, M 1000, S 16). Fitted to MI355X: the forward's
+    split adds two launches and a second pass, and is bound by the chunks' two walks
+    while they leave issue slots free, then by their work; the training pair walks a
+    chunk 2.6 times as long a step with one workgroup a CU, 3.2 with two."""
+    if steps >= L:
+        return L
+    if train:
+        return 80 + (2.6 if base * -(-L // steps) <= cus else 3.2) * steps
+    return 145 + max(2.0 * steps, 1.2 * L * base / cus)
+
+
 def ragged_chunk(B: int, L: int, M: int, S: int, cus: int, nc: int, train: bool) -> int:
     """Steps of a chunk where the equal split into ``nc`` chunks (time_chunks, or
     train_chunks with ``train``) ended because 2 nc does not divide L (into whole
     checkpoint blocks with ``train``), though the grid still leaves CUs idle: chunks
     of this many steps, the last one shorter (0: keep the equal split). A multiple of
     16 near MIN_CHUNK or above, with which the grid reaches what the equal planners
-    aim at. One sequence of 1021 steps (M 1024, S 16) runs 86 us whole and 38 us in
-    eight chunks on MI355X."""
+    aim at, and only where _split_cost says a tenth or more is gained, in training also
+    80 us (250 steps): its five more launches take 30 us of host time where the host
+    is what a pass waits for. Whole / split, us on MI355X (M 1000, S 16): forward, one
+    sequence of 301 steps 30 / 36, 501 46 / 35, 1021 86 / 42; two of 389 38 / 43, 501
+    46 / 40, 1021 87 / 65; three of 1021 87 / 86. Forward and backward, one sequence of
+    643 steps 234 / 264 (host), 1021 339 / 264, 1501 487 / 264; two of 1501 490 / 344;
+    three of 1501 494 / 521."""
     if L % ((32 if train else 2) * nc) == 0:
         return 0
     sp, base = _grid(B, M, S)
@@ -115,7 +134,10 @@ def ragged_chunk(B: int, L: int, M: int, S: int, cus: int, nc: int, train: bool)
     if want <= nc:
         return 0
     steps = -(-L // (16 * want)) * 16
-    return steps if MIN_CHUNK <= steps < L else 0
+    if not MIN_CHUNK <= steps < L:
+        return 0
+    split, even = _split_cost(L, steps, base, cus, train), _split_cost(L, -(-L // nc), base, cus, train)
+    return steps if split < 0.9 * even and (not train or split + 250 < even) else 0
 
 
 def _plan(B: int, L: int, M: int, S: int, dev: torch.device, train: bool) -> tuple[int, int]:

@@ -14,10 +14,15 @@ def test_ragged_plan():
     plan = fused.ragged_chunk
     # 64 workgroups: eight chunks of 128 steps, the last one of 125.
     assert plan(1, 1021, 1024, 16, 256, 1, False) == 128
-    assert plan(1, 257, 1024, 16, 256, 1, False) == 144      # the fewest steps that make two chunks: 144 + 113
+    assert plan(1, 301, 1024, 16, 256, 1, False) == 0        # two chunks gain less than their launches
+    assert plan(1, 501, 1024, 16, 256, 1, False) == 128      # four do: 3 x 128 + 117
     assert plan(1, 191, 1024, 16, 256, 1, False) == 0        # one chunk
     assert plan(1, 2500, 8, 16, 256, 4, False) == 128        # four equal chunks leave the grid small
-    assert plan(2, 500, 768, 16, 256, 1, True) == 128        # 96 workgroups with gradients
+    assert plan(2, 389, 1000, 16, 256, 1, False) == 0        # 126 workgroups: the second pass is not free
+    assert plan(3, 1501, 1000, 16, 256, 1, False) == 0
+    assert plan(2, 1021, 1000, 16, 256, 1, True) == 208      # with gradients
+    assert plan(1, 643, 1000, 16, 256, 1, True) == 0         # gains less than its launches take of the host
+    assert plan(2, 500, 768, 16, 256, 1, True) == plan(3, 1501, 1000, 16, 256, 1, True) == 0
     assert plan(4, 1023, 1024, 16, 256, 1, False) == 0       # one workgroup per CU already
     assert plan(1, 1024, 1024, 16, 256, 8, False) == 0       # equal chunks serve
     assert plan(0, 1021, 1024, 16, 256, 1, False) == plan(1, 1021, 0, 16, 256, 1, True) == 0
@@ -73,7 +78,7 @@ def test_forced_ragged_split_matches_float64(cuda, monkeypatch, shape, steps, wi
 
 @pytest.mark.gpu
 def test_unforced_ragged_lengths_match_float64(cuda):
-    for B, L, M, S in ((1, 1021, 64, 16), (2, 389, 40, 8)):
+    for B, L, M, S in ((1, 1021, 64, 16), (2, 771, 40, 8)):
         ins = make_inputs(B, L, M, S, seed=33)
         cus = fused._cus(cuda.index or 0)
         assert fused.ragged_chunk(B, L, M, S, cus, fused.time_chunks(B, L, M, S, cus), False)
