@@ -154,9 +154,8 @@ class KLALayer(nn.Module):
         cfg = self.config
         S = self.d_state
         if self._qk_project_on_hip(z):
-            # Inference at few tokens: value and variance columns as one hipBLASLt
-            # product, k and q with their norm and clip as one HIP kernel (a 2S-row
-            # tail would otherwise set hipBLASLt's tile for the whole product).
+            # Inference at few tokens: value and variance columns as one product, k and
+            # q with their norm and clip as one HIP kernel.
             from kla.ops.hip.linear import linear_f32, linear_f32_ok
             from kla.ops.hip.sensors import qk_project_hip
 
