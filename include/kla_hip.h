@@ -629,8 +629,10 @@ int kla_rows_linear_conv_fwd(const float *x, int64_t ldx, const float *w, int64_
  * runs on the fp16 matrix cores over operands split into two fp16 planes (scaled
  * per row), summed in fp32: no larger an error than an fp32 product's, at about
  * 2.5 times its rate. Rows holding an infinity or a NaN give what fp32 arithmetic
- * gives. No gradient; deterministic (fixed-order sums). workspace: 256-byte
- * aligned, at least kla_linear_f32_workspace_bytes, contents not kept.
+ * gives. No gradient; deterministic (fixed-order sums). y may be res itself, with
+ * the same row stride (an add in place); otherwise it overlaps no operand.
+ * workspace: 256-byte aligned, at least kla_linear_f32_workspace_bytes, contents
+ * not kept.
  * Replaces, in inference over a sequence, the nn.Linear calls of KLALayer
  * (reference src/kla/layers/kla_layer.py:61, :88, :127), MLP and RMSNorm
  * (src/kla/layers/common.py:45-55, :99-123), the block's residual adds

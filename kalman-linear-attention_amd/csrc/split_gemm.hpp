@@ -480,6 +480,7 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   const bool vec_res = EPI == kGemmResidual && p.ldres % 4 == 0 && reinterpret_cast<uintptr_t>(p.res) % 16 == 0;
   static_assert(EPI != kGemmSwiglu || FN % 2 == 0, "a wave holds a gate block with its up block");
   constexpr int STEP = EPI == kGemmSwiglu ? 2 : 1;
+  constexpr int kMarkedW = kSplitMarked - 2 * kSplitExp;    // a marked row in s_we
 #pragma unroll
   for (int a = 0; a < FN; a += STEP)
 #pragma unroll
@@ -506,6 +507,16 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
                           swiglu_value(v.z, ldexpf(u[4 * g + 2], ex + eu.z) + bu.z),
                           swiglu_value(v.w, ldexpf(u[4 * g + 3], ex + eu.w) + bu.w));
         }
+        // Outputs of marked rows are left to split_exact_outputs, which reads res (y
+        // may be res itself).
+        bool mine[4] = {ex != kSplitMarked && en.x != kMarkedW, ex != kSplitMarked && en.y != kMarkedW,
+                        ex != kSplitMarked && en.z != kMarkedW, ex != kSplitMarked && en.w != kMarkedW};
+        if constexpr (EPI == kGemmSwiglu) {
+          const int4 eu = *reinterpret_cast<const int4 *>(s_we + nl + kSplitRows);
+          mine[0] = mine[0] && eu.x != kMarkedW, mine[1] = mine[1] && eu.y != kMarkedW;
+          mine[2] = mine[2] && eu.z != kMarkedW, mine[3] = mine[3] && eu.w != kMarkedW;
+        }
+        const bool all = mine[0] && mine[1] && mine[2] && mine[3];
         if (t < p.rows) {
           float *out = p.y + t * p.ldy + n;
           if constexpr (EPI == kGemmResidual) {
@@ -520,19 +531,18 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
               if (n + 3 < p.n) v.w = res[3] + v.w;
             }
           }
-          if (vec && n + 4 <= p.n) {
+          if (vec && all && n + 4 <= p.n) {
             *reinterpret_cast<float4 *>(out) = v;
           } else {
-            if (n < p.n) out[0] = v.x;
-            if (n + 1 < p.n) out[1] = v.y;
-            if (n + 2 < p.n) out[2] = v.z;
-            if (n + 3 < p.n) out[3] = v.w;
+            if (mine[0] && n < p.n) out[0] = v.x;
+            if (mine[1] && n + 1 < p.n) out[1] = v.y;
+            if (mine[2] && n + 2 < p.n) out[2] = v.z;
+            if (mine[3] && n + 3 < p.n) out[3] = v.w;
           }
         }
       }
     }
-  // Marked rows or columns: their outputs once more, from the operands. (The
-  // barrier orders the two stores.)
+  // The outputs of marked rows or columns, from the operands.
   if (__syncthreads_or(marked)) split_exact_outputs<EPI, TN, TT>(p, n0, t0);
 }
 

@@ -2,10 +2,13 @@
 edges, strided and unaligned operands, rows fp16 could not hold, rows with an
 infinity or a NaN, and which calls of a module take it."""
 
+import ctypes
+
 import pytest
 import torch
 import torch.nn.functional as F
 
+from kla.ops.hip import _lib
 from kla.ops.hip import linear as lin
 
 pytestmark = pytest.mark.gpu
@@ -213,6 +216,36 @@ def test_folded_options_with_infinities_and_nans(cuda):
         for r in (3, 64):
             assert torch.equal(torch.isfinite(got[r]), torch.isfinite(want[r].float())), (opts.keys(), r)
         assert not torch.isfinite(got[rows, 9]).all()
+
+
+def _in_place(x, w, bias, res):
+    """kla_linear_f32_fwd with the residual add in place (y is res): the returned tensor."""
+    lib, p = _lib.lib(), _lib.ptr
+    y, (rows, k), n = res.clone(), x.shape, w.shape[0]
+    nbytes = lib.kla_linear_f32_workspace_bytes(rows, n, k, _lib.KLA_ROWS_RESIDUAL)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    args = _lib.LinearF32(epilogue=_lib.KLA_ROWS_RESIDUAL, x=p(x), w=p(w), bias=p(bias), res=p(y), y=p(y), ldx=k, ldw=k,
+                          ldres=n, ldy=n, rows=rows, n=n, k=k)
+    _lib.check("kla_linear_f32_fwd", lib.kla_linear_f32_fwd(ctypes.byref(args), p(ws), nbytes, _lib.stream(x.device)))
+    return y
+
+
+def test_residual_in_place(cuda):
+    """y is res: the same values as out of place, rows and columns that hold an infinity or
+    a NaN included (their outputs read res where no earlier store has been)."""
+    g = torch.Generator(device=cuda).manual_seed(9)
+    x, w, bias, res = (torch.randn(*s, device=cuda, generator=g) for s in ((150, 70), (133, 70), (133,), (150, 133)))
+    assert torch.equal(_in_place(x, w, bias, res), lin.linear_f32(x, w, bias, residual=res))
+    x[3, 4], x[64, 0], w[9, 2], w[128, 1] = float("inf"), float("nan"), -float("inf"), float("nan")
+    x[:, 2] = x[:, 2].abs()     # a finite value against W's infinity leaves no 0 * inf
+    got, want = _in_place(x, w, bias, res), lin.linear_f32(x, w, bias, residual=res)
+    assert torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+    assert torch.isfinite(want[5, :9]).all() and not torch.isfinite(want[3]).any() and torch.isnan(want[:, 128]).all()
+    w[9, 2], w[9, 3] = 0.0, float("inf")
+    x[:, 3] = 0.0
+    x[7, 3] = 1.0
+    got, want = _in_place(x, w, bias, res), lin.linear_f32(x, w, bias, residual=res)
+    assert torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)) and got[7, 9] == float("inf")
 
 
 def test_blocks_fold_their_norms_and_residuals(cuda, monkeypatch):
