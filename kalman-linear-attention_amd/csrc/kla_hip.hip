@@ -1741,8 +1741,8 @@ int linear_f32(const char *fn, const kla_linear_f32_args &a, void *workspace, si
   if (misaligned_bytes(workspace, 256)) return fail(KLA_ERR_WORKSPACE, "%s: workspace not 256-byte aligned", fn);
 
   SplitGemmParams g{};
-  g.w = a.w, g.bias = a.bias, g.res = a.res, g.y = a.y;
-  g.ldw = a.ldw, g.ldres = a.ldres, g.ldy = a.ldy;
+  g.x = a.x, g.w = a.w, g.bias = a.bias, g.norm_w = a.norm_w, g.eps = a.eps, g.res = a.res, g.y = a.y;
+  g.ldx = a.ldx, g.ldw = a.ldw, g.ldres = a.ldres, g.ldy = a.ldy;
   g.rows = a.rows, g.n = a.n, g.k = a.k, g.glu_off = a.glu_off;
   g.chunks = (a.k + kSplitK - 1) / kSplitK;
   g.xblocks = (a.rows + kSplitRows - 1) / kSplitRows;

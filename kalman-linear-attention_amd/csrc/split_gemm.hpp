@@ -16,9 +16,8 @@
 // magnitude into [2^14, 2^15); the scales go back in with one ldexp per output.
 // Entries more than 2^17 below their row's largest lose low bits of lo to
 // fp16's smallest spacing, at most 2^-39 of the row's largest value each. A row with an
-// infinity or a NaN is marked instead and its planes hold the two halves of the
-// fp32 words, from which every output it touches is summed in plain fp32
-// (split_exact_outputs).
+// infinity or a NaN is marked instead: every output it touches is summed in plain
+// fp32 from the operands (split_exact_block).
 //
 // What surrounds a product in a block is folded in: before it the RMSNorm of x's
 // rows (formed as the rows are split, never stored in fp32: 13.1 us at 4096 x 512
@@ -38,6 +37,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "causal_conv.hpp"
 #include "scan_ops.hpp"
@@ -199,14 +200,9 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float u = norm ? (v[8 * f + i] * scale) * w[8 * f + i] : v[8 * f + i];
-        const float s = ldexpf(u, shift);
+        const float s = marked ? 0.0f : ldexpf(u, shift);
         hi[i] = static_cast<_Float16>(s);
         lo[i] = static_cast<_Float16>(s - static_cast<float>(hi[i]));
-        if (marked) {
-          const uint32_t b = __float_as_uint(u);
-          hi[i] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(b >> 16));
-          lo[i] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(b));
-        }
       }
       *reinterpret_cast<f16x8_t *>(out + (2 * f) * 512) = hi;
       *reinterpret_cast<f16x8_t *>(out + (2 * f + 1) * 512) = lo;
@@ -231,60 +227,109 @@ enum SplitEpilogue { kGemmPlain = 0, kGemmResidual = 1, kGemmSwiglu = 2 };
 struct SplitGemmParams {
   const _Float16 *xs, *ws;       // split planes of x (tokens) and W (features)
   const int *xe, *we;            // row exponents
-  const float *w, *bias;         // W itself (row stride ldw; marked rows), bias by W's rows or NULL
+  const float *x, *norm_w;       // x itself (row stride ldx) and the RMSNorm's weight or NULL: split_exact_block
+  const float *w, *bias;         // W itself (row stride ldw: split_exact_block), bias by W's rows or NULL
   const float *res;              // [rows, n], row stride ldres (kGemmResidual)
   float *y;                      // [rows, n], row stride ldy
-  int64_t ldw, ldres, ldy, rows, n, k, chunks;
+  int64_t ldx, ldw, ldres, ldy, rows, n, k, chunks;
+  float eps;
   int64_t glu_off;               // kGemmSwiglu: W row of the up half of output column 0
   int64_t xblocks, wblocks;      // 32-row blocks of x and of W
   int64_t tiles_n, tiles_t;      // output tiles over W's blocks and tokens
 };
 
-// Element (row of the split operand, k) in fp32: as it was in a marked row, else the
-// sum of its planes with the row's scale.
-__device__ __forceinline__ float split_element(const _Float16 *planes, int64_t chunks, int e, int64_t row, int64_t k) {
-  const int64_t at = ((row / kSplitRows) * chunks + k / kSplitK) * kSplitChunk + 2 * ((k % 16) / 8) * 512 +
-                     ((k % kSplitK) / 16 * 32 + row % kSplitRows) * 8 + k % 8;
-  const _Float16 hi = planes[at], lo = planes[at + 512];
-  if (e == kSplitMarked)
-    return __uint_as_float(static_cast<uint32_t>(__builtin_bit_cast(uint16_t, hi)) << 16 |
-                           __builtin_bit_cast(uint16_t, lo));
-  return ldexpf(static_cast<float>(hi) + static_cast<float>(lo), e - kSplitExp);
-}
-
 // silu(g) u, as the MLP forms it.
 __device__ __forceinline__ float swiglu_value(float g, float u) { return activation(kActSilu, g) * u; }
 
-// Outputs of the tile that a marked row touches, one at a time in plain fp32: n0 and
-// TN count W's blocks' rows (two a column with SwiGLU).
-template <int EPI, int TN, int TT>
-__device__ __forceinline__ void split_exact_outputs(const SplitGemmParams &p, int64_t n0, int64_t t0) {
-  auto dot = [&](int64_t t, int64_t w_row) {
-    const int xe = p.xe[t];
-    const float *w = p.w + w_row * p.ldw;
-    float s = 0.0f;
-    for (int64_t i = 0; i < p.k; ++i) s = fmaf(split_element(p.xs, p.chunks, xe, t, i), w[i], s);
-    return s;
-  };
-  constexpr int COLS = EPI == kGemmSwiglu ? TN / 2 : TN;
-  for (int e = static_cast<int>(threadIdx.x); e < COLS * TT; e += static_cast<int>(blockDim.x)) {
-    const int64_t t = t0 + e / COLS;
-    const int64_t n = (EPI == kGemmSwiglu ? n0 / 2 : n0) + e % COLS;
-    if (n >= p.n || t >= p.rows) continue;
-    const int64_t wr = EPI == kGemmSwiglu ? (n / 32) * 64 + n % 32 : n;
-    const bool m = p.xe[t] == kSplitMarked || p.we[wr] == kSplitMarked;
-    float v;
-    if constexpr (EPI == kGemmSwiglu) {
-      if (!m && p.we[wr + 32] != kSplitMarked) continue;
-      const float g = dot(t, n) + (p.bias ? p.bias[n] : 0.0f);
-      v = swiglu_value(g, dot(t, p.glu_off + n) + (p.bias ? p.bias[p.glu_off + n] : 0.0f));
+// The kernel's arguments, read where they are used (and not before).
+typedef const __attribute__((address_space(4))) SplitGemmParams *SplitGemmArgs;
+
+// The fp32 products of four rows of W from w0 and eight of x from t0 (rows past the
+// last of either read the last again), formed by one wave from the operands as they
+// are: lane l returns that of W row w0 + l / 16 and x row t0 + l / 2 % 8. A lane sums
+// k = 256 i + 4 l + 0..3 by fma and the lanes' sums are added along a fixed tree, so
+// a value depends on its two rows alone. Bound by the operand rows' way from L2.
+template <bool NORM>
+__device__ __forceinline__ float split_exact_block(SplitGemmArgs p, int64_t t0, int64_t w0, int64_t w_last) {
+  constexpr int64_t kStep = 4 * kWave;
+  const int lane = static_cast<int>(threadIdx.x) % kWave;
+  const int64_t k = p->k;
+  const float *x[8], *w[4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] = p->x + (t0 + i < p->rows ? t0 + i : p->rows - 1) * p->ldx;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = p->w + (w0 + i < w_last ? w0 + i : w_last) * p->ldw;
+  // Elements 4 l + 0..3 of the 256 from `at`, of which n are left unless FULL (0 past
+  // the end).
+  auto load4 = [&](const float *at, int64_t n, auto full) __attribute__((always_inline)) {
+    f32x4_any_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+    const float *mine = reinterpret_cast<const float *>(reinterpret_cast<const char *>(at) + 16u * lane);
+    if (decltype(full)::value || 4 * lane + 4 <= n) {
+      v = *reinterpret_cast<const f32x4_any_t *>(mine);
     } else {
-      if (!m) continue;
-      v = dot(t, n) + (p.bias ? p.bias[n] : 0.0f);
-      if constexpr (EPI == kGemmResidual) v = p.res[t * p.ldres + n] + v;
+      if (4 * lane < n) v.x = mine[0];
+      if (4 * lane + 1 < n) v.y = mine[1];
+      if (4 * lane + 2 < n) v.z = mine[2];
     }
-    p.y[t * p.ldy + n] = v;
+    return v;
+  };
+  float scale[NORM ? 8 : 1];
+  if constexpr (NORM) {
+    float ss[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss[i] = 0.0f;
+    auto add = [&](int64_t k0, auto full) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const f32x4_any_t v = load4(x[i] + k0, k - k0, full);
+        ss[i] = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss[i]))));
+      }
+    };
+    int64_t k0 = 0;
+#pragma unroll 1
+    for (; k0 + kStep <= k; k0 += kStep) add(k0, std::true_type{});
+    if (k0 < k) add(k0, std::false_type{});
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int h = kWave / 2; h; h /= 2) ss[i] += __shfl_xor(ss[i], h);
+      scale[i] = rsqrtf(ss[i] / static_cast<float>(k) + p->eps);
+    }
   }
+  float s[32];    // [W row][x row]
+#pragma unroll
+  for (int i = 0; i < 32; ++i) s[i] = 0.0f;
+  auto add = [&](int64_t k0, auto full) __attribute__((always_inline)) {
+    f32x4_any_t xv[8], wv[4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) xv[i] = load4(x[i] + k0, k - k0, full);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wv[i] = load4(w[i] + k0, k - k0, full);
+    if constexpr (NORM) {
+      const f32x4_any_t nw = load4(p->norm_w + k0, k - k0, full);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) xv[i] = (xv[i] * scale[i]) * nw;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int i = 0; i < 32; ++i) s[i] = fmaf(xv[i % 8][c], wv[i / 8][c], s[i]);
+  };
+  int64_t k0 = 0;
+#pragma unroll 1
+  for (; k0 + kStep <= k; k0 += kStep) add(k0, std::true_type{});
+  if (k0 < k) add(k0, std::false_type{});
+  // Halve the sums a lane holds at each bit of its index: lane l is left with sum l / 2.
+#pragma unroll
+  for (int h = 16; h; h /= 2) {
+    const bool up = lane & (2 * h);
+#pragma unroll
+    for (int i = 0; i < h; ++i) {
+      const float keep = up ? s[i + h] : s[i], give = up ? s[i] : s[i + h];
+      s[i] = keep + __shfl_xor(give, 2 * h);
+    }
+  }
+  return s[0] + __shfl_xor(s[0], 1);
 }
 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
@@ -344,6 +389,10 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   __shared__ __align__(16) int s_we[TN];
   __shared__ __align__(16) float s_bias[TN];
   __shared__ int s_xe[TT];
+  // By wave, block of its features, feature octet and token block: the lanes whose
+  // outputs split_exact_block forms.
+  constexpr int STEP = EPI == kGemmSwiglu ? 2 : 1;
+  __shared__ uint64_t s_exact[NW][FN / STEP * 4 * FT];
 
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid % kWave;
@@ -476,10 +525,11 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   // No load into this workgroup's LDS may outlive it.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
+  const bool exact = __syncthreads_or(marked);    // any in the tile
+
   const bool vec = p.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(p.y) % 16 == 0;
   const bool vec_res = EPI == kGemmResidual && p.ldres % 4 == 0 && reinterpret_cast<uintptr_t>(p.res) % 16 == 0;
   static_assert(EPI != kGemmSwiglu || FN % 2 == 0, "a wave holds a gate block with its up block");
-  constexpr int STEP = EPI == kGemmSwiglu ? 2 : 1;
   constexpr int kMarkedW = kSplitMarked - 2 * kSplitExp;    // a marked row in s_we
 #pragma unroll
   for (int a = 0; a < FN; a += STEP)
@@ -507,17 +557,17 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
                           swiglu_value(v.z, ldexpf(u[4 * g + 2], ex + eu.z) + bu.z),
                           swiglu_value(v.w, ldexpf(u[4 * g + 3], ex + eu.w) + bu.w));
         }
-        // Outputs of marked rows are left to split_exact_outputs, which reads res (y
-        // may be res itself).
-        bool mine[4] = {ex != kSplitMarked && en.x != kMarkedW, ex != kSplitMarked && en.y != kMarkedW,
-                        ex != kSplitMarked && en.z != kMarkedW, ex != kSplitMarked && en.w != kMarkedW};
-        if constexpr (EPI == kGemmSwiglu) {
-          const int4 eu = *reinterpret_cast<const int4 *>(s_we + nl + kSplitRows);
-          mine[0] = mine[0] && eu.x != kMarkedW, mine[1] = mine[1] && eu.y != kMarkedW;
-          mine[2] = mine[2] && eu.z != kMarkedW, mine[3] = mine[3] && eu.w != kMarkedW;
+        bool skip = false;
+        if (exact) {
+          skip = ex == kSplitMarked || en.x == kMarkedW || en.y == kMarkedW || en.z == kMarkedW || en.w == kMarkedW;
+          if constexpr (EPI == kGemmSwiglu) {
+            const int4 eu = *reinterpret_cast<const int4 *>(s_we + nl + kSplitRows);
+            skip = skip || eu.x == kMarkedW || eu.y == kMarkedW || eu.z == kMarkedW || eu.w == kMarkedW;
+          }
+          const uint64_t lanes = __ballot(skip && t < p.rows && n < p.n);
+          if (lane == 0) s_exact[wave][(a / STEP * 4 + g) * FT + b] = lanes;
         }
-        const bool all = mine[0] && mine[1] && mine[2] && mine[3];
-        if (t < p.rows) {
+        if (t < p.rows && !skip) {
           float *out = p.y + t * p.ldy + n;
           if constexpr (EPI == kGemmResidual) {
             const float *res = p.res + t * p.ldres + n;
@@ -531,19 +581,49 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
               if (n + 3 < p.n) v.w = res[3] + v.w;
             }
           }
-          if (vec && all && n + 4 <= p.n) {
+          if (vec && n + 4 <= p.n) {
             *reinterpret_cast<float4 *>(out) = v;
           } else {
-            if (mine[0] && n < p.n) out[0] = v.x;
-            if (mine[1] && n + 1 < p.n) out[1] = v.y;
-            if (mine[2] && n + 2 < p.n) out[2] = v.z;
-            if (mine[3] && n + 3 < p.n) out[3] = v.w;
+            if (n < p.n) out[0] = v.x;
+            if (n + 1 < p.n) out[1] = v.y;
+            if (n + 2 < p.n) out[2] = v.z;
+            if (n + 3 < p.n) out[3] = v.w;
           }
         }
       }
     }
-  // The outputs of marked rows or columns, from the operands.
-  if (__syncthreads_or(marked)) split_exact_outputs<EPI, TN, TT>(p, n0, t0);
+  // What was left out: the outputs of marked rows or columns, 4 x 8 at a time, each
+  // read of res and store of y here and nowhere else (y may be res itself).
+  if (!exact) return;
+  __syncthreads();
+  SplitGemmArgs args = (SplitGemmArgs)__builtin_amdgcn_kernarg_segment_ptr();
+#ifdef __OPTIMIZE__
+  asm volatile("" : "+s"(args));    // (nothing of this is to be ready, or held, any earlier)
+#endif
+  auto dots = [&](int64_t t, int64_t w, int64_t w_last) __attribute__((always_inline)) {
+    return args->norm_w ? split_exact_block<true>(args, t, w, w_last) : split_exact_block<false>(args, t, w, w_last);
+  };
+#pragma unroll 1
+  for (int i = 0; i < FN / STEP * 4 * FT * 8; ++i) {    // a half of the lanes (four features), eight tokens each
+    const int q = i % 8, b = i / 8 % FT, g = i / 8 / FT % 4, a = i / 8 / FT / 4;
+    const uint32_t part = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s_exact[wave][i / 8] >> (8 * q)) & 0xff);
+    if (!part) continue;
+    const int64_t tq = t0 + (wt * FT + b) * kSplitRows + q % 4 * 8;
+    const int64_t nq = n0 / STEP + (wn * FN / STEP + a) * kSplitRows + 8 * g + q / 4 * 4;
+    const int64_t n = nq + lane / 16, t = tq + lane / 2 % 8, rows_n = args->n;
+    const bool in = n < rows_n && t < args->rows;
+    const float *bias = args->bias;
+    float v = dots(tq, nq, rows_n - 1) + (bias && in ? bias[n] : 0.0f);
+    if constexpr (EPI == kGemmSwiglu) {
+      const int64_t off = args->glu_off;
+      const float u = dots(tq, off + nq, off + rows_n - 1);
+      v = swiglu_value(v, u + (bias && in ? bias[off + n] : 0.0f));
+    }
+    if (in && lane % 2 == 0 && (part >> (lane / 2 % 8) & 1)) {
+      if constexpr (EPI == kGemmResidual) v = args->res[t * args->ldres + n] + v;
+      args->y[t * args->ldy + n] = v;
+    }
+  }
 }
 
 }  // namespace kla

@@ -218,6 +218,31 @@ def test_folded_options_with_infinities_and_nans(cuda):
         assert not torch.isfinite(got[rows, 9]).all()
 
 
+def _best_ms(f):
+    times = []
+    for _ in range(3):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        f()
+        b.record()
+        b.synchronize()
+        times.append(a.elapsed_time(b))
+    return min(times)
+
+
+def test_a_batch_of_nans_stays_near_the_library(cuda):
+    """Every output formed in plain fp32: a few times the library product (3 to 5 measured),
+    not the hundreds of a serial sum a lane."""
+    g = torch.Generator(device=cuda).manual_seed(10)
+    x, w = (torch.randn(2048, 1024, device=cuda, generator=g) for _ in range(2))
+    x[:, 5] = float("nan")
+    assert torch.isnan(lin.linear_f32(x, w)).all()
+    F.linear(x, w)
+    got, library = _best_ms(lambda: lin.linear_f32(x, w)), _best_ms(lambda: F.linear(x, w))
+    print(f"[linear_f32] NaN rows {got:.3f} ms, library {library:.3f} ms", flush=True)
+    assert got < 20 * library + 0.2
+
+
 def _in_place(x, w, bias, res):
     """kla_linear_f32_fwd with the residual add in place (y is res): the returned tensor."""
     lib, p = _lib.lib(), _lib.ptr
