@@ -1665,7 +1665,7 @@ int rows_linear_launch(const char *fn, int epi, RowsLinearParams &p, hipStream_t
 }
 
 // The split fp32 product (split_gemm.hpp). Workspace: the planes of x and of W (two
-// sets of 32-row blocks with SwiGLU), then their row exponents.
+// sets of 32-row blocks with SwiGLU), then their row words.
 int64_t linear_f32_wblocks(int64_t n, bool swiglu) {
   const int64_t b = sadd(n, kSplitRows - 1) / kSplitRows;
   return swiglu ? smul(2, b) : b;
@@ -1752,8 +1752,8 @@ int linear_f32(const char *fn, const kla_linear_f32_args &a, void *workspace, si
     return fail(KLA_ERR_INVALID_ARG, "%s: grid too large", fn);
   _Float16 *xs = static_cast<_Float16 *>(workspace);
   _Float16 *ws = xs + g.xblocks * g.chunks * kSplitChunk;
-  int *xe = reinterpret_cast<int *>(ws + g.wblocks * g.chunks * kSplitChunk);
-  int *we = xe + g.xblocks * kSplitRows;
+  uint32_t *xe = reinterpret_cast<uint32_t *>(ws + g.wblocks * g.chunks * kSplitChunk);
+  uint32_t *we = xe + g.xblocks * kSplitRows;
   g.xs = xs, g.ws = ws, g.xe = xe, g.we = we;
 
   SplitParams sp{};
@@ -1761,6 +1761,7 @@ int linear_f32(const char *fn, const kla_linear_f32_args &a, void *workspace, si
   sp.op[1] = SplitOperand{a.w, a.ldw, a.n, ws, we, g.wblocks};
   sp.k = a.k;
   sp.chunks = g.chunks;
+  sp.share = static_cast<float>(kSplitShare) / static_cast<float>(a.k);
   if (swiglu) sp.glu_off = a.glu_off, sp.glu_rows = a.n;
   sp.norm_w = a.norm_w, sp.eps = a.eps;
   if (a.norm_w)

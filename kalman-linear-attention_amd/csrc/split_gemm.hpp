@@ -14,10 +14,18 @@
 //
 // Each row of x and of W is scaled by the power of two that brings its largest
 // magnitude into [2^14, 2^15); the scales go back in with one ldexp per output.
-// Entries more than 2^17 below their row's largest lose low bits of lo to
-// fp16's smallest spacing, at most 2^-39 of the row's largest value each. A row with an
-// infinity or a NaN is marked instead: every output it touches is summed in plain
-// fp32 from the operands (split_exact_block).
+// Entries more than 2^16 below their row's largest lose low bits of lo to fp16's
+// smallest spacing, up to 2^-39 of the row's largest value each: nothing beside the
+// row's other terms, but all there is where those are multiplied by zeros (a feature
+// of 1e9 that the weights ignore). So the row split counts c, the entries that lose,
+// and h, those below 2^6 at the row's scale. The other operand lies below 2^15, so an
+// output is off by (c_x + c_w) 2^-10 of its scale at most. At least k - h_x - h_w of its
+// terms are 2^12 and more, so their fp32 rounding alone comes to 2^-12 of that number:
+// where h + 4 c of the two rows is k or less, no fp32 sum promises more. Rows of
+// dense weights and activations have 0.01 to 0.3 k of it, ReLU's 0.55 k. Where it is
+// more, an output that the loss could move by more than 2^-23 of the sum the matrix
+// cores gave is summed in plain fp32 from the operands (split_exact_block), as is
+// every output of a row with an infinity or a NaN.
 //
 // What surrounds a product in a block is folded in: before it the RMSNorm of x's
 // rows (formed as the rows are split, never stored in fp32: 13.1 us at 4096 x 512
@@ -52,13 +60,22 @@ constexpr int kSplitRows = 32;                       // rows of a fragment
 constexpr int kSplitK = 32;                          // k of a pair of fragments (a chunk)
 constexpr int kSplitChunk = kSplitRows * kSplitK * 2;   // fp16 of a chunk: 2 k halves x 2 planes x 512
 constexpr int kSplitExp = 14;                        // scaled rows lie in [2^14, 2^15)
-constexpr int kSplitMarked = 1 << 20;                // row exponent of a row with an infinity or NaN
+// A row's word. Its exponent + kSplitBias; kSplitZero for a row of zeros; 2^13 c as the
+// exponent of a float, rounded up (infinite for a row with an infinity or a NaN); and
+// h + 4 c in units of k / kSplitShare, rounded up.
+constexpr int kSplitBias = 160, kSplitShare = 8192;
+constexpr uint32_t kSplitZero = 1u << 23;
+constexpr uint32_t kSplitNoRow = kSplitZero | kSplitBias << 14;
+
+__device__ __forceinline__ int split_exp(uint32_t word) { return static_cast<int>(word >> 14 & 0x1ff) - kSplitBias; }
+__device__ __forceinline__ float split_lost(uint32_t word) { return __uint_as_float(word >> 24 << 23); }
+__device__ __forceinline__ int split_share(uint32_t word) { return static_cast<int>(word & 0x3fff); }
 
 struct SplitOperand {
   const float *src;    // [rows, k], row stride ld
   int64_t ld, rows;
   _Float16 *dst;       // [blocks][chunks][2 k halves][2 planes][64 lanes][8]
-  int *exps;           // [blocks * 32]: s = src * 2^(kSplitExp - exp), or kSplitMarked
+  uint32_t *words;     // [blocks * 32]: by row, s = src * 2^(kSplitExp - split_exp(word))
   int64_t blocks;      // 32-row blocks
 };
 
@@ -66,6 +83,7 @@ struct SplitParams {
   SplitOperand op[2];  // x, W
   int64_t k;
   int64_t chunks;      // ceil(k / 32)
+  float share;         // kSplitShare / k
   // NORM: x -> (x * rsqrt(mean(x^2) + eps)) * norm_w
   const float *norm_w;
   float eps;
@@ -112,6 +130,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
   constexpr int NWV = kSplitThreads / kWave;
   __shared__ uint32_t s_max[NWV][kSplitRows];
   __shared__ float s_sum[NORM ? NWV : 1][kSplitRows];
+  __shared__ int s_count[2][NWV][kSplitRows];
   const bool second = static_cast<int64_t>(blockIdx.x) >= p.op[0].blocks;
   const SplitOperand &op = p.op[second ? 1 : 0];
   const int64_t blk = static_cast<int64_t>(blockIdx.x) - (second ? p.op[0].blocks : 0);
@@ -187,8 +206,8 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
   // The exponent of the row's largest magnitude (that of 1 for a row of zeros).
   int ex = 0;
   if (!marked && bound != 0.0f) ex = __builtin_amdgcn_frexp_expf(bound) - 1;
-  if (wave == 0 && half == 0) op.exps[blk * kSplitRows + r] = marked ? kSplitMarked : ex;
 
+  int lossy = 0, small = 0;    // this lane's part of c and h
   const int shift = kSplitExp - ex;
   auto put = [&](const float (&v)[16], int64_t ch) {
     _Float16 *out = op.dst + (blk * p.chunks + ch) * kSplitChunk + lane * 8;
@@ -200,9 +219,11 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float u = norm ? (v[8 * f + i] * scale) * w[8 * f + i] : v[8 * f + i];
-        const float s = marked ? 0.0f : ldexpf(u, shift);
+        const float s = ldexpf(u, shift);
         hi[i] = static_cast<_Float16>(s);
         lo[i] = static_cast<_Float16>(s - static_cast<float>(hi[i]));
+        small += fabsf(s) < 0x1p6f;
+        lossy += fabsf(s) < 0x1p-2f && u != 0.0f;    // (from 2^-2 on lo is good to 2^-23 of s)
       }
       *reinterpret_cast<f16x8_t *>(out + (2 * f) * 512) = hi;
       *reinterpret_cast<f16x8_t *>(out + (2 * f + 1) * 512) = lo;
@@ -220,13 +241,34 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
       put(x[0], ch);
     }
   }
+  lossy += __shfl_xor(lossy, 32);
+  small += __shfl_xor(small, 32);
+  if (half == 0) s_count[0][wave][r] = lossy, s_count[1][wave][r] = small;
+  __syncthreads();
+  if (wave == 0 && half == 0) {
+    float c = 0.0f, h = static_cast<float>(p.k - p.chunks * kSplitK);    // (less the zeros past the rows' end)
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) {
+      c += static_cast<float>(s_count[0][w][r]);
+      h += static_cast<float>(s_count[1][w][r]);
+    }
+    uint32_t word = static_cast<uint32_t>(ex + kSplitBias) << 14;
+    if (marked) {
+      word |= 0xffu << 24 | 0x3fff;
+    } else if (in) {
+      const float share = ceilf((h + 4.0f * c) * p.share);
+      const uint32_t lost = __float_as_uint(c * 0x1p13f);
+      word |= (lost + 0x7fffffu) >> 23 << 24 | static_cast<uint32_t>(fminf(share, 0x3fff));
+    }
+    op.words[blk * kSplitRows + r] = word | (!marked && bound == 0.0f ? kSplitZero : 0u);
+  }
 }
 
 enum SplitEpilogue { kGemmPlain = 0, kGemmResidual = 1, kGemmSwiglu = 2 };
 
 struct SplitGemmParams {
   const _Float16 *xs, *ws;       // split planes of x (tokens) and W (features)
-  const int *xe, *we;            // row exponents
+  const uint32_t *xe, *we;       // row words
   const float *x, *norm_w;       // x itself (row stride ldx) and the RMSNorm's weight or NULL: split_exact_block
   const float *w, *bias;         // W itself (row stride ldw: split_exact_block), bias by W's rows or NULL
   const float *res;              // [rows, n], row stride ldres (kGemmResidual)
@@ -389,6 +431,7 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   __shared__ __align__(16) int s_we[TN];
   __shared__ __align__(16) float s_bias[TN];
   __shared__ int s_xe[TT];
+  __shared__ int s_doubt[NW];    // by wave, of the rows whose words it read
   // By wave, block of its features, feature octet and token block: the lanes whose
   // outputs split_exact_block forms.
   constexpr int STEP = EPI == kGemmSwiglu ? 2 : 1;
@@ -479,23 +522,27 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   load(s_0, 0);
   if constexpr (ST > 2) load(s_1, chunks > 1 ? 1 : chunks - 1);
   if constexpr (ST > 3) load(s_2, chunks > 2 ? 2 : chunks - 1);
-  // The tile's row exponents and bias, for the epilogue (they arrive with the first chunks).
+  // The tile's row words and bias, for the epilogue (they arrive with the first chunks).
   const int64_t n0 = tn * TN, t0 = tt * TT;
-  bool marked = false;
+  // Bit 0: a row of the tile lost something; bit 1: one takes more than its part of h +
+  // 4 c <= k (a quarter for W, whose entries are of a size; three quarters for x).
+  int doubt = 0;
   for (int i = tid; i < TN + TT; i += NW * kWave) {
     const bool isn = i < TN;
     const int64_t r = isn ? n0 + i : t0 + (i - TN);
-    const int e = r < (isn ? p.wblocks : p.xblocks) * kSplitRows ? (isn ? p.we : p.xe)[r] : 0;
-    marked = marked || e == kSplitMarked;
+    const uint32_t e = r < (isn ? p.wblocks : p.xblocks) * kSplitRows ? (isn ? p.we : p.xe)[r] : kSplitNoRow;
+    doubt |= (split_lost(e) != 0.0f) | (split_share(e) > (isn ? kSplitShare / 4 : kSplitShare / 4 * 3)) << 1;
     if (isn) {
       int64_t col = r;
       if constexpr (EPI == kGemmSwiglu) col = (r / 64) * 32 + r % 32;
-      s_we[i] = e - 2 * kSplitExp;
+      s_we[i] = split_exp(e) - 2 * kSplitExp;
       s_bias[i] = p.bias && col < p.n ? p.bias[EPI == kGemmSwiglu && r / 32 % 2 ? p.glu_off + col : col] : 0.0f;
     } else {
-      s_xe[i - TN] = e;
+      s_xe[i - TN] = split_exp(e);
     }
   }
+  doubt = (__any(doubt & 1) ? 1 : 0) | (__any(doubt & 2) ? 2 : 0);
+  if (lane == 0) s_doubt[wave] = doubt;
   int c = 0;
   if constexpr (ST == 2) {
     for (; c + 2 <= chunks; c += 2) {
@@ -525,12 +572,30 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   // No load into this workgroup's LDS may outlive it.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  const bool exact = __syncthreads_or(marked);    // any in the tile
+  // (A step's barrier lies between.) Then, for the sums of token t against the four rows
+  // of W from wr: whether one has to be formed again, by what their rows lost (nothing
+  // against a row of zeros; an infinity against one is, as NaN).
+  doubt = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) doubt |= s_doubt[w];
+  const bool exact = doubt == 3;
+  auto off = [&](const f32x16_t &acc, int g, int64_t t, int64_t wr) __attribute__((always_inline)) {
+    const uint32_t xw = p.xe[t];
+    const uint4 w4 = *reinterpret_cast<const uint4 *>(p.we + wr);
+    const uint32_t ww[4] = {w4.x, w4.y, w4.z, w4.w};
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float lost = split_lost(xw) * (ww[j] & kSplitZero ? 0.0f : 1.0f) +
+                         split_lost(ww[j]) * (xw & kSplitZero ? 0.0f : 1.0f);
+      any = any || (split_share(xw) + split_share(ww[j]) > kSplitShare && !(fabsf(acc[4 * g + j]) >= lost));
+    }
+    return any;
+  };
 
   const bool vec = p.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(p.y) % 16 == 0;
   const bool vec_res = EPI == kGemmResidual && p.ldres % 4 == 0 && reinterpret_cast<uintptr_t>(p.res) % 16 == 0;
   static_assert(EPI != kGemmSwiglu || FN % 2 == 0, "a wave holds a gate block with its up block");
-  constexpr int kMarkedW = kSplitMarked - 2 * kSplitExp;    // a marked row in s_we
 #pragma unroll
   for (int a = 0; a < FN; a += STEP)
 #pragma unroll
@@ -559,12 +624,11 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
         }
         bool skip = false;
         if (exact) {
-          skip = ex == kSplitMarked || en.x == kMarkedW || en.y == kMarkedW || en.z == kMarkedW || en.w == kMarkedW;
-          if constexpr (EPI == kGemmSwiglu) {
-            const int4 eu = *reinterpret_cast<const int4 *>(s_we + nl + kSplitRows);
-            skip = skip || eu.x == kMarkedW || eu.y == kMarkedW || eu.z == kMarkedW || eu.w == kMarkedW;
+          if (t < p.rows && n < p.n) {
+            skip = off(acc[a][b], g, t, n0 + nl);
+            if constexpr (EPI == kGemmSwiglu) skip = skip || off(acc[a + 1][b], g, t, n0 + nl + kSplitRows);
           }
-          const uint64_t lanes = __ballot(skip && t < p.rows && n < p.n);
+          const uint64_t lanes = __ballot(skip);
           if (lane == 0) s_exact[wave][(a / STEP * 4 + g) * FT + b] = lanes;
         }
         if (t < p.rows && !skip) {
@@ -592,7 +656,7 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
         }
       }
     }
-  // What was left out: the outputs of marked rows or columns, 4 x 8 at a time, each
+  // What was left out: the outputs to be formed again, 4 x 8 at a time, each
   // read of res and store of y here and nowhere else (y may be res itself).
   if (!exact) return;
   __syncthreads();
