@@ -7,10 +7,12 @@
 //   x w = hi_x hi_w + hi_x lo_w + lo_x hi_w   (+ lo_x lo_w, below 2^-22 of it)
 // with every product exact and every sum fp32: three MFMA products, a third of
 // the fp16 rate, and sums that round three times a 16-wide step of k instead of
-// up to 16 times, so the result is closer to the exact one than the fp32
-// product's. Relative error (2-norm) against float64, normal entries, this
-// product / the library's fp32 product: k = 512 2.6e-7 / 4.1e-7, k = 1024 3.6e-7
-// / 5.7e-7, k = 1365 4.1e-7 / 6.6e-7, k = 2048 5.0e-7 / 8.1e-7.
+// up to 16 times. A sum of many terms is so closer to the exact one than the fp32
+// product's, a sum of few is not. Relative error (2-norm) against float64, normal
+// entries, this product / the library's fp32 product: k = 1 8.1e-8 / 2.5e-8, k = 4
+// 8.2e-8 / 4.0e-8, k = 16 8.8e-8 / 7.4e-8, k = 28 9.7e-8 / 9.6e-8, k = 32 9.5e-8 /
+// 1.03e-7, k = 64 1.1e-7 / 1.4e-7, k = 512 2.6e-7 / 4.1e-7, k = 1024 3.6e-7 /
+// 5.7e-7, k = 1365 4.1e-7 / 6.6e-7, k = 2048 5.0e-7 / 8.1e-7.
 //
 // Each row of x and of W is scaled by the power of two that brings its largest
 // magnitude into [2^14, 2^15); the scales go back in with one ldexp per output.

@@ -275,6 +275,11 @@ def linear_split(mod: torch.nn.Linear, x: torch.Tensor, sizes: list[int]):
 # product of 256 to 512 rows takes 19 us (x [256, 512], W [2048, 512]: 15.2 against
 # 20; x [2048, 512], W [2048, 512]: 28 against 42), and below 256 rows the two meet.
 F32_MIN_ROWS = 256
+# Shortest rows for it: the operands' 23 bits weigh less than the fewer roundings of
+# its sums from here on (2-norm error against float64 over the library's fp32
+# product's, normal / gated entries: k = 16 1.20 / 1.25, 24 1.01 / 1.08, 28 1.01 / 1.04,
+# 32 0.92 / 0.96, 64 0.79 / 0.80, 512 0.64 / 0.64).
+F32_MIN_K = 32
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -320,9 +325,11 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = 
                norm: Optional[tuple[torch.Tensor, float]] = None, residual: Optional[torch.Tensor] = None,
                swiglu: bool = False) -> torch.Tensor:
     """``F.linear(x, w, bias)`` for fp32 x [..., k], w [n, k] (k > 0), bias [n] on one
-    ROCm GPU, on the fp16 matrix cores from split operands: fp32 sums of exact
-    products, no larger an error than the fp32 product's (measured against float64
-    at k = 512, 1024, 2048: 0.63 of it). No gradient. Folded in where given:
+    ROCm GPU, on the fp16 matrix cores from split operands: fp32 sums of products
+    of 23-bit operands. For normal entries the error against float64 is 0.92 of the
+    fp32 product's at k = 32 and 0.63 of it at k = 1024, more than it below k = 32;
+    rows of wide range, infinities and NaNs give what fp32 does
+    (``kla_linear_f32_fwd``). No gradient. Folded in where given:
     ``norm`` (weight [k], eps), RMSNorm of x's rows before it; after it ``residual``
     [..., n], ``residual + (...)``, or ``swiglu`` (w [2 H, k]), ``silu(a[..., :H]) *
     a[..., H:]`` of the product a (a view of rows H rounded up to 4 apart).
@@ -350,9 +357,9 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = 
 def linear_f32_ok(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
     """Whether ``F.linear(x, w, bias)`` of a hip-family module runs as
     :func:`linear_f32`: fp32 on a ROCm GPU outside autocast, no gradient to carry,
-    and at least F32_MIN_ROWS rows."""
+    and at least F32_MIN_ROWS rows of F32_MIN_K."""
     k = w.shape[-1]
-    if (x.dtype != torch.float32 or w.dtype != torch.float32 or not x.is_cuda or k == 0 or w.shape[0] == 0
+    if (x.dtype != torch.float32 or w.dtype != torch.float32 or not x.is_cuda or k < F32_MIN_K or w.shape[0] == 0
             or x.numel() < F32_MIN_ROWS * k or x.shape[-1] != k or w.device != x.device):
         return False
     if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)):
