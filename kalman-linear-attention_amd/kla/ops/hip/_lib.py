@@ -246,14 +246,20 @@ class _Recorded(torch.autograd.Function):
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
+# What _eager asks, bound once (1.2 us a call, half of it with the lookups).
+_compiling = torch.compiler.is_compiling
+_trace_state = torch._C._get_tracing_state
+_interpreter = torch._C._functorch.peek_interpreter_stack
+_forward_ad = torch.autograd.forward_ad
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+
 
 def _eager() -> bool:
     """Whether nothing but autograd watches the call: no compile, export or jit trace,
     no functorch transform, no forward-mode level, no dispatch or function mode."""
-    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
-                or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0
-                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack())
+    return not (_compiling() or _forward_ad._current_level >= 0 or _dispatch_modes() or _function_modes()
+                or _interpreter() is not None or _trace_state() is not None)
 
 
 def call(op, *args):

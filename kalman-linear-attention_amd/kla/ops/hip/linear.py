@@ -329,7 +329,7 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = 
     of 23-bit operands. For normal entries the error against float64 is 0.92 of the
     fp32 product's at k = 32 and 0.63 of it at k = 1024, more than it below k = 32;
     rows of wide range, infinities and NaNs give what fp32 does
-    (``kla_linear_f32_fwd``). No gradient. Folded in where given:
+    (``kla_linear_f32_fwd``). No gradient and no tangent. Folded in where given:
     ``norm`` (weight [k], eps), RMSNorm of x's rows before it; after it ``residual``
     [..., n], ``residual + (...)``, or ``swiglu`` (w [2 H, k]), ``silu(a[..., :H]) *
     a[..., H:]`` of the product a (a view of rows H rounded up to 4 apart).
@@ -351,20 +351,25 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = 
     if w.stride(1) != 1 or (w.shape[0] > 1 and w.stride(0) < k):
         w = w.contiguous()
     bias, norm_w = (None if t is None else t.contiguous() for t in (bias, norm_w))
-    return _lib.call(_linear_f32_op, x, w, bias, norm_w, float(norm[1]) if norm else 0.0, residual, swiglu)
+    args = (x, w, bias, norm_w, float(norm[1]) if norm else 0.0, residual, swiglu)
+    return _lib.call(_linear_f32_op, *args) if _lib._eager() else _linear_f32_op(*args)
 
 
 def linear_f32_ok(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
     """Whether ``F.linear(x, w, bias)`` of a hip-family module runs as
-    :func:`linear_f32`: fp32 on a ROCm GPU outside autocast, no gradient to carry,
-    and at least F32_MIN_ROWS rows of F32_MIN_K."""
+    :func:`linear_f32`: plain fp32 tensors on a ROCm GPU outside autocast, no gradient
+    to carry, at least F32_MIN_ROWS rows of F32_MIN_K, and nothing but autograd
+    watching (a tangent, vmap, a trace, a dispatch or function mode: those see
+    F.linear)."""
     k = w.shape[-1]
     if (x.dtype != torch.float32 or w.dtype != torch.float32 or not x.is_cuda or k < F32_MIN_K or w.shape[0] == 0
             or x.numel() < F32_MIN_ROWS * k or x.shape[-1] != k or w.device != x.device):
         return False
     if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)):
         return False
-    return not torch.is_autocast_enabled("cuda") and (bias is None or bias.dtype == torch.float32)
+    if type(x) not in _lib._PLAIN or type(w) not in _lib._PLAIN or (bias is not None and type(bias) not in _lib._PLAIN):
+        return False
+    return not torch.is_autocast_enabled("cuda") and (bias is None or bias.dtype == torch.float32) and _lib._eager()
 
 
 def unhooked(mod: torch.nn.Module, kind: type) -> bool:
@@ -377,8 +382,7 @@ def unhooked(mod: torch.nn.Module, kind: type) -> bool:
 
 def product_ok(mod: torch.nn.Module, x: torch.Tensor) -> bool:
     """Whether ``mod(x)`` is F.linear on plain parameters and runs as :func:`linear_f32`."""
-    return (unhooked(mod, torch.nn.Linear) and type(mod.weight) in (torch.Tensor, torch.nn.Parameter)
-            and linear_f32_ok(x, mod.weight, mod.bias))
+    return unhooked(mod, torch.nn.Linear) and linear_f32_ok(x, mod.weight, mod.bias)
 
 
 def plain_linear(mod: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:

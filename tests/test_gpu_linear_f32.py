@@ -222,6 +222,40 @@ def test_which_calls_take_it(cuda, monkeypatch):
         orig(x.double(), mod.weight)
 
 
+def test_what_watches_a_product_sees_the_module(cuda):
+    """Tangents, vmap, dispatch and function modes and tensor subclasses meet F.linear, as
+    with any nn.Linear, in MLPs and layers of a hip backend too."""
+    from torch.autograd import forward_ad
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from kla.layers.common import MLP
+
+    mlp = MLP(64, 2.0, kind="gelu").to(cuda)
+    mlp.backend = "hip"
+    x, t = (torch.randn(300, 64, device=cuda) for _ in range(2))
+    with torch.no_grad():
+        want = mlp(x)
+        with forward_ad.dual_level():
+            out = forward_ad.unpack_dual(mlp(forward_ad.make_dual(x, t)))
+        assert out.tangent is not None
+        h = 1e-3
+        slope = (mlp(x + h * t) - mlp(x - h * t)) / (2 * h)
+        assert torch.allclose(out.tangent, slope, rtol=1e-2, atol=1e-2)
+        batched = torch.func.vmap(mlp)(torch.stack([x, t]))
+        assert torch.allclose(batched[0], want, rtol=1e-4, atol=1e-5)
+        with FlopCounterMode(display=False) as flops:
+            mlp(x)
+        assert flops.get_total_flops() == 2 * 300 * 64 * 2 * mlp.w1.weight.shape[0]
+        with torch.overrides.BaseTorchFunctionMode():
+            assert not lin.product_ok(mlp.w1, x)
+        assert lin.product_ok(mlp.w1, x)
+
+        class Sub(torch.Tensor):
+            pass
+
+        assert not lin.product_ok(mlp.w1, x.as_subclass(Sub)) and isinstance(mlp.w1(x.as_subclass(Sub)), Sub)
+
+
 @pytest.mark.parametrize("k", [1, 4, 16, 31, 32, 40, 64, 100, 512, 1365, 2049])
 def test_modules_keep_the_library_accuracy(cuda, k):
     """No module's fp32 inference product is further from float64 (2-norm) than the
