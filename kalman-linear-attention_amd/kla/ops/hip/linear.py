@@ -374,9 +374,10 @@ def linear_f32_ok(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]
 
 def unhooked(mod: torch.nn.Module, kind: type) -> bool:
     """Whether ``mod`` is a ``kind`` itself, not a subclass (nor a parametrised one), with
-    no forward hooks: calling it runs kind.forward and nothing else."""
+    no forward hooks and no forward of its own (as offloading and patching tools set on
+    an instance): calling it runs kind.forward and nothing else."""
     hooks = torch.nn.modules.module
-    return (type(mod) is kind and not (mod._forward_hooks or mod._forward_pre_hooks or hooks._global_forward_hooks
+    return (type(mod) is kind and "forward" not in vars(mod) and not (mod._forward_hooks or mod._forward_pre_hooks or hooks._global_forward_hooks
                                        or hooks._global_forward_pre_hooks))
 
 

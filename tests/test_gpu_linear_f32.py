@@ -222,6 +222,29 @@ def test_which_calls_take_it(cuda, monkeypatch):
         orig(x.double(), mod.weight)
 
 
+def test_a_forward_set_on_an_instance_is_called(cuda):
+    """A module whose instance carries its own forward keeps that call, wherever the split
+    product or a block's folded norms would step past it."""
+    from kla import KLAConfig
+    from kla.configs import ModelConfig
+    from kla.models import Block
+
+    torch.manual_seed(0)
+    block = Block(64, KLAConfig(backend="hip"), ModelConfig(d_model=64)).to(cuda)
+    x = torch.randn(2, 200, 64, device=cuda)
+    with torch.no_grad():
+        want = block(x)
+        mods = (block.mixer.in_proj, block.mixer.out_proj, block.mlp.w12, block.mlp.w3, block.mixer_norm,
+                block.mlp_norm, block.mlp, block.mixer)
+        for mod in mods:
+            seen, plain = [], mod.forward
+            mod.forward = lambda *a, **kw: seen.append(1) or plain(*a, **kw)
+            got = block(x)
+            del mod.forward
+            assert len(seen) == 1, type(mod).__name__
+            assert torch.allclose(got, want, rtol=1e-4, atol=1e-5 * want.abs().max().item())
+
+
 def test_what_watches_a_product_sees_the_module(cuda):
     """Tangents, vmap, dispatch and function modes and tensor subclasses meet F.linear, as
     with any nn.Linear, in MLPs and layers of a hip backend too."""
