@@ -175,10 +175,11 @@ class MLP(nn.Module):
         return rows_linear_hip(h, self.w3.weight, self.w3.bias, residual=x2).reshape(x.shape)
 
     def block_forward_hip(self, x: torch.Tensor, norm: "RMSNorm") -> torch.Tensor | None:
-        """``x + self(norm(x))`` as two split fp32 products, the norm and the SwiGLU folded
-        into the first, the residual into the second (kla.ops.hip.linear.linear_f32),
-        or None where that does not serve: not a SwiGLU MLP in fp32 inference on a hip
-        backend over enough rows. The same operations as the torch lines."""
+        """``x + self(norm(x))`` with split fp32 products, the norm and the SwiGLU folded
+        into the first, the residual into the second where w3 is one too
+        (kla.ops.hip.linear.linear_f32), or None where that does not serve: not a SwiGLU
+        MLP in fp32 inference on a hip backend over enough rows. The same operations as
+        the torch lines."""
         if self.kind != "swiglu" or x.dtype != torch.float32 or not _hip_inference(
                 self.backend, x, *self.parameters(), *norm.parameters()):
             return None
@@ -186,11 +187,10 @@ class MLP(nn.Module):
 
         w12, w3 = self.w12, self.w3
         args = norm_args(norm, x)
-        if args is None or not unhooked(self, MLP) or not product_ok(w12, x) or w12.weight.shape[0] % 2 \
-                or not unhooked(w3, nn.Linear) or any(p.dtype != torch.float32 for p in w3.parameters()):
+        if args is None or not unhooked(self, MLP) or not product_ok(w12, x) or w12.weight.shape[0] % 2:
             return None
         h = linear_f32(x, w12.weight, w12.bias, norm=args, swiglu=True)
-        return linear_f32(h, w3.weight, w3.bias, residual=x)
+        return linear_f32(h, w3.weight, w3.bias, residual=x) if product_ok(w3, h) else x + w3(h)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.kind == "swiglu":

@@ -222,6 +222,41 @@ def test_which_calls_take_it(cuda, monkeypatch):
         orig(x.double(), mod.weight)
 
 
+def test_an_mlp_whose_second_weight_is_no_plain_tensor(cuda):
+    """A block's MLP whose w3 the product cannot take (a tensor subclass, another dtype's
+    module) runs w3's own call on the folded first product."""
+    from kla.layers.common import MLP, RMSNorm
+
+    class Doubling(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            if func is F.linear:
+                return 2 * F.linear(args[0], args[1].as_subclass(torch.Tensor), *args[2:])
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    torch.manual_seed(0)
+    mlp, norm = MLP(64, 4.0).to(cuda).requires_grad_(False), RMSNorm(64).to(cuda).requires_grad_(False)
+    mlp.backend = norm.backend = "hip"
+    x = torch.randn(300, 64, device=cuda)
+    want = mlp.block_forward_hip(x, norm)
+    w = mlp.w3.weight
+    del mlp.w3.weight
+    mlp.w3.weight = w.detach().as_subclass(Doubling)
+    got = mlp.block_forward_hip(x, norm)
+    assert torch.allclose((got - x).as_subclass(torch.Tensor), 2 * (want - x), rtol=1e-4, atol=1e-5)
+
+    class Half(torch.nn.Module):
+        def __init__(self, weight):
+            super().__init__()
+            self.weight = torch.nn.Parameter(weight.bfloat16(), requires_grad=False)
+
+        def forward(self, h):
+            return F.linear(h, self.weight.float())
+
+    mlp.w3 = Half(w)
+    assert torch.allclose(mlp.block_forward_hip(x, norm), want, rtol=2e-2, atol=2e-2)
+
+
 def test_a_forward_set_on_an_instance_is_called(cuda):
     """A module whose instance carries its own forward keeps that call, wherever the split
     product or a block's folded norms would step past it."""
