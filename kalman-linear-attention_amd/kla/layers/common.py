@@ -187,10 +187,10 @@ class MLP(nn.Module):
 
         w12, w3 = self.w12, self.w3
         args = norm_args(norm, x)
-        if args is None or not unhooked(self, MLP) or not product_ok(w12, x) or w12.weight.shape[0] % 2:
+        if args is None or not unhooked(self, MLP) or not product_ok(w12, x, folds=True) or w12.weight.shape[0] % 2:
             return None
         h = linear_f32(x, w12.weight, w12.bias, norm=args, swiglu=True)
-        return linear_f32(h, w3.weight, w3.bias, residual=x) if product_ok(w3, h) else x + w3(h)
+        return linear_f32(h, w3.weight, w3.bias, residual=x) if product_ok(w3, h, folds=True) else x + w3(h)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.kind == "swiglu":

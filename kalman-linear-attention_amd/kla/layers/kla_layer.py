@@ -264,7 +264,8 @@ class KLALayer(nn.Module):
         if _step_on_hip(self.config.backend, x):
             from kla.ops.hip.linear import linear, linear_f32, product_ok
 
-            if not torch.is_grad_enabled() and product_ok(mod, x) and (residual is None or residual.dtype == x.dtype):
+            if (not torch.is_grad_enabled() and product_ok(mod, x, folds=residual is not None)
+                    and (residual is None or residual.dtype == x.dtype)):
                 return linear_f32(x, mod.weight, mod.bias, residual=residual)
             out = linear(mod, x) if torch.is_grad_enabled() else mod(x)
         else:
@@ -285,7 +286,7 @@ class KLALayer(nn.Module):
         if _step_on_hip(self.config.backend, x):
             from kla.ops.hip.linear import linear_f32, linear_split, product_ok, split_blocks
 
-            if not torch.is_grad_enabled() and product_ok(mod, x):
+            if norm is not None or (not torch.is_grad_enabled() and product_ok(mod, x)):
                 return torch.split(linear_f32(x, mod.weight, mod.bias, norm=norm), sizes, dim=-1)
             pieces = linear_split(mod, x, sizes) if torch.is_grad_enabled() else None
             if pieces is None and not (torch.is_grad_enabled() and x.requires_grad):
@@ -469,7 +470,7 @@ class KLALayer(nn.Module):
             return None
         from kla.ops.hip.linear import norm_args, product_ok, unhooked
 
-        if not (unhooked(self, KLALayer) and product_ok(self.in_proj, x) and unhooked(self.out_proj, nn.Linear)
+        if not (unhooked(self, KLALayer) and product_ok(self.in_proj, x, folds=True) and unhooked(self.out_proj, nn.Linear)
                 and all(p.dtype == torch.float32 for p in self.out_proj.parameters())):
             return None
         return norm_args(norm, x)

@@ -163,7 +163,7 @@ class SequenceModel(MarginalReadout, nn.Module):
             from kla.ops.hip.linear import linear_f32, norm_args, product_ok
 
             norm = norm_args(self.norm_f, x)
-            if norm is not None and product_ok(self.lm_head, x):
+            if norm is not None and product_ok(self.lm_head, x, folds=True):
                 return linear_f32(x, self.lm_head.weight, self.lm_head.bias, norm=norm)
         return self.lm_head(self.norm_f(x))
 

@@ -271,9 +271,7 @@ def linear_split(mod: torch.nn.Linear, x: torch.Tensor, sizes: list[int]):
 
 # ------------------------------------------------------------- fp32 inference
 
-# Fewest rows for linear_f32. Its two kernels take 7.5 + 8 us at least; the library
-# product of 256 to 512 rows takes 19 us (x [256, 512], W [2048, 512]: 15.2 against
-# 20; x [2048, 512], W [2048, 512]: 28 against 42), and below 256 rows the two meet.
+# Fewest rows for linear_f32 (from there on by f32_pays).
 F32_MIN_ROWS = 256
 # Shortest rows for it: the operands' 23 bits weigh less than the fewer roundings of
 # its sums from here on (2-norm error against float64 over the library's fp32
@@ -329,7 +327,8 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = 
     of 23-bit operands. For normal entries the error against float64 is 0.92 of the
     fp32 product's at k = 32 and 0.63 of it at k = 1024, more than it below k = 32;
     rows of wide range, infinities and NaNs give what fp32 does
-    (``kla_linear_f32_fwd``). No gradient and no tangent. Folded in where given:
+    (``kla_linear_f32_fwd``). No gradient and no tangent, and no mode sees it
+    (:func:`linear_f32_ok` asks for that). Folded in where given:
     ``norm`` (weight [k], eps), RMSNorm of x's rows before it; after it ``residual``
     [..., n], ``residual + (...)``, or ``swiglu`` (w [2 H, k]), ``silu(a[..., :H]) *
     a[..., H:]`` of the product a (a view of rows H rounded up to 4 apart).
@@ -351,19 +350,43 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = 
     if w.stride(1) != 1 or (w.shape[0] > 1 and w.stride(0) < k):
         w = w.contiguous()
     bias, norm_w = (None if t is None else t.contiguous() for t in (bias, norm_w))
-    args = (x, w, bias, norm_w, float(norm[1]) if norm else 0.0, residual, swiglu)
-    return _lib.call(_linear_f32_op, *args) if _lib._eager() else _linear_f32_op(*args)
+    return _lib.call(_linear_f32_op, x, w, bias, norm_w, float(norm[1]) if norm else 0.0, residual, swiglu)
 
 
-def linear_f32_ok(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
+def f32_pays(rows: int, n: int, k: int, folds: bool) -> bool:
+    """Whether the split product of x [rows, k], w [n, k] is no slower than the library's
+    on MI355X. Up to rows * k = 2^22 it is the host's time that counts: a layer's forward
+    (its widest products run over k = twice its width) then takes the GPU less than the
+    210 us that issuing it takes, and one library call among hand-launched kernels costs
+    14 us more of those (width 512, 2048 tokens: 204 against 218 us, where the GPU needs 183
+    and 178). Above, by both kernels' time in us: the split product's two launches, its
+    row split (8 bytes an element at 4 TB/s) and a product bound by a tile's walk over k
+    (12 ns a step, however few tiles) or by 260 TFLOP/s, what it averages here; the
+    library's at 120 TFLOP/s, with its own split over k where tiles are few. ``folds``
+    counts the kernel (a norm, an add or an activation) that the library's would need
+    beside it. Split / library, in HIP graphs: 2048 x 96, k 2048 38 / 13; 8192 x 160, k
+    2048 67 / 46; 4096 x 512, k 1365 42 / 52; 8188 x 4096, k 1024 215 / 515. A low-rank
+    layer of width 1024 over 2048 and 8190 tokens 290 -> 265 and 835 -> 803 us with it."""
+    if rows * k < 1 << 22:
+        return True
+    ops = 2.0 * rows * n * k
+    split = 7 + 2e-6 * (rows + n) * k + max(0.012 * k, ops / 260e6)
+    library = 4 + ops / 120e6 + (4 if folds else 0)
+    return k >= 96 and split <= library
+
+
+def linear_f32_ok(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, folds: bool = False) -> bool:
     """Whether ``F.linear(x, w, bias)`` of a hip-family module runs as
     :func:`linear_f32`: plain fp32 tensors on a ROCm GPU outside autocast, no gradient
-    to carry, at least F32_MIN_ROWS rows of F32_MIN_K, and nothing but autograd
-    watching (a tangent, vmap, a trace, a dispatch or function mode: those see
+    to carry, at least F32_MIN_ROWS rows of F32_MIN_K, a size that gains (f32_pays, with
+    ``folds`` where a neighbour is folded in), and nothing but autograd watching (a tangent, vmap, a trace, a dispatch or function mode: those see
     F.linear)."""
-    k = w.shape[-1]
-    if (x.dtype != torch.float32 or w.dtype != torch.float32 or not x.is_cuda or k < F32_MIN_K or w.shape[0] == 0
-            or x.numel() < F32_MIN_ROWS * k or x.shape[-1] != k or w.device != x.device):
+    n, k = w.shape
+    if (x.dtype != torch.float32 or w.dtype != torch.float32 or not x.is_cuda or k < F32_MIN_K or n == 0
+            or x.shape[-1] != k or w.device != x.device):
+        return False
+    rows = x.numel() // k
+    if rows < F32_MIN_ROWS or not f32_pays(rows, n, k, folds):
         return False
     if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)):
         return False
@@ -381,9 +404,13 @@ def unhooked(mod: torch.nn.Module, kind: type) -> bool:
                                        or hooks._global_forward_pre_hooks))
 
 
-def product_ok(mod: torch.nn.Module, x: torch.Tensor) -> bool:
-    """Whether ``mod(x)`` is F.linear on plain parameters and runs as :func:`linear_f32`."""
-    return unhooked(mod, torch.nn.Linear) and linear_f32_ok(x, mod.weight, mod.bias)
+def product_ok(mod: torch.nn.Module, x: torch.Tensor, folds: bool = False) -> bool:
+    """Whether ``mod(x)`` is F.linear on plain parameters and runs as :func:`linear_f32`
+    (``folds``: with a norm, a residual or an activation folded in)."""
+    params = vars(mod).get("_parameters", {})     # (not through Module.__getattr__: half a us each)
+    w = params.get("weight")
+    return (w is not None and "bias" in params and unhooked(mod, torch.nn.Linear)
+            and linear_f32_ok(x, w, params["bias"], folds))
 
 
 def plain_linear(mod: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
