@@ -95,10 +95,11 @@ def qk_sensors_hip(k: torch.Tensor, q: torch.Tensor, *, norm: bool, clip: float 
 
 # Token counts below which the k, q columns of the sensor projection run as
 # kla_rows_linear_qk_fwd, apart from the value and variance columns: with the split
-# fp32 product (kla.ops.hip.linear.linear_f32) for those, a layer's forward of width
-# 512 takes 292 us at 4096 tokens against 299 with one product for all columns and
-# the sensor kernel after it, and 1133 against 1116 us at 8188 tokens of width 1024.
-QK_PROJECT_MAX_TOKENS = 6144
+# fp32 product (kla.ops.hip.linear.linear_f32) for those. A layer's forward in us, apart /
+# one product for all columns and the sensor kernel after it: 4096 tokens of width 512
+# 258 / 261, 768 410 / 419, 1024 584 / 603; 5120 tokens of width 256 188 / 179, 512 321 /
+# 307, 768 519 / 513, 1024 737 / 730; 7168 tokens 2 to 4% in favour of one product.
+QK_PROJECT_MAX_TOKENS = 4608
 
 
 def qk_project_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, S: int, *, norm: bool,
