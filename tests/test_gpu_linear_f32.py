@@ -69,6 +69,64 @@ def test_scales_of_rows(cuda):
     assert torch.isinf(got[over]).all() and torch.equal(got[over] > 0, want[over] > 0)
 
 
+# A size for each tile of split_gemm_launch (W rows x tokens), ragged at both ends, and the
+# lengths of its three- or four-deep pipeline: steps of 16 (32 for 64 x 64) with every
+# remainder, and the split's widths (held in registers up to 2048, read twice beyond).
+TILES = {"64x64": (2040, 510), "128x64": (4090, 1020), "128x128": (4090, 2040), "256x128": (8190, 4090)}
+
+
+@pytest.mark.parametrize("k", [512, 1024, 1056, 1088, 1365, 2049])
+@pytest.mark.parametrize("tile", TILES)
+def test_no_tile_is_less_exact_than_the_library(cuda, tile, k):
+    """2-norm error against float64 at most the library's fp32 product's on the same
+    operands (0.62 to 0.64 of it measured; a product that left out either low half would
+    have 500 times it), and each output within _bound."""
+    rows, n = TILES[tile]
+    print(f"[linear_f32] {tile} {rows} x {k} -> {n}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(n + k)
+    x, w = torch.randn(rows, k, device=cuda, generator=g), torch.randn(n, k, device=cuda, generator=g)
+    got, want = lin.linear_f32(x, w), x.double() @ w.double().t()
+    err, library = ((y.double() - want).norm() / want.norm() for y in (got, F.linear(x, w)))
+    assert err <= library and err <= 8e-7, (err.item(), library.item())
+    _check(got, x, w)
+
+
+@pytest.mark.parametrize("what", ["residual", "norm+swiglu", "norm+residual"])
+@pytest.mark.parametrize("k", [1024, 1056, 1088])
+@pytest.mark.parametrize("tile", ["128x128", "256x128"])
+def test_folded_options_on_large_tiles(cuda, tile, k, what):
+    """The same options against the product and torch's operations apart, with a row and a
+    column of non-finite values and rows of wide range inside the tiles."""
+    rows, n = TILES[tile]
+    if "swiglu" in what:
+        n //= 2                     # two rows of W a column
+    print(f"[linear_f32] {tile} {what} {rows} x {k} -> {n}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(n + k)
+
+    def rn(*s):
+        return torch.randn(*s, device=cuda, generator=g)
+
+    x, w, bias, opts = rn(rows, k), rn(n * (2 if "swiglu" in what else 1), k) * k ** -0.5, rn(n * (2 if "swiglu" in what else 1)), {}
+    x[777, 5], w[n - 3, 11] = float("nan"), float("inf")
+    x[1500:1504, 3], w[:, 3] = 1e12, 0
+    if "norm" in what:
+        opts["norm"] = (1 + 0.1 * rn(k), 1e-5)
+    if "residual" in what:
+        opts["residual"] = rn(rows, n)
+    opts["swiglu"] = "swiglu" in what
+    got = lin.linear_f32(x, w, bias, **opts)
+    want, xd, a = _folded(x, w, bias, opts)
+    fin = torch.isfinite(want)
+    assert fin.sum() == (rows - 1) * (n - 1) and torch.equal(torch.isfinite(got), fin)
+    # Plain: fp32's accuracy (2-norm 3.6e-7 at k = 1024, measured); the norm, silu and the
+    # adds round a few times more.
+    err = ((got.double() - want)[fin].norm() / want[fin].norm()).item()
+    assert err <= 1e-6, err
+    part = 1500 if "norm" not in what else 1600     # the wide rows by themselves
+    err = ((got.double() - want)[part][fin[part]].norm() / want[part][fin[part]].norm()).item()
+    assert err <= 2e-6, err
+
+
 def _wide(kind, x, w):
     """Operands whose rows span more than two fp16 planes hold, made from x [rows, k], w [n, k]."""
     k = x.shape[1]
