@@ -10,6 +10,7 @@
 #include <stdio.h>
 
 #include <algorithm>
+#include <cmath>
 #include <initializer_list>
 #include <mutex>
 #include <type_traits>
@@ -1762,6 +1763,7 @@ int linear_f32(const char *fn, const kla_linear_f32_args &a, void *workspace, si
   sp.k = a.k;
   sp.chunks = g.chunks;
   sp.share = static_cast<float>(kSplitShare) / static_cast<float>(a.k);
+  sp.least = 65536.0f / std::sqrt(static_cast<float>(a.k));
   if (swiglu) sp.glu_off = a.glu_off, sp.glu_rows = a.n;
   sp.norm_w = a.norm_w, sp.eps = a.eps;
   if (a.norm_w)

@@ -25,9 +25,13 @@
 // terms are 2^12 and more, so their fp32 rounding alone comes to 2^-12 of that number:
 // where h + 4 c of the two rows is k or less, no fp32 sum promises more. Rows of
 // dense weights and activations have 0.01 to 0.3 k of it, ReLU's 0.55 k. Where it is
-// more, an output that the loss could move by more than 2^-23 of the sum the matrix
-// cores gave is summed in plain fp32 from the operands (split_exact_block), as is
-// every output of a row with an infinity or a NaN.
+// more, an output that the loss could move by more than 2^-26 sqrt(k) of the sum the
+// matrix cores gave (0.85 of the fp32 product's 2-norm error for normal entries) is
+// summed in plain fp32 from the operands (split_exact_block), as is every output of a
+// row with an infinity or a NaN. 8188 x 4096, k 1024, this product / the library's, us:
+// normal entries 210 / 501; one row of NaNs 321 / 483; every output formed again 1130 /
+// 475; one feature of 1.7e9 778 / 486; log-normal entries of sigma 1 210 / 500, 4 1170 /
+// 476.
 //
 // What surrounds a product in a block is folded in: before it the RMSNorm of x's
 // rows (formed as the rows are split, never stored in fp32: 13.1 us at 4096 x 512
@@ -62,8 +66,9 @@ constexpr int kSplitRows = 32;                       // rows of a fragment
 constexpr int kSplitK = 32;                          // k of a pair of fragments (a chunk)
 constexpr int kSplitChunk = kSplitRows * kSplitK * 2;   // fp16 of a chunk: 2 k halves x 2 planes x 512
 constexpr int kSplitExp = 14;                        // scaled rows lie in [2^14, 2^15)
-// A row's word. Its exponent + kSplitBias; kSplitZero for a row of zeros; 2^13 c as the
-// exponent of a float, rounded up (infinite for a row with an infinity or a NaN); and
+// A row's word. Its exponent + kSplitBias; kSplitZero for a row of zeros; the least sum
+// that may stand against its loss, c 2^16 / sqrt(k), as the exponent of a float,
+// rounded up (infinite for a row with an infinity or a NaN); and
 // h + 4 c in units of k / kSplitShare, rounded up.
 constexpr int kSplitBias = 160, kSplitShare = 8192;
 constexpr uint32_t kSplitZero = 1u << 23;
@@ -85,7 +90,7 @@ struct SplitParams {
   SplitOperand op[2];  // x, W
   int64_t k;
   int64_t chunks;      // ceil(k / 32)
-  float share;         // kSplitShare / k
+  float share, least;  // kSplitShare / k, 2^16 / sqrt(k)
   // NORM: x -> (x * rsqrt(mean(x^2) + eps)) * norm_w
   const float *norm_w;
   float eps;
@@ -108,9 +113,10 @@ constexpr int kSplitThreads = 512;
 // rows of odd length ([512, 1365]) load as widely as aligned ones.
 typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));
 
-__device__ __forceinline__ void split_load16(float (&x)[16], const float *row, int64_t k0, int64_t k) {
+template <int N>
+__device__ __forceinline__ void split_load(float (&x)[N], const float *row, int64_t k0, int64_t k) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < N / 4; ++i) {
     f32x4_any_t v = {0.0f, 0.0f, 0.0f, 0.0f};
     const int64_t at = k0 + 4 * i;
     if (at + 4 <= k) {
@@ -150,7 +156,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
   const float *src = op.src + src_row * op.ld;
   const bool norm = NORM && !second;
 
-  auto load = [&](float (&v)[16], int64_t ch) { split_load16(v, src, ch * kSplitK + 16 * half, kin); };
+  auto load = [&](float (&v)[16], int64_t ch) { split_load(v, src, ch * kSplitK + 16 * half, kin); };
 
   constexpr int HELD = NC > 0 ? NC : 1;
   float x[HELD][16];
@@ -158,7 +164,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
   float squares = 0.0f;
   auto scan = [&](const float (&v)[16], int64_t ch) {
     float w[16];
-    if (norm) split_load16(w, p.norm_w, ch * kSplitK + 16 * half, kin);
+    if (norm) split_load(w, p.norm_w, ch * kSplitK + 16 * half, kin);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       uint32_t b = __float_as_uint(v[i]) & 0x7fffffffu;
@@ -214,7 +220,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
   auto put = [&](const float (&v)[16], int64_t ch) {
     _Float16 *out = op.dst + (blk * p.chunks + ch) * kSplitChunk + lane * 8;
     float w[16];
-    if (norm) split_load16(w, p.norm_w, ch * kSplitK + 16 * half, kin);
+    if (norm) split_load(w, p.norm_w, ch * kSplitK + 16 * half, kin);
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
       f16x8_t hi, lo;
@@ -259,7 +265,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
       word |= 0xffu << 24 | 0x3fff;
     } else if (in) {
       const float share = ceilf((h + 4.0f * c) * p.share);
-      const uint32_t lost = __float_as_uint(c * 0x1p13f);
+      const uint32_t lost = __float_as_uint(c * p.least);
       word |= (lost + 0x7fffffu) >> 23 << 24 | static_cast<uint32_t>(fminf(share, 0x3fff));
     }
     op.words[blk * kSplitRows + r] = word | (!marked && bound == 0.0f ? kSplitZero : 0u);
@@ -288,92 +294,55 @@ __device__ __forceinline__ float swiglu_value(float g, float u) { return activat
 // The kernel's arguments, read where they are used (and not before).
 typedef const __attribute__((address_space(4))) SplitGemmParams *SplitGemmArgs;
 
-// The fp32 products of four rows of W from w0 and eight of x from t0 (rows past the
-// last of either read the last again), formed by one wave from the operands as they
-// are: lane l returns that of W row w0 + l / 16 and x row t0 + l / 2 % 8. A lane sums
-// k = 256 i + 4 l + 0..3 by fma and the lanes' sums are added along a fixed tree, so
-// a value depends on its two rows alone. Bound by the operand rows' way from L2.
+// The fp32 products of 32 rows of W from w0 and 32 of x from t0 (rows past the last of
+// either read the last again), formed by one wave from the operands as they are on the
+// fp32 matrix cores, in the layout of split_gemm_kernel's sums. Lane l loads k = 16 i +
+// 8 (l / 32) + 0..7 of its two rows, a step ahead of the eight products that use them; a
+// value depends on its two rows alone.
 template <bool NORM>
-__device__ __forceinline__ float split_exact_block(SplitGemmArgs p, int64_t t0, int64_t w0, int64_t w_last) {
-  constexpr int64_t kStep = 4 * kWave;
+__device__ __forceinline__ f32x16_t split_exact_block(SplitGemmArgs p, int64_t t0, int64_t w0, int64_t w_last) {
+  constexpr int64_t kStep = 16;
   const int lane = static_cast<int>(threadIdx.x) % kWave;
-  const int64_t k = p->k;
-  const float *x[8], *w[4];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) x[i] = p->x + (t0 + i < p->rows ? t0 + i : p->rows - 1) * p->ldx;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = p->w + (w0 + i < w_last ? w0 + i : w_last) * p->ldw;
-  // Elements 4 l + 0..3 of the 256 from `at`, of which n are left unless FULL (0 past
-  // the end).
-  auto load4 = [&](const float *at, int64_t n, auto full) __attribute__((always_inline)) {
-    f32x4_any_t v = {0.0f, 0.0f, 0.0f, 0.0f};
-    const float *mine = reinterpret_cast<const float *>(reinterpret_cast<const char *>(at) + 16u * lane);
-    if (decltype(full)::value || 4 * lane + 4 <= n) {
-      v = *reinterpret_cast<const f32x4_any_t *>(mine);
-    } else {
-      if (4 * lane < n) v.x = mine[0];
-      if (4 * lane + 1 < n) v.y = mine[1];
-      if (4 * lane + 2 < n) v.z = mine[2];
-    }
-    return v;
-  };
-  float scale[NORM ? 8 : 1];
+  const int r = lane % kSplitRows;
+  const int64_t k = p->k, own = lane / kSplitRows * 8;
+  const float *x = p->x + (t0 + r < p->rows ? t0 + r : p->rows - 1) * p->ldx;
+  const float *w = p->w + (w0 + r < w_last ? w0 + r : w_last) * p->ldw;
+  float scale = 1.0f;
   if constexpr (NORM) {
-    float ss[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ss[i] = 0.0f;
-    auto add = [&](int64_t k0, auto full) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const f32x4_any_t v = load4(x[i] + k0, k - k0, full);
-        ss[i] = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss[i]))));
-      }
-    };
-    int64_t k0 = 0;
+    float ss = 0.0f;
 #pragma unroll 1
-    for (; k0 + kStep <= k; k0 += kStep) add(k0, std::true_type{});
-    if (k0 < k) add(k0, std::false_type{});
+    for (int64_t k0 = own; k0 < k; k0 += kStep) {
+      float v[8];
+      split_load(v, x, k0, k);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-#pragma unroll
-      for (int h = kWave / 2; h; h /= 2) ss[i] += __shfl_xor(ss[i], h);
-      scale[i] = rsqrtf(ss[i] / static_cast<float>(k) + p->eps);
+      for (int i = 0; i < 8; ++i) ss = fmaf(v[i], v[i], ss);
     }
+    ss += __shfl_xor(ss, 32);
+    scale = rsqrtf(ss / static_cast<float>(k) + p->eps);
   }
-  float s[32];    // [W row][x row]
+  f32x16_t acc;
 #pragma unroll
-  for (int i = 0; i < 32; ++i) s[i] = 0.0f;
-  auto add = [&](int64_t k0, auto full) __attribute__((always_inline)) {
-    f32x4_any_t xv[8], wv[4];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) xv[i] = load4(x[i] + k0, k - k0, full);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) wv[i] = load4(w[i] + k0, k - k0, full);
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+  float xv[8], wv[8];
+  split_load(xv, x, own, k);
+  split_load(wv, w, own, k);
+#pragma unroll 1
+  for (int64_t k0 = 0; k0 < k; k0 += kStep) {
+    float xn[8], wn[8];
+    split_load(xn, x, k0 + kStep + own, k);
+    split_load(wn, w, k0 + kStep + own, k);
     if constexpr (NORM) {
-      const f32x4_any_t nw = load4(p->norm_w + k0, k - k0, full);
+      float nw[8];
+      split_load(nw, p->norm_w, k0 + own, k);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) xv[i] = (xv[i] * scale[i]) * nw;
+      for (int i = 0; i < 8; ++i) xv[i] = (xv[i] * scale) * nw[i];
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int i = 0; i < 8; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[i], xv[i], acc, 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < 32; ++i) s[i] = fmaf(xv[i % 8][c], wv[i / 8][c], s[i]);
-  };
-  int64_t k0 = 0;
-#pragma unroll 1
-  for (; k0 + kStep <= k; k0 += kStep) add(k0, std::true_type{});
-  if (k0 < k) add(k0, std::false_type{});
-  // Halve the sums a lane holds at each bit of its index: lane l is left with sum l / 2.
-#pragma unroll
-  for (int h = 16; h; h /= 2) {
-    const bool up = lane & (2 * h);
-#pragma unroll
-    for (int i = 0; i < h; ++i) {
-      const float keep = up ? s[i + h] : s[i], give = up ? s[i] : s[i + h];
-      s[i] = keep + __shfl_xor(give, 2 * h);
-    }
+    for (int i = 0; i < 8; ++i) xv[i] = xn[i], wv[i] = wn[i];
   }
-  return s[0] + __shfl_xor(s[0], 1);
+  return acc;
 }
 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
@@ -434,8 +403,8 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
   __shared__ __align__(16) float s_bias[TN];
   __shared__ int s_xe[TT];
   __shared__ int s_doubt[NW];    // by wave, of the rows whose words it read
-  // By wave, block of its features, feature octet and token block: the lanes whose
-  // outputs split_exact_block forms.
+  // By wave, block of its features, four features of it and token block: the lanes
+  // whose outputs split_exact_block forms.
   constexpr int STEP = EPI == kGemmSwiglu ? 2 : 1;
   __shared__ uint64_t s_exact[NW][FN / STEP * 4 * FT];
 
@@ -658,8 +627,8 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
         }
       }
     }
-  // What was left out: the outputs to be formed again, 4 x 8 at a time, each
-  // read of res and store of y here and nowhere else (y may be res itself).
+  // What was left out: the outputs to be formed again, 32 x 32 at a time, each read of
+  // res and store of y here and nowhere else (y may be res itself).
   if (!exact) return;
   __syncthreads();
   SplitGemmArgs args = (SplitGemmArgs)__builtin_amdgcn_kernarg_segment_ptr();
@@ -670,22 +639,23 @@ __global__ void __launch_bounds__(WAVN * WAVT * kWave, OCC) split_gemm_kernel(Sp
     return args->norm_w ? split_exact_block<true>(args, t, w, w_last) : split_exact_block<false>(args, t, w, w_last);
   };
 #pragma unroll 1
-  for (int i = 0; i < FN / STEP * 4 * FT * 8; ++i) {    // a half of the lanes (four features), eight tokens each
-    const int q = i % 8, b = i / 8 % FT, g = i / 8 / FT % 4, a = i / 8 / FT / 4;
-    const uint32_t part = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s_exact[wave][i / 8] >> (8 * q)) & 0xff);
-    if (!part) continue;
-    const int64_t tq = t0 + (wt * FT + b) * kSplitRows + q % 4 * 8;
-    const int64_t nq = n0 / STEP + (wn * FN / STEP + a) * kSplitRows + 8 * g + q / 4 * 4;
-    const int64_t n = nq + lane / 16, t = tq + lane / 2 % 8, rows_n = args->n;
-    const bool in = n < rows_n && t < args->rows;
-    const float *bias = args->bias;
-    float v = dots(tq, nq, rows_n - 1) + (bias && in ? bias[n] : 0.0f);
-    if constexpr (EPI == kGemmSwiglu) {
-      const int64_t off = args->glu_off;
-      const float u = dots(tq, off + nq, off + rows_n - 1);
-      v = swiglu_value(v, u + (bias && in ? bias[off + n] : 0.0f));
-    }
-    if (in && lane % 2 == 0 && (part >> (lane / 2 % 8) & 1)) {
+  for (int i = 0; i < FN / STEP * FT; ++i) {
+    const int a = i / FT, b = i % FT;
+    bool mine[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) mine[g] = s_exact[wave][(a * 4 + g) * FT + b] >> lane & 1;
+    if (!__any(mine[0] || mine[1] || mine[2] || mine[3])) continue;
+    const int64_t tq = t0 + (wt * FT + b) * kSplitRows, nq = n0 / STEP + (wn * FN / STEP + a) * kSplitRows;
+    const int64_t t = tq + lane % 32, n_end = args->n;
+    const f32x16_t sum = dots(tq, nq, n_end - 1);
+    f32x16_t up;
+    if constexpr (EPI == kGemmSwiglu) up = dots(tq, args->glu_off + nq, args->glu_off + n_end - 1);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int64_t n = nq + 8 * (j / 4) + 4 * (lane / 32) + j % 4;
+      if (!mine[j / 4] || n >= n_end) continue;
+      float v = sum[j] + (args->bias ? args->bias[n] : 0.0f);
+      if constexpr (EPI == kGemmSwiglu) v = swiglu_value(v, up[j] + (args->bias ? args->bias[args->glu_off + n] : 0.0f));
       if constexpr (EPI == kGemmResidual) v = args->res[t * args->ldres + n] + v;
       args->y[t * args->ldy + n] = v;
     }
