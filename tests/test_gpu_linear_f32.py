@@ -93,7 +93,7 @@ def test_no_tile_is_less_exact_than_the_library(cuda, tile, k):
 
 @pytest.mark.parametrize("what", ["residual", "norm+swiglu", "norm+residual"])
 @pytest.mark.parametrize("k", [1024, 1056, 1088])
-@pytest.mark.parametrize("tile", ["128x128", "256x128"])
+@pytest.mark.parametrize("tile", ["128x64", "128x128", "256x128"])
 def test_folded_options_on_large_tiles(cuda, tile, k, what):
     """The same options against the product and torch's operations apart, with a row and a
     column of non-finite values and rows of wide range inside the tiles."""

@@ -46,6 +46,13 @@ def test_qk_project_matches_float64(cuda, S, rows, K, norm, clip):
         assert err.max().item() <= 1.0, f"worst ratio {err.max().item():.3g}"
 
 
+@pytest.mark.parametrize("rows,K", [(40, 2048), (33, 1601)])
+def test_qk_project_over_rows_past_one_pass(cuda, rows, K):
+    """Rows longer than the waves of a workgroup hold in one pass (96 k each), with 16-byte
+    loads and with single ones: the kernel's loop over passes."""
+    test_qk_project_matches_float64(cuda, 16, rows, K, True, 0.3)
+
+
 def test_layer_inference_takes_the_kernel_and_matches_torch(cuda, monkeypatch):
     """KLALayer(512, d_state=16) inference on hip runs the k, q sensors through
     qk_project_hip and agrees with the torch backend (float64 on the CPU)."""
