@@ -119,11 +119,17 @@ def ragged_chunk(B: int, L: int, M: int, S: int, cus: int, nc: int, train: bool)
     16 near MIN_CHUNK or above, with which the grid reaches what the equal planners
     aim at, and only where _split_cost says a tenth or more is gained, in training also
     80 us (250 steps): its five more launches take 30 us of host time where the host
-    is what a pass waits for. Whole / split, us on MI355X (M 1000, S 16): forward, one
+    is what a pass waits for. The cost is fitted at S 16; other widths' steps take longer
+    in both walks, so what it takes there gains at least as much: at S 1, 4, 8, 32, 64, 128
+    and 256, eleven shapes each, every split it picks is the faster, one sequence of 1021
+    steps (M 1000, 1000, 500, 1000, 250, 125, 62) forward 114 / 40, 114 / 40, 100 / 37, 87 /
+    67, 98 / 44, 118 / 48, 163 / 61, forward and backward 470 / 240, 470 / 236, 414 / 235,
+    344 / 256, 388 / 232, 510 / 234, 757 / 248. Whole / split, us on MI355X (M 1000, S 16): forward, one
     sequence of 301 steps 30 / 36, 501 46 / 35, 1021 86 / 42; two of 389 38 / 43, 501
     46 / 40, 1021 87 / 65; three of 1021 87 / 86. Forward and backward, one sequence of
     643 steps 234 / 264 (host), 1021 339 / 264, 1501 487 / 264; two of 1501 490 / 344;
-    three of 1501 494 / 521."""
+    three of 1501 494 / 521; four of 771, M 100, 222 / 233 (the host's time: the GPU's
+    gains)."""
     if L % ((32 if train else 2) * nc) == 0:
         return 0
     sp, base = _grid(B, M, S)

@@ -4,7 +4,7 @@ kla_scan_torch, reference src/kla/layers/kla_layer.py:235-349,
 src/kla/ops/kla_ops.py:188-290).
 
 C1, KLALayer(512, d_state=16) forward on x (2, 1024, 512) fp32: the hip layer
-(fp32 projections through torch, every other part in HIP kernels) against the
+(fp32 projections as split products, every other part in HIP kernels) against the
 same weights on backend "torch" on the host CPU in float64, with the
 reference's float32 scan inputs evaluated in float64 (the algorithm's exact
 value), and in float32 (the reference's own CPU run). Bar: the scan's fp32

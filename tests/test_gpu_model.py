@@ -209,7 +209,7 @@ def test_mc_readout_matches_torch_backend(cuda, mc_samples):
 
 
 def test_c5_prefill_logits_against_float64(cuda, monkeypatch):
-    """C5's prefill on hip (fp32 GEMMs through torch, the fused scan and HIP glue)
+    """C5's prefill on hip (split fp32 products, the fused scan and HIP glue)
     against the same model evaluated in float64 on the GPU: float64 GEMMs, and the
     reference layer's float32 scan inputs (kla_layer.py:224-231) evaluated by the
     scan in float64, on the same static dynamics (a_bar, p_bar) as the hip layers.
