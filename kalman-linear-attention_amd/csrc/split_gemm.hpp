@@ -217,6 +217,10 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
 
   int lossy = 0, small = 0;    // this lane's part of c and h
   const int shift = kSplitExp - ex;
+  // What loses: 0 < |u| < 2^-2 of the row's scale (from there on lo is good to 2^-23 of s),
+  // as one unsigned comparison of the bits without the sign.
+  const uint32_t quarter = __float_as_uint(ldexpf(0.25f, -shift)) << 1;
+  const uint32_t below = quarter ? quarter - 1 : 0;
   auto put = [&](const float (&v)[16], int64_t ch) {
     _Float16 *out = op.dst + (blk * p.chunks + ch) * kSplitChunk + lane * 8;
     float w[16];
@@ -231,7 +235,7 @@ __global__ void __launch_bounds__(kSplitThreads) split_rows_kernel(SplitParams p
         hi[i] = static_cast<_Float16>(s);
         lo[i] = static_cast<_Float16>(s - static_cast<float>(hi[i]));
         small += fabsf(s) < 0x1p6f;
-        lossy += fabsf(s) < 0x1p-2f && u != 0.0f;    // (from 2^-2 on lo is good to 2^-23 of s)
+        lossy += (__float_as_uint(u) << 1) - 1 < below;
       }
       *reinterpret_cast<f16x8_t *>(out + (2 * f) * 512) = hi;
       *reinterpret_cast<f16x8_t *>(out + (2 * f + 1) * 512) = lo;
